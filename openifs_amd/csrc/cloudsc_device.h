@@ -121,13 +121,19 @@ __device__ __forceinline__ void supersatcheck(const KCT& c, T pt, T pq, T pa, T 
 // u: byte offset common to the wave (block and level); v: the lane's byte offset within the level.  The sum is
 // formed in 32 bits, so every array access is one vector offset on a scalar base; with wave-uniform blocks
 // (NPROMA a multiple of 64) u is a scalar and the block-dependent offsets cost no vector registers.
+// The casts to the global address space (1) keep the scalar-base form also for bases the compiler cannot trace to a
+// kernel argument.
 template <typename T>
 __device__ __forceinline__ T LD(const T* base, uint32_t u, uint32_t v) {
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + (u + v));
+  typedef const __attribute__((address_space(1))) char gchar;
+  typedef const __attribute__((address_space(1))) T gT;
+  return *(gT*)((gchar*)base + (u + v));
 }
 template <typename T>
 __device__ __forceinline__ void ST(T* base, uint32_t u, uint32_t v, T x) {
-  *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + (u + v)) = x;
+  typedef __attribute__((address_space(1))) char gchar;
+  typedef __attribute__((address_space(1))) T gT;
+  *(gT*)((gchar*)base + (u + v)) = x;
 }
 
 }  // namespace cloudsc_gpu

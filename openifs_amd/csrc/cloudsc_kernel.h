@@ -91,19 +91,21 @@ struct KConstDefault {
   int32_t ncldtop;
 };
 
-// Device pointers of one launch, blocked layout.
+// Device pointers of one launch, blocked layout, in the order the level sweep uses them (neighbours are read from the
+// kernel arguments by one wide scalar load).
 template <typename R>
 struct KPtrs {
-  const R *pt, *pq, *tcml_t, *tcml_q, *tcml_a, *tcml_cld;
-  R *tloc_t, *tloc_q, *tloc_a, *tloc_cld;
-  const R *pvfl, *pvfi, *pap, *paph, *plsm;
-  const int32_t *ldcum, *ktype;
-  const R *peis, *plu;
+  const R *pt, *pq, *pa, *tcml_t, *tcml_q, *tcml_a, *pap, *paph;
+  const R *pclv, *tcml_cld, *pvfl, *pvfi, *pludeli, *pmfu, *pmfd, *plu;
   R* plude;
-  const R *pludeli, *psnde, *pmfu, *pmfd, *pa, *pclv;
-  R *pcovptot, *prainfrac_toprfz;
-  R *pfsqlf, *pfsqif, *pfcqnng, *pfcqlng, *pfsqrf, *pfsqsf, *pfcqrng, *pfcqsng, *pfsqltur, *pfsqitur;
+  const R* psnde;
+  R *tloc_t, *tloc_q, *tloc_a, *tloc_cld;
+  R *pfsqlf, *pfsqif, *pfsqrf, *pfsqsf, *pfcqlng, *pfcqnng, *pfcqrng, *pfcqsng, *pfsqltur, *pfsqitur;
   R *pfplsl, *pfplsn, *pfhpsl, *pfhpsn;
+  R *pcovptot, *prainfrac_toprfz;
+  const R* plsm;
+  const int32_t *ldcum, *ktype;
+  const R* peis;
 };
 
 // Extra device pointers of the fused saturation adjustment + CLOUDSC launch (the CALLPAR sequence
@@ -145,6 +147,18 @@ struct KDims {
   // NULL, or two device counters the launch adds to: points where the reference writes its negative-condensate
   // warnings (cloudsc.F90:3794 liquid, :3802 ice; condensate below -RLMIN before the clean-up)
   uint32_t* nwarn = nullptr;
+};
+
+// The kernel's arguments as one structure, so that the kernel can address a member inside its argument segment.
+template <typename R, typename KC, typename KCD>
+struct KArgs {
+  KC c;
+  KCD cd;
+  KPtrs<R> p;
+  KDims d;
+  int ssc_off;
+  KSatPtrs<R> s;
+  KBudPtrs<R> bp;
 };
 
 // Blocked launch over all blocks (cloudsc_kernel.hip): splits the grid so that every array of one launch spans

@@ -43,8 +43,24 @@ __device__ __forceinline__ void count_warnings(uint32_t* n, bool wl, bool wi) {
 template <typename R, typename RD, typename KC, typename KCD, int BLOCK, bool UNI, bool SAT, bool BUD, int WPE = 0,
           int KL = 0>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE > 0 ? WPE : 1))) void
-cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d, int ssc_off, const KSatPtrs<R> s,
-                      const KBudPtrs<R> bp) {
+cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
+  const KC& c = args.c;
+  const KCD& cd = args.cd;
+  const KPtrs<R>& p = args.p;
+  const KDims& d = args.d;
+  const KSatPtrs<R>& s = args.s;
+  const KBudPtrs<R>& bp = args.bp;
+  const int ssc_off = args.ssc_off;
+  // The ~40 array bases exceed the scalar registers: held across the level loop they would be spilled to vector
+  // lanes and come back through v_readlane (57 in the mixed kernel's code, 172 with the loads ahead).  Inside the loop
+  // they are read from the kernel arguments (scalar cache) where they are used; the empty asm hides that the address
+  // is loop-invariant.
+  typedef const __attribute__((address_space(4))) KArgs<R, KC, KCD> CArgs;
+  auto fresh = [] {
+    uint64_t a = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    return (CArgs*)a;
+  };
   const uint32_t g = blockIdx.x * BLOCK + threadIdx.x;
   const uint32_t nproma = (uint32_t)d.nproma, klev = KL > 0 ? (uint32_t)KL : (uint32_t)d.klev;
   if (g >= (uint32_t)d.ngpblks * nproma) return;
@@ -118,25 +134,62 @@ cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d,
   R paph_k = LD(p.paph, bh, jo);
   R pmfu_k = LD(p.pmfu, b2, jo), pmfd_k = LD(p.pmfd, b2, jo);
 
+  // The inputs of one level (and PMFU, PMFD, PLU of the level below it).  They are loaded at the end of the level
+  // before, ahead of its ~20 stores: loads and stores share one in-order wait counter, so loads issued after the stores
+  // would also wait for those.  At that point few temporaries are live and the ~26 values raise no register peak
+  // (FP32 138 -> 140, mixed 167 -> 166).  With the bases read where they are used (above), same box: mixed 655,360 x
+  // L137 4.17 -> 3.84 ms, FP32 327,680 x L137 2.24 -> 2.02 ms, FP64 65,536 x L137 2.29 -> 1.99 ms, FP32 40,007 x L91 in
+  // blocks of 100 563 -> 466 us, fused FP32 262,144 x L137 2.85 -> 2.45 ms.
+  struct Level {
+    R paph1, pap, t, q, a, ct, cq, ca, vfl, vfi, lude1, lude2, ql, qi, qr, qs, cl, ci, cr, cs;
+    R mfu_n, mfd_n, lu_n, lude, snde1, snde2;
+    R hrsw, hrlw, vdft, vdfq, lude3, lude4, vervel;  // SAT only
+  };
+  auto load = [&](uint32_t k) {
+    const uint32_t i2 = b2 + k * lstep, ih1 = bh + k * lstep + lstep, i5 = b5 + k * lstep, i4 = b4 + k * lstep;
+    const bool below = k + 1 < klev, active = (int)k >= ncldtop0;
+    CArgs* const g = fresh();
+    Level v;
+    v.paph1 = LD(g->p.paph, ih1, jo); v.pap = LD(g->p.pap, i2, jo);
+    v.t = LD(g->p.pt, i2, jo); v.q = LD(g->p.pq, i2, jo); v.a = LD(g->p.pa, i2, jo);
+    v.ct = LD(g->p.tcml_t, i2, jo); v.cq = LD(g->p.tcml_q, i2, jo); v.ca = LD(g->p.tcml_a, i2, jo);
+    v.ql = LD(g->p.pclv, i5, jo); v.qi = LD(g->p.pclv, i5 + sstep, jo);
+    v.qr = LD(g->p.pclv, i5 + 2 * sstep, jo); v.qs = LD(g->p.pclv, i5 + 3 * sstep, jo);
+    v.cl = LD(g->p.tcml_cld, i5, jo); v.ci = LD(g->p.tcml_cld, i5 + sstep, jo);
+    v.cr = LD(g->p.tcml_cld, i5 + 2 * sstep, jo); v.cs = LD(g->p.tcml_cld, i5 + 3 * sstep, jo);
+    v.vfl = LD(g->p.pvfl, i2, jo); v.vfi = LD(g->p.pvfi, i2, jo);
+    v.lude1 = LD(g->p.pludeli, i4, jo); v.lude2 = LD(g->p.pludeli, i4 + sstep, jo);
+    v.mfu_n = below ? LD(g->p.pmfu, i2 + lstep, jo) : R(0);
+    v.mfd_n = below ? LD(g->p.pmfd, i2 + lstep, jo) : R(0);
+    v.lu_n = below ? LD(g->p.plu, i2 + lstep, jo) : R(0);
+    v.lude = active ? LD(g->p.plude, i2, jo) : R(0);
+    const bool snow = active && below && c.lmfdsnow;
+    v.snde1 = snow ? LD(g->p.psnde, b2x + k * lstep, jo) : R(0);
+    v.snde2 = snow ? LD(g->p.psnde, b2x + k * lstep + sstep, jo) : R(0);
+    if constexpr (SAT) {
+      v.hrsw = active ? LD(g->s.phrsw, i2, jo) : R(0); v.hrlw = active ? LD(g->s.phrlw, i2, jo) : R(0);
+      v.vdft = active ? LD(g->s.tvdf_t, i2, jo) : R(0); v.vdfq = active ? LD(g->s.tvdf_q, i2, jo) : R(0);
+      v.lude3 = active ? LD(g->p.pludeli, i4 + 2 * sstep, jo) : R(0);
+      v.lude4 = active ? LD(g->p.pludeli, i4 + 3 * sstep, jo) : R(0);
+      v.vervel = active ? LD(g->s.pvervel, i2, jo) : R(0);
+    }
+    return v;
+  };
+
+  const bool tsat = SAT && s.tsat_t;
+
+  Level nxt = load(0);
   for (uint32_t k = 0; k < klev; ++k) {
     const uint32_t i2 = b2 + k * lstep;        // level k of a (NPROMA,KLEV) array
     const uint32_t ih0 = bh + k * lstep;       // upper half level of layer k
     const uint32_t ih1 = ih0 + lstep;          // lower half level
-    const uint32_t i5 = b5 + k * lstep;
-    const uint32_t i4 = b4 + k * lstep;        // (all wave-uniform with UNI; the lane adds jo)
+    const uint32_t i5 = b5 + k * lstep;        // (all wave-uniform with UNI; the lane adds jo)
     const bool has_next = k + 1 < klev;
-    const R pmfu_n = has_next ? LD(p.pmfu, i2 + lstep, jo) : R(0);
-    const R pmfd_n = has_next ? LD(p.pmfd, i2 + lstep, jo) : R(0);
-    const R plu_n = has_next ? LD(p.plu, i2 + lstep, jo) : R(0);
-    const R paph_k1 = LD(p.paph, ih1, jo);
-    const R pap = LD(p.pap, i2, jo);
-    const R pt = LD(p.pt, i2, jo), pq = LD(p.pq, i2, jo), pa = LD(p.pa, i2, jo);
-    R tcml_t = LD(p.tcml_t, i2, jo), tcml_q = LD(p.tcml_q, i2, jo), tcml_a = LD(p.tcml_a, i2, jo);
-    const R pvfl = LD(p.pvfl, i2, jo), pvfi = LD(p.pvfi, i2, jo);
-    const R pludeli1 = LD(p.pludeli, i4, jo);
-    const R pludeli2 = LD(p.pludeli, i4 + sstep, jo);
-    const R pcl_l = LD(p.pclv, i5, jo), pcl_i = LD(p.pclv, i5 + sstep, jo);
-    R tcml_l = LD(p.tcml_cld, i5, jo), tcml_i = LD(p.tcml_cld, i5 + sstep, jo);
+    const Level in = nxt;
+    const R pmfu_n = in.mfu_n, pmfd_n = in.mfd_n, plu_n = in.lu_n, paph_k1 = in.paph1, pap = in.pap;
+    const R pt = in.t, pq = in.q, pa = in.a, pvfl = in.vfl, pvfi = in.vfi, pludeli1 = in.lude1, pludeli2 = in.lude2;
+    const R pcl_l = in.ql, pcl_i = in.qi;
+    R tcml_t = in.ct, tcml_q = in.cq, tcml_a = in.ca, tcml_l = in.cl, tcml_i = in.ci;
 
     if constexpr (SAT) {
       if ((int)k >= ncldtop0) {  // CLOUD_SATADJ for this point, then TENDENCY_CML += its tendencies
@@ -144,34 +197,34 @@ cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d,
         x.pt = pt, x.pq = pq, x.pa = pa, x.pl = pcl_l, x.pi = pcl_i, x.pap = pap;
         x.paph0 = paph_k, x.paph1 = paph_k1, x.psurf = paph_surf;
         x.tct = tcml_t, x.tcq = tcml_q, x.tca = tcml_a, x.tcl = tcml_l, x.tci = tcml_i;
-        x.hrsw = LD(s.phrsw, i2, jo), x.hrlw = LD(s.phrlw, i2, jo);
-        x.vdft = LD(s.tvdf_t, i2, jo), x.vdfq = LD(s.tvdf_q, i2, jo);
-        x.lude3 = LD(p.pludeli, i4 + 2 * sstep, jo), x.lude4 = LD(p.pludeli, i4 + 3 * sstep, jo);
-        x.vervel = LD(s.pvervel, i2, jo);
+        x.hrsw = in.hrsw, x.hrlw = in.hrlw, x.vdft = in.vdft, x.vdfq = in.vdfq;
+        x.lude3 = in.lude3, x.lude4 = in.lude4, x.vervel = in.vervel;
         const SatOut<R> y = satadj_point<R, RD, KC, KCD>(c, cd, x);
         tcml_t = tcml_t + y.t;
         tcml_q = tcml_q + y.q;
         tcml_a = tcml_a + y.a;
         tcml_l = tcml_l + y.l;
         tcml_i = tcml_i + y.i;
-        ST(s.tcml_t, i2, jo, tcml_t);
-        ST(s.tcml_q, i2, jo, tcml_q);
-        ST(s.tcml_a, i2, jo, tcml_a);
-        ST(s.tcml_cld, i5, jo, tcml_l);
-        ST(s.tcml_cld, i5 + sstep, jo, tcml_i);
-        if (s.tsat_t) {
-          ST(s.tsat_t, i2, jo, y.t);
-          ST(s.tsat_q, i2, jo, y.q);
-          ST(s.tsat_a, i2, jo, y.a);
-          ST(s.tsat_cld, i5, jo, y.l);
-          ST(s.tsat_cld, i5 + sstep, jo, y.i);
+        CArgs* const g = fresh();
+        ST(g->s.tcml_t, i2, jo, tcml_t);
+        ST(g->s.tcml_q, i2, jo, tcml_q);
+        ST(g->s.tcml_a, i2, jo, tcml_a);
+        ST(g->s.tcml_cld, i5, jo, tcml_l);
+        ST(g->s.tcml_cld, i5 + sstep, jo, tcml_i);
+        if (tsat) {
+          ST(g->s.tsat_t, i2, jo, y.t);
+          ST(g->s.tsat_q, i2, jo, y.q);
+          ST(g->s.tsat_a, i2, jo, y.a);
+          ST(g->s.tsat_cld, i5, jo, y.l);
+          ST(g->s.tsat_cld, i5 + sstep, jo, y.i);
         }
-      } else if (s.tsat_t) {  // zero above NCLDTOP (cloud_satadj.F90:338-348); TENDENCY_CML unchanged
-        ST(s.tsat_t, i2, jo, R(0));
-        ST(s.tsat_q, i2, jo, R(0));
-        ST(s.tsat_a, i2, jo, R(0));
-        ST(s.tsat_cld, i5, jo, R(0));
-        ST(s.tsat_cld, i5 + sstep, jo, R(0));
+      } else if (tsat) {  // zero above NCLDTOP (cloud_satadj.F90:338-348); TENDENCY_CML unchanged
+        CArgs* const g = fresh();
+        ST(g->s.tsat_t, i2, jo, R(0));
+        ST(g->s.tsat_q, i2, jo, R(0));
+        ST(g->s.tsat_a, i2, jo, R(0));
+        ST(g->s.tsat_cld, i5, jo, R(0));
+        ST(g->s.tsat_cld, i5 + sstep, jo, R(0));
       }
     }
 
@@ -182,8 +235,8 @@ cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d,
     const R zaorig = za;
     const R ql0 = pcl_l + ptsphy * tcml_l;
     const R qi0 = pcl_i + ptsphy * tcml_i;
-    const R qr0 = LD(p.pclv, i5 + 2 * sstep, jo) + ptsphy * LD(p.tcml_cld, i5 + 2 * sstep, jo);
-    const R qs0 = LD(p.pclv, i5 + 3 * sstep, jo) + ptsphy * LD(p.tcml_cld, i5 + 3 * sstep, jo);
+    const R qr0 = in.qr + ptsphy * in.cr;
+    const R qs0 = in.qs + ptsphy * in.cs;
     R ql = ql0, qi = qi0, qr = qr0, qs = qs0;
 
     // saturation values (:1087-1115)
@@ -243,10 +296,11 @@ cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d,
     // PFPLSL/PFPLSN/PFHPSL/PFHPSN at the upper half level (:4218-4224,4297-4302)
     {
       const R fl = pf_r + R(0), fn = pf_s + pf_i;
-      ST(p.pfplsl, ih0, jo, fl);
-      ST(p.pfplsn, ih0, jo, fn);
-      ST(p.pfhpsl, ih0, jo, -c.rlvtt * fl);
-      ST(p.pfhpsn, ih0, jo, -c.rlstt * fn);
+      CArgs* const g = fresh();
+      ST(g->p.pfplsl, ih0, jo, fl);
+      ST(g->p.pfplsn, ih0, jo, fn);
+      ST(g->p.pfhpsl, ih0, jo, -c.rlvtt * fl);
+      ST(g->p.pfhpsn, ih0, jo, -c.rlstt * fn);
     }
 
     // ZLFSD, ZANEWP, ZRATFSD of this level (LRAD_CLOUD_INHOMOG); above NCLDTOP they keep these values (:944-951)
@@ -260,7 +314,7 @@ cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d,
       Pre3D<R> bud_pre;
       if constexpr (BUD && sizeof(R) == 4) budget_prefetch(bud_pre, bp, ext, k + 1);
       R zrainaut = R(0), zrainacc = R(0), zsnowaut = R(0), zsnowrime = R(0);  // (:1239-1242)
-      const R plude_in = LD(p.plude, i2, jo);
+      const R plude_in = in.lude;
       // derived variables (:1281-1324)
       const R zdp = paph_k1 - paph_k;
       const R zgdp = m_div(c.rg, zdp);
@@ -321,12 +375,12 @@ cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d,
           plude = R(0);
         }
         if (c.lmfdsnow) {
-          csrc_r = LD(p.psnde, b2x + k * lstep, jo) * zdtgdp;
-          csrc_s = LD(p.psnde, b2x + k * lstep + sstep, jo) * zdtgdp;
+          csrc_r = in.snde1 * zdtgdp;
+          csrc_s = in.snde2 * zdtgdp;
           dr = dr + csrc_r;
           ds = ds + csrc_s;
         }
-        ST(p.plude, i2, jo, plude);
+        ST(fresh()->p.plude, i2, jo, plude);
       }
 
       // 3.3 subsidence from the level above (:1419-1492)
@@ -769,7 +823,7 @@ cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d,
         const R zq_upd = pq + ptsphy * (tq + tcml_q);
         const R zt_upd = pt + ptsphy * (tt + tcml_t);
         const R za_upd = pa + ptsphy * (ta + tcml_a);
-        const R pp = ssc_off ? LD(p.pap, i2 + (uint32_t)ssc_off * E, jo) : pap;
+        const R pp = ssc_off ? LD(fresh()->p.pap, i2 + (uint32_t)ssc_off * E, jo) : pap;
         R t_adj, q_adj, a_adj, l_adj, i_adj;
         supersatcheck<R, KC>(c, zt_upd, zq_upd, za_upd, pp, t_adj, q_adj, a_adj, l_adj, i_adj);
         tq = tq + R(q_adj) * zqtmst;
@@ -798,7 +852,7 @@ cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d,
           tt = tt - c.ralsdcp * zi * zqtmst;
         }
       }
-      ST(p.pcovptot, i2, jo, zcovptot);  // (:3814-3816)
+      ST(fresh()->p.pcovptot, i2, jo, zcovptot);  // (:3814-3816)
       if constexpr (BUD) {
         if (bp.fsd) {
           // cloud fraction at the end of the step with the precipitation fraction (:3818-3822); ZDA = ZANEW - ZAORIG
@@ -828,14 +882,17 @@ cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d,
       }
     }
 
+    if (has_next) nxt = load(k + 1);
+
     // store tendencies of this level (levels above NCLDTOP keep the tidy-up terms only)
-    ST(p.tloc_t, i2, jo, tt);
-    ST(p.tloc_q, i2, jo, tq);
-    ST(p.tloc_a, i2, jo, ta);
-    ST(p.tloc_cld, i5, jo, tcld_l);
-    ST(p.tloc_cld, i5 + sstep, jo, tcld_i);
-    ST(p.tloc_cld, i5 + 2 * sstep, jo, tcld_r);
-    ST(p.tloc_cld, i5 + 3 * sstep, jo, tcld_s);
+    CArgs* const g = fresh();
+    ST(g->p.tloc_t, i2, jo, tt);
+    ST(g->p.tloc_q, i2, jo, tq);
+    ST(g->p.tloc_a, i2, jo, ta);
+    ST(g->p.tloc_cld, i5, jo, tcld_l);
+    ST(g->p.tloc_cld, i5 + sstep, jo, tcld_i);
+    ST(g->p.tloc_cld, i5 + 2 * sstep, jo, tcld_r);
+    ST(g->p.tloc_cld, i5 + 3 * sstep, jo, tcld_s);
 
     // DDH fluxes at the lower half level (:4244-4291)
     {
@@ -850,16 +907,17 @@ cloudsc_column_kernel(const KC c, const KCD cd, const KPtrs<R> p, const KDims d,
       sqif = sqif + (qxn_i - qi0 + pvfi * ptsphy) * zgdph_r + pludeli2;
       cqnng = cqnng + zlneg_i * zgdph_r;
       sqitur = sqitur + pvfi * ptsphy * zgdph_r;
-      ST(p.pfsqlf, ih1, jo, sqlf);
-      ST(p.pfsqif, ih1, jo, sqif);
-      ST(p.pfsqrf, ih1, jo, sqrf);
-      ST(p.pfsqsf, ih1, jo, sqsf);
-      ST(p.pfcqlng, ih1, jo, cqlng);
-      ST(p.pfcqnng, ih1, jo, cqnng);
-      ST(p.pfcqrng, ih1, jo, cqrng);
-      ST(p.pfcqsng, ih1, jo, cqsng);
-      ST(p.pfsqltur, ih1, jo, sqltur);
-      ST(p.pfsqitur, ih1, jo, sqitur);
+      CArgs* const h = fresh();
+      ST(h->p.pfsqlf, ih1, jo, sqlf);
+      ST(h->p.pfsqif, ih1, jo, sqif);
+      ST(h->p.pfsqrf, ih1, jo, sqrf);
+      ST(h->p.pfsqsf, ih1, jo, sqsf);
+      ST(h->p.pfcqlng, ih1, jo, cqlng);
+      ST(h->p.pfcqnng, ih1, jo, cqnng);
+      ST(h->p.pfcqrng, ih1, jo, cqrng);
+      ST(h->p.pfcqsng, ih1, jo, cqsng);
+      ST(h->p.pfsqltur, ih1, jo, sqltur);
+      ST(h->p.pfsqitur, ih1, jo, sqitur);
     }
 
     // carry to the next level
@@ -1048,7 +1106,7 @@ hipError_t launch_one(unsigned ncols, const KC& c, const KCD& cd, const KPtrs<R>
                       const KSatPtrs<R>& s, hipStream_t stream) {
   const KBudPtrs<R> nb{};
   hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, BLOCK, true, SAT, false, WPE, KL>),
-                     dim3((ncols + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, stream, c, cd, p, d, ssc_off, s, nb);
+                     dim3((ncols + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
   return hipGetLastError();
 }
 
@@ -1078,7 +1136,7 @@ hipError_t launch_variant(const LaunchCfg& l, bool uni, unsigned ncols, const KC
   const KBudPtrs<R> nb{};
   if (!uni) {  // blocks not aligned to waves: per-lane block offsets, 256-lane groups
     hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, 256, false, SAT, false>), dim3((ncols + 255) / 256),
-                       dim3(256), 0, stream, c, cd, p, d, ssc_off, s, nb);
+                       dim3(256), 0, stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
     return hipGetLastError();
   }
   // the tuned instantiations (register bound, compiled-in KLEV) exist for the default configuration of CLOUDSC
@@ -1103,7 +1161,7 @@ hipError_t launch_either(bool sat, const LaunchCfg& l, bool uni, unsigned ncols,
                          const KBudPtrs<R>* bud, hipStream_t stream) {
   if (bud) {  // budget-instrumented kernel: one instantiation per variant (diagnostic runs); one wave per group
     hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, 64, false, false, true>), dim3((ncols + 63) / 64),
-                       dim3(64), 0, stream, c, cd, p, d, ssc_off, s, *bud);
+                       dim3(64), 0, stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, *bud});
     return hipGetLastError();
   }
   return sat ? launch_variant<true, R, RD>(l, uni, ncols, c, cd, p, d, ssc_off, s, stream)
