@@ -136,4 +136,33 @@ __device__ __forceinline__ void ST(T* base, uint32_t u, uint32_t v, T x) {
   *(gT*)((gchar*)base + (u + v)) = x;
 }
 
+// The same with the non-temporal hint where NT: fields that a sweep reads or writes once, in whole lines.  Rows that share
+// a line with the next wave's (NPROMA no multiple of 64) keep the plain form: there the hint drops lines that are
+// needed again (FP32 40,007 x L91 in blocks of 100: 375 us without, 398 us with it; mixed 655,360 x L137 in blocks of
+// 128: 3.82 ms without, 3.76 ms with it).
+template <bool NT, typename T>
+__device__ __forceinline__ T LDN(const T* base, uint32_t u, uint32_t v) {
+  typedef const __attribute__((address_space(1))) char gchar;
+  typedef const __attribute__((address_space(1))) T gT;
+  if constexpr (NT) return __builtin_nontemporal_load((gT*)((gchar*)base + (u + v)));
+  return *(gT*)((gchar*)base + (u + v));
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void STN(T* base, uint32_t u, uint32_t v, T x) {
+  typedef __attribute__((address_space(1))) char gchar;
+  typedef __attribute__((address_space(1))) T gT;
+  if constexpr (NT)
+    __builtin_nontemporal_store(x, (gT*)((gchar*)base + (u + v)));
+  else
+    *(gT*)((gchar*)base + (u + v)) = x;
+}
+
+// Work-group number -> position in the grid.  The dispatcher deals consecutive work-groups to the 8 XCDs in turn; here
+// each XCD takes one contiguous eighth of the columns, so the groups that run together on it share the pages (and, in
+// ragged blocks, the lines) of the ~50 field arrays.  A bijection for every grid size.
+__device__ __forceinline__ uint32_t xcd_group(uint32_t id, uint32_t n) {
+  const uint32_t x = id & 7u, r = n & 7u;
+  return x * (n >> 3) + (x < r ? x : r) + (id >> 3);
+}
+
 }  // namespace cloudsc_gpu

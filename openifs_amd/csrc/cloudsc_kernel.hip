@@ -61,7 +61,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
     asm volatile("" : "+s"(a));
     return (CArgs*)a;
   };
-  const uint32_t g = blockIdx.x * BLOCK + threadIdx.x;
+  const uint32_t g = xcd_group(blockIdx.x, gridDim.x) * BLOCK + threadIdx.x;
   const uint32_t nproma = (uint32_t)d.nproma, klev = KL > 0 ? (uint32_t)KL : (uint32_t)d.klev;
   if (g >= (uint32_t)d.ngpblks * nproma) return;
   uint32_t b = g / nproma;
@@ -134,12 +134,15 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
   R paph_k = LD(p.paph, bh, jo);
   R pmfu_k = LD(p.pmfu, b2, jo), pmfd_k = LD(p.pmfd, b2, jo);
 
-  // The inputs of one level (and PMFU, PMFD, PLU of the level below it).  They are loaded at the end of the level
-  // before, ahead of its ~20 stores: loads and stores share one in-order wait counter, so loads issued after the stores
+  // The inputs of one level (and PMFU, PMFD, PLU of the level below it).  They are loaded near the end of the level
+  // before, after its implicit solve and ahead of its ~20 stores: loads and stores share one in-order wait counter, so loads issued after the stores
   // would also wait for those.  At that point few temporaries are live and the ~26 values raise no register peak
   // (FP32 138 -> 140, mixed 167 -> 166).  With the bases read where they are used (above), same box: mixed 655,360 x
   // L137 4.17 -> 3.84 ms, FP32 327,680 x L137 2.24 -> 2.02 ms, FP64 65,536 x L137 2.29 -> 1.99 ms, FP32 40,007 x L91 in
   // blocks of 100 563 -> 466 us, fused FP32 262,144 x L137 2.85 -> 2.45 ms.
+  // Earlier (before the truncation) the peak grows: mixed 3.84 -> 4.50 ms.  In FP64, whose state fills the registers,
+  // they are loaded after the supersaturation check instead (65,536 x L137: 1.99 ms, before the check 2.06 ms).
+  constexpr bool AHEAD = sizeof(R) == 4;
   struct Level {
     R paph1, pap, t, q, a, ct, cq, ca, vfl, vfi, lude1, lude2, ql, qi, qr, qs, cl, ci, cr, cs;
     R mfu_n, mfd_n, lu_n, lude, snde1, snde2;
@@ -150,28 +153,28 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
     const bool below = k + 1 < klev, active = (int)k >= ncldtop0;
     CArgs* const g = fresh();
     Level v;
-    v.paph1 = LD(g->p.paph, ih1, jo); v.pap = LD(g->p.pap, i2, jo);
-    v.t = LD(g->p.pt, i2, jo); v.q = LD(g->p.pq, i2, jo); v.a = LD(g->p.pa, i2, jo);
-    v.ct = LD(g->p.tcml_t, i2, jo); v.cq = LD(g->p.tcml_q, i2, jo); v.ca = LD(g->p.tcml_a, i2, jo);
-    v.ql = LD(g->p.pclv, i5, jo); v.qi = LD(g->p.pclv, i5 + sstep, jo);
-    v.qr = LD(g->p.pclv, i5 + 2 * sstep, jo); v.qs = LD(g->p.pclv, i5 + 3 * sstep, jo);
-    v.cl = LD(g->p.tcml_cld, i5, jo); v.ci = LD(g->p.tcml_cld, i5 + sstep, jo);
-    v.cr = LD(g->p.tcml_cld, i5 + 2 * sstep, jo); v.cs = LD(g->p.tcml_cld, i5 + 3 * sstep, jo);
-    v.vfl = LD(g->p.pvfl, i2, jo); v.vfi = LD(g->p.pvfi, i2, jo);
-    v.lude1 = LD(g->p.pludeli, i4, jo); v.lude2 = LD(g->p.pludeli, i4 + sstep, jo);
-    v.mfu_n = below ? LD(g->p.pmfu, i2 + lstep, jo) : R(0);
-    v.mfd_n = below ? LD(g->p.pmfd, i2 + lstep, jo) : R(0);
-    v.lu_n = below ? LD(g->p.plu, i2 + lstep, jo) : R(0);
-    v.lude = active ? LD(g->p.plude, i2, jo) : R(0);
+    v.paph1 = LDN<UNI>(g->p.paph, ih1, jo); v.pap = LDN<UNI>(g->p.pap, i2, jo);
+    v.t = LDN<UNI>(g->p.pt, i2, jo); v.q = LDN<UNI>(g->p.pq, i2, jo); v.a = LDN<UNI>(g->p.pa, i2, jo);
+    v.ct = LDN<UNI>(g->p.tcml_t, i2, jo); v.cq = LDN<UNI>(g->p.tcml_q, i2, jo); v.ca = LDN<UNI>(g->p.tcml_a, i2, jo);
+    v.ql = LDN<UNI>(g->p.pclv, i5, jo); v.qi = LDN<UNI>(g->p.pclv, i5 + sstep, jo);
+    v.qr = LDN<UNI>(g->p.pclv, i5 + 2 * sstep, jo); v.qs = LDN<UNI>(g->p.pclv, i5 + 3 * sstep, jo);
+    v.cl = LDN<UNI>(g->p.tcml_cld, i5, jo); v.ci = LDN<UNI>(g->p.tcml_cld, i5 + sstep, jo);
+    v.cr = LDN<UNI>(g->p.tcml_cld, i5 + 2 * sstep, jo); v.cs = LDN<UNI>(g->p.tcml_cld, i5 + 3 * sstep, jo);
+    v.vfl = LDN<UNI>(g->p.pvfl, i2, jo); v.vfi = LDN<UNI>(g->p.pvfi, i2, jo);
+    v.lude1 = LDN<UNI>(g->p.pludeli, i4, jo); v.lude2 = LDN<UNI>(g->p.pludeli, i4 + sstep, jo);
+    v.mfu_n = below ? LDN<UNI>(g->p.pmfu, i2 + lstep, jo) : R(0);
+    v.mfd_n = below ? LDN<UNI>(g->p.pmfd, i2 + lstep, jo) : R(0);
+    v.lu_n = below ? LDN<UNI>(g->p.plu, i2 + lstep, jo) : R(0);
+    v.lude = active ? LDN<UNI>(g->p.plude, i2, jo) : R(0);
     const bool snow = active && below && c.lmfdsnow;
-    v.snde1 = snow ? LD(g->p.psnde, b2x + k * lstep, jo) : R(0);
-    v.snde2 = snow ? LD(g->p.psnde, b2x + k * lstep + sstep, jo) : R(0);
+    v.snde1 = snow ? LDN<UNI>(g->p.psnde, b2x + k * lstep, jo) : R(0);
+    v.snde2 = snow ? LDN<UNI>(g->p.psnde, b2x + k * lstep + sstep, jo) : R(0);
     if constexpr (SAT) {
-      v.hrsw = active ? LD(g->s.phrsw, i2, jo) : R(0); v.hrlw = active ? LD(g->s.phrlw, i2, jo) : R(0);
-      v.vdft = active ? LD(g->s.tvdf_t, i2, jo) : R(0); v.vdfq = active ? LD(g->s.tvdf_q, i2, jo) : R(0);
-      v.lude3 = active ? LD(g->p.pludeli, i4 + 2 * sstep, jo) : R(0);
-      v.lude4 = active ? LD(g->p.pludeli, i4 + 3 * sstep, jo) : R(0);
-      v.vervel = active ? LD(g->s.pvervel, i2, jo) : R(0);
+      v.hrsw = active ? LDN<UNI>(g->s.phrsw, i2, jo) : R(0); v.hrlw = active ? LDN<UNI>(g->s.phrlw, i2, jo) : R(0);
+      v.vdft = active ? LDN<UNI>(g->s.tvdf_t, i2, jo) : R(0); v.vdfq = active ? LDN<UNI>(g->s.tvdf_q, i2, jo) : R(0);
+      v.lude3 = active ? LDN<UNI>(g->p.pludeli, i4 + 2 * sstep, jo) : R(0);
+      v.lude4 = active ? LDN<UNI>(g->p.pludeli, i4 + 3 * sstep, jo) : R(0);
+      v.vervel = active ? LDN<UNI>(g->s.pvervel, i2, jo) : R(0);
     }
     return v;
   };
@@ -206,25 +209,25 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
         tcml_l = tcml_l + y.l;
         tcml_i = tcml_i + y.i;
         CArgs* const g = fresh();
-        ST(g->s.tcml_t, i2, jo, tcml_t);
-        ST(g->s.tcml_q, i2, jo, tcml_q);
-        ST(g->s.tcml_a, i2, jo, tcml_a);
-        ST(g->s.tcml_cld, i5, jo, tcml_l);
-        ST(g->s.tcml_cld, i5 + sstep, jo, tcml_i);
+        STN<UNI>(g->s.tcml_t, i2, jo, tcml_t);
+        STN<UNI>(g->s.tcml_q, i2, jo, tcml_q);
+        STN<UNI>(g->s.tcml_a, i2, jo, tcml_a);
+        STN<UNI>(g->s.tcml_cld, i5, jo, tcml_l);
+        STN<UNI>(g->s.tcml_cld, i5 + sstep, jo, tcml_i);
         if (tsat) {
-          ST(g->s.tsat_t, i2, jo, y.t);
-          ST(g->s.tsat_q, i2, jo, y.q);
-          ST(g->s.tsat_a, i2, jo, y.a);
-          ST(g->s.tsat_cld, i5, jo, y.l);
-          ST(g->s.tsat_cld, i5 + sstep, jo, y.i);
+          STN<UNI>(g->s.tsat_t, i2, jo, y.t);
+          STN<UNI>(g->s.tsat_q, i2, jo, y.q);
+          STN<UNI>(g->s.tsat_a, i2, jo, y.a);
+          STN<UNI>(g->s.tsat_cld, i5, jo, y.l);
+          STN<UNI>(g->s.tsat_cld, i5 + sstep, jo, y.i);
         }
       } else if (tsat) {  // zero above NCLDTOP (cloud_satadj.F90:338-348); TENDENCY_CML unchanged
         CArgs* const g = fresh();
-        ST(g->s.tsat_t, i2, jo, R(0));
-        ST(g->s.tsat_q, i2, jo, R(0));
-        ST(g->s.tsat_a, i2, jo, R(0));
-        ST(g->s.tsat_cld, i5, jo, R(0));
-        ST(g->s.tsat_cld, i5 + sstep, jo, R(0));
+        STN<UNI>(g->s.tsat_t, i2, jo, R(0));
+        STN<UNI>(g->s.tsat_q, i2, jo, R(0));
+        STN<UNI>(g->s.tsat_a, i2, jo, R(0));
+        STN<UNI>(g->s.tsat_cld, i5, jo, R(0));
+        STN<UNI>(g->s.tsat_cld, i5 + sstep, jo, R(0));
       }
     }
 
@@ -297,10 +300,10 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
     {
       const R fl = pf_r + R(0), fn = pf_s + pf_i;
       CArgs* const g = fresh();
-      ST(g->p.pfplsl, ih0, jo, fl);
-      ST(g->p.pfplsn, ih0, jo, fn);
-      ST(g->p.pfhpsl, ih0, jo, -c.rlvtt * fl);
-      ST(g->p.pfhpsn, ih0, jo, -c.rlstt * fn);
+      STN<UNI>(g->p.pfplsl, ih0, jo, fl);
+      STN<UNI>(g->p.pfplsn, ih0, jo, fn);
+      STN<UNI>(g->p.pfhpsl, ih0, jo, -c.rlvtt * fl);
+      STN<UNI>(g->p.pfhpsn, ih0, jo, -c.rlstt * fn);
     }
 
     // ZLFSD, ZANEWP, ZRATFSD of this level (LRAD_CLOUD_INHOMOG); above NCLDTOP they keep these values (:944-951)
@@ -380,7 +383,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
           dr = dr + csrc_r;
           ds = ds + csrc_s;
         }
-        ST(fresh()->p.plude, i2, jo, plude);
+        STN<UNI>(fresh()->p.plude, i2, jo, plude);
       }
 
       // 3.3 subsidence from the level above (:1419-1492)
@@ -818,6 +821,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
         ta = zda * zqtmst;
       }
 
+      if (AHEAD && has_next) nxt = load(k + 1);
       // 6.4 CLOUD_SUPERSATCHECK on the updated state (:3765-3777), in R
       {
         const R zq_upd = pq + ptsphy * (tq + tcml_q);
@@ -852,7 +856,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
           tt = tt - c.ralsdcp * zi * zqtmst;
         }
       }
-      ST(fresh()->p.pcovptot, i2, jo, zcovptot);  // (:3814-3816)
+      STN<UNI>(fresh()->p.pcovptot, i2, jo, zcovptot);  // (:3814-3816)
       if constexpr (BUD) {
         if (bp.fsd) {
           // cloud fraction at the end of the step with the precipitation fraction (:3818-3822); ZDA = ZANEW - ZAORIG
@@ -882,17 +886,17 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
       }
     }
 
-    if (has_next) nxt = load(k + 1);
+    if (has_next && !(AHEAD && (int)k >= ncldtop0)) nxt = load(k + 1);
 
     // store tendencies of this level (levels above NCLDTOP keep the tidy-up terms only)
     CArgs* const g = fresh();
-    ST(g->p.tloc_t, i2, jo, tt);
-    ST(g->p.tloc_q, i2, jo, tq);
-    ST(g->p.tloc_a, i2, jo, ta);
-    ST(g->p.tloc_cld, i5, jo, tcld_l);
-    ST(g->p.tloc_cld, i5 + sstep, jo, tcld_i);
-    ST(g->p.tloc_cld, i5 + 2 * sstep, jo, tcld_r);
-    ST(g->p.tloc_cld, i5 + 3 * sstep, jo, tcld_s);
+    STN<UNI>(g->p.tloc_t, i2, jo, tt);
+    STN<UNI>(g->p.tloc_q, i2, jo, tq);
+    STN<UNI>(g->p.tloc_a, i2, jo, ta);
+    STN<UNI>(g->p.tloc_cld, i5, jo, tcld_l);
+    STN<UNI>(g->p.tloc_cld, i5 + sstep, jo, tcld_i);
+    STN<UNI>(g->p.tloc_cld, i5 + 2 * sstep, jo, tcld_r);
+    STN<UNI>(g->p.tloc_cld, i5 + 3 * sstep, jo, tcld_s);
 
     // DDH fluxes at the lower half level (:4244-4291)
     {
@@ -908,16 +912,16 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
       cqnng = cqnng + zlneg_i * zgdph_r;
       sqitur = sqitur + pvfi * ptsphy * zgdph_r;
       CArgs* const h = fresh();
-      ST(h->p.pfsqlf, ih1, jo, sqlf);
-      ST(h->p.pfsqif, ih1, jo, sqif);
-      ST(h->p.pfsqrf, ih1, jo, sqrf);
-      ST(h->p.pfsqsf, ih1, jo, sqsf);
-      ST(h->p.pfcqlng, ih1, jo, cqlng);
-      ST(h->p.pfcqnng, ih1, jo, cqnng);
-      ST(h->p.pfcqrng, ih1, jo, cqrng);
-      ST(h->p.pfcqsng, ih1, jo, cqsng);
-      ST(h->p.pfsqltur, ih1, jo, sqltur);
-      ST(h->p.pfsqitur, ih1, jo, sqitur);
+      STN<UNI>(h->p.pfsqlf, ih1, jo, sqlf);
+      STN<UNI>(h->p.pfsqif, ih1, jo, sqif);
+      STN<UNI>(h->p.pfsqrf, ih1, jo, sqrf);
+      STN<UNI>(h->p.pfsqsf, ih1, jo, sqsf);
+      STN<UNI>(h->p.pfcqlng, ih1, jo, cqlng);
+      STN<UNI>(h->p.pfcqnng, ih1, jo, cqnng);
+      STN<UNI>(h->p.pfcqrng, ih1, jo, cqrng);
+      STN<UNI>(h->p.pfcqsng, ih1, jo, cqsng);
+      STN<UNI>(h->p.pfsqltur, ih1, jo, sqltur);
+      STN<UNI>(h->p.pfsqitur, ih1, jo, sqitur);
     }
 
     // carry to the next level
