@@ -35,7 +35,8 @@ int cloudsc_mlp_destroy(cloudsc_mlp_t *m);
 int cloudsc_mlp_dims(const cloudsc_mlp_t *m, int *n_layers, int *din, int *dout);
 /* y[M x n_out] (fp32) = network(x[M x n_in] bf16). */
 int cloudsc_mlp_forward(cloudsc_mlp_t *m, const uint16_t *x, int M, float *y, void *stream);
-/* Forward + backward for L = sum_{m,n} wgt[n] (y[m,n] - t[m,n])^2 / M; x and its transpose xT[n_in x M]. */
+/* Forward + backward for L = sum_{m,n} wgt[n] (y[m,n] - t[m,n])^2 / M; x and its transpose xT[n_in x M] (must not be
+ * NULL; not read: the weight-gradient products transpose x themselves). */
 int cloudsc_mlp_gradients(cloudsc_mlp_t *m, const uint16_t *x, const uint16_t *xT, const float *t, const float *wgt,
                           int M, void *stream);
 /* One Adam step on the gradients of the last cloudsc_mlp_gradients call. */

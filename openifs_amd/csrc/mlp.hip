@@ -1,21 +1,23 @@
 // BF16 MFMA multilayer perceptron for gfx950: forward, backward and Adam, all on the device.
 //
 // Network: x[n_in] -> (Linear, SiLU) x n_hidden_layers -> Linear -> y[n_out].  Weights W_l [n_out_l x n_in_l]
-// are held in FP32 (master copy, Adam moments) and mirrored to BF16 in two layouts: W_l [n_out x n_in] for the
-// forward product and W_l^T [n_in x n_out] for the input-gradient product.  Activations are BF16, every product
-// accumulates in FP32 on the matrix cores (v_mfma_f32_32x32x16_bf16).
+// are held in FP32 (master copy, Adam moments) and mirrored to BF16.  Activations are BF16, every product accumulates
+// in FP32 on the matrix cores (v_mfma_f32_32x32x16_bf16), 16 contraction entries at a time in ascending order, so a
+// result does not depend on the tile that computed it.
 //
-// All products have the one form C[M x N] = A[M x K] * B[N x K]^T with A and B K-contiguous:
-//   forward        Z_l   = X_l  * W_l^T         (A = X_l,   B = W_l)
-//   input grad     dX_l  = dZ_l * W_l           (A = dZ_l,  B = W_l^T)
+// All products have the one form C[M x N] = A[M x K] * B[N x K]^T:
+//   forward        Z_l   = X_l  * W_l^T         (A = X_l,    B = W_l)
+//   input grad     dX_l  = dZ_l * W_l           (A = dZ_l,   B = W_l^T)
 //   weight grad    dW_l  = dZ_l^T * X_l         (A = dZ_l^T, B = X_l^T, contraction over the batch)
-// so the forward and backward epilogues also store the transposed BF16 copies the weight-gradient product reads.
+// Every matrix is stored once, row-major; an operand whose contraction index is its row index (W_l^T, dZ_l^T, X_l^T)
+// is transposed on the way from LDS to the registers (ds_read_b64_tr_b16).
 // Dimensions must be multiples of 128 (M, N) and 32 (K); callers pad features and outputs with zeros.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/cloudsc_surrogate.h"
@@ -28,18 +30,16 @@ namespace mlp {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// Block tiles: TBM x TBN per 256-lane group (2 x 2 waves, each (TBM/2) x (TBN/2) in 32x32 MFMA tiles), K-step TBK.
-// 128 x 128 for small products (training batches), 256 x 128 / 256 x 256 for large ones (inference), where the
-// larger wave tile reads fewer LDS bytes per MFMA (1 KB / 0.75 KB / 0.5 KB).
-constexpr int BM = 128, BN = 128, BK = 32;  // smallest tile: the granularity of every dimension
+constexpr int BM = 128, BN = 128, BK = 32;  // granularity of every dimension
 constexpr int MAX_SPLIT = 4;                // stretches of a split weight-gradient contraction
 
 enum Epi : int {
   EPI_F32 = 0,      // C (fp32)
-  EPI_HIDDEN = 1,   // z = acc + bias -> Z (fp32, kept for the backward pass); a = silu(z) -> A, A^T (bf16)
-  EPI_HIDDEN_INF = 2,  // inference: a = silu(acc + bias) -> A (bf16) only
+  EPI_HIDDEN = 1,   // z = acc + bias -> C (fp32, kept for the backward pass); a = silu(z) -> act (bf16)
+  EPI_HIDDEN_INF = 2,  // inference: a = silu(acc + bias) -> act (bf16) only
   EPI_OUT = 3,      // y = acc + bias -> C (fp32)
-  EPI_DHIDDEN = 4,  // g = acc * silu'(Z) -> A, A^T (bf16): the gradient w.r.t. the previous pre-activation
+  EPI_DHIDDEN = 4,  // g = acc * silu'(z) -> act (bf16): the gradient w.r.t. the previous pre-activation
+  EPI_LOSS = 5,     // y as EPI_OUT, and the loss L = sum wgt[n] (y - t)^2 / M and its gradient -> act (bf16)
 };
 
 struct EpiArgs {
@@ -47,57 +47,174 @@ struct EpiArgs {
   float* c;        // fp32 [M x N], leading dimension ldc
   int ldc;
   bf16* act;       // bf16 [M x N], leading dimension ldc
-  bf16* actT;      // bf16 [N x M], leading dimension ldt
-  int ldt;
-  const float* z;  // fp32 [M x N] pre-activation (EPI_DHIDDEN), leading dimension ldc
+  const float* z;  // fp32 [M x N] pre-activation (EPI_DHIDDEN) or target (EPI_LOSS), leading dimension ldc
   long zstride;    // split contraction (EPI_F32, grid z > 1): elements between the partial products of the splits
+  const float* wgt;  // EPI_LOSS: weight per column
+  float* loss;       // EPI_LOSS: accumulated here by atomics; EPI_HIDDEN: set to 0 if not NULL
+  float batch;       // EPI_LOSS: rows of the batch
 };
 
 __device__ __forceinline__ float sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
 
-template <int EPI, int TBM, int TBN, int TBK>
-__global__ __launch_bounds__(256) void gemm_tn(const bf16* __restrict__ A, int lda, const bf16* __restrict__ B,
-                                               int ldb, int K, EpiArgs e) {
-  constexpr int FM = TBM / 64, FN = TBN / 64;        // 32x32 fragments per wave in M and N
-  constexpr int CPR = TBK / 8, RPP = 256 / CPR;      // 16-byte chunks per row; rows per pass of 256 lanes
-  constexpr int LA = TBM / RPP, LB = TBN / RPP;      // chunks per thread per K-step, A and B
-  // LDS rows of TBK bf16 (no padding); chunk c of row r sits in slot c ^ ((r >> SH) & (CPR - 1)), SH = log2(16 / CPR):
-  // the 16 rows one fragment read touches (one chunk each) and the rows one store pass writes then fall in 16
-  // distinct 16-byte slots of each 256-byte bank window -- no bank conflict on either side
-  constexpr int LDKT = TBK, SH = CPR == 4 ? 2 : (CPR == 8 ? 1 : 0);
-  static_assert(CPR == 4 || CPR == 8, "K-step 32 or 64");
-  __shared__ bf16 As[2][TBM * LDKT];
-  __shared__ bf16 Bs[2][TBN * LDKT];
-  auto slot = [](int r, int c) { return 8 * (c ^ ((r >> SH) & (CPR - 1))); };
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wm = w >> 1, wn = w & 1;
-  const int m0 = blockIdx.y * TBM, n0 = blockIdx.x * TBN;
-  // split contraction: group z multiplies the z-th stretch of K columns into its own partial product
-  A += (size_t)blockIdx.z * K;
-  B += (size_t)blockIdx.z * K;
-  if (EPI == EPI_F32) e.c += (size_t)blockIdx.z * e.zstride;
-  // global -> LDS in chunks of 8 bf16; thread t moves rows r0, r0 + RPP, ...
-  const int r0 = tid / CPR, kq = (tid % CPR) * 8;
-  const bf16* ag = A + (size_t)(m0 + r0) * lda + kq;
-  const bf16* bg = B + (size_t)(n0 + r0) * ldb + kq;
-  bf16x8 ra[LA], rb[LB];
-  auto gload = [&](int k0) {
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+// Epilogue of a wave's FM x FN fragments of C^T = B A^T: register r of lane l holds C[m][n] with m = lane & 31 of the
+// fragment's rows and n = 8 (r >> 2) + 4 (l >> 5) + (r & 3) of its columns, so each lane owns runs of 4 consecutive
+// columns of one row, stored as one 16-byte (fp32) or 8-byte (bf16) write each.  row, col: this lane's first row and
+// column.  All loads come before the first store: loads and stores share one in-order wait counter.
+template <int EPI, int NW, int FM, int FN>
+__device__ __forceinline__ void epilogue(const EpiArgs& e, const f32x16 (&acc)[FM][FN], int row, int col) {
+  constexpr bool BIAS = EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_INF || EPI == EPI_OUT || EPI == EPI_LOSS;
+  constexpr bool READZ = EPI == EPI_DHIDDEN || EPI == EPI_LOSS;
+  f32x4 bias[FN][4], wgt[FN][4], z[FM][FN][4];
 #pragma unroll
-    for (int i = 0; i < LA; ++i) ra[i] = *reinterpret_cast<const bf16x8*>(ag + (size_t)(RPP * i) * lda + k0);
+  for (int j = 0; j < FN; ++j)
 #pragma unroll
-    for (int i = 0; i < LB; ++i) rb[i] = *reinterpret_cast<const bf16x8*>(bg + (size_t)(RPP * i) * ldb + k0);
-  };
-  auto sstore = [&](int buf) {
+    for (int q = 0; q < 4; ++q) {
+      if (BIAS) bias[j][q] = *reinterpret_cast<const f32x4*>(e.bias + col + j * 32 + 8 * q);
+      if (EPI == EPI_LOSS) wgt[j][q] = *reinterpret_cast<const f32x4*>(e.wgt + col + j * 32 + 8 * q);
+      if (READZ)
 #pragma unroll
-    for (int i = 0; i < LA; ++i) {
-      const int r = r0 + RPP * i;
-      *reinterpret_cast<bf16x8*>(&As[buf][r * LDKT + slot(r, kq / 8)]) = ra[i];
+        for (int i = 0; i < FM; ++i)
+          z[i][j][q] = *reinterpret_cast<const f32x4*>(e.z + (size_t)(row + i * 32) * e.ldc + col + j * 32 + 8 * q);
     }
+  float l = 0.0f;
 #pragma unroll
-    for (int i = 0; i < LB; ++i) {
-      const int r = r0 + RPP * i;
-      *reinterpret_cast<bf16x8*>(&Bs[buf][r * LDKT + slot(r, kq / 8)]) = rb[i];
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const size_t o = (size_t)(row + i * 32) * e.ldc + col + j * 32 + 8 * q;
+        f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        if (BIAS) v = v + bias[j][q];
+        if (EPI != EPI_HIDDEN_INF && EPI != EPI_DHIDDEN) *reinterpret_cast<f32x4*>(e.c + o) = v;
+        if (EPI == EPI_F32 || EPI == EPI_OUT) continue;
+        bf16x4 a;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          if (EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_INF) {
+            a[t] = (bf16)(v[t] * sigmoid(v[t]));
+          } else if (EPI == EPI_DHIDDEN) {
+            const float zt = z[i][j][q][t], s = sigmoid(zt);
+            a[t] = (bf16)(v[t] * (s * (1.0f + zt * (1.0f - s))));
+          } else {
+            const float d = v[t] - z[i][j][q][t];
+            const float wd = wgt[j][q][t] * d;
+            l += wd * d;
+            a[t] = (bf16)(2.0f * wd / e.batch);
+          }
+        }
+        *reinterpret_cast<bf16x4*>(e.act + o) = a;
+      }
+  if constexpr (EPI == EPI_LOSS) {  // one atomic per group: they all go to one address and are served one by one
+    __shared__ float part[NW];
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = l;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int i = 1; i < NW; ++i) l += part[i];
+      atomicAdd(e.loss, l / e.batch);
     }
+  }
+}
+
+// One operand tile of TB rows x 64 contraction entries in LDS, filled by global_load_lds_dwordx4 (lane l of a load
+// writes 16 bytes at 16 l).  Each lane fetches the global chunk that belongs in its LDS slot.
+//  T = false: the matrix is [rows][K].  LDS row r of 128 bytes, chunk c (16 B) in slot c ^ ((r >> 1) & 7): a fragment
+//    read (16 lanes = 16 consecutive rows, one chunk) finds its rows in distinct slots of the banks.
+//  T = true: the matrix is [K][rows].  LDS row k of TB entries, its 64-byte chunk c in slot c ^ f(k) such that the 4
+//    rows k..k+3 which one transposing read touches lie in distinct quarters of the banks.
+template <int TB, bool T, int NW>
+struct Tile {
+  static constexpr int W = T ? TB * 2 : 128;        // bytes per LDS row
+  static constexpr int NLD = TB * 128 / 1024 / NW;  // loads per wave
+  static __device__ __forceinline__ int swz(int k) { return TB == 128 ? (k & 3) : ((k >> 1) & 1); }
+  // p: the matrix at (row0, k0 = 0).  CLAMP: only K entries may be read (the last step of a contraction that is no
+  // multiple of 64 repeats its last entries, which are not multiplied).
+  template <bool CLAMP>
+  static __device__ __forceinline__ void load(bf16* lds, const bf16* p, int ld, int k0, int K, int w, int lane) {
+    typedef bf16 __attribute__((address_space(3))) lbf16;
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+      const int g = NW * i + w;  // 1 KB group of the tile
+      const bf16* src;
+      if (T) {
+        const int r = lane / (W / 16), s = lane % (W / 16), k = g * (1024 / W) + r;
+        src = p + (size_t)(CLAMP ? min(k0 + k, K - 1) : k0 + k) * ld + 32 * ((s >> 2) ^ swz(k)) + 8 * (s & 3);
+      } else {
+        const int r = 8 * g + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        src = p + (size_t)r * ld + (CLAMP ? min(k0 + 8 * c, K - 8) : k0 + 8 * c);
+      }
+      __builtin_amdgcn_global_load_lds((const void*)src, (lbf16*)(lds + g * 512), 16, 0, 0);
+    }
+  }
+  // MFMA 32x32x16 operand: lane l supplies row (l & 31) of the 32-row block rb and k = ks + 8 (l >> 5) .. +7.  A
+  // transposing read gives lane i of 16 the column i of 4 rows, whose 16-byte quarters the lanes 4 j + q address.
+  static __device__ __forceinline__ bf16x8 frag(const bf16* lds, int rb, int ks, int lane) {
+    if (T) {
+      typedef short s16x4 __attribute__((ext_vector_type(4)));
+      typedef s16x4 __attribute__((address_space(3))) ls16x4;
+      const int j = (lane >> 2) & 3, n = 16 * ((lane >> 4) & 1) + 4 * (lane & 3), k = ks + 8 * (lane >> 5) + j;
+      const bf16* a = lds + k * TB + 32 * ((rb >> 5) ^ swz(k)) + n;
+      const bf16* b = lds + (k + 4) * TB + 32 * ((rb >> 5) ^ swz(k + 4)) + n;
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls16x4*)a);
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls16x4*)b);
+      typedef short s16x8 __attribute__((ext_vector_type(8)));
+      const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      return __builtin_bit_cast(bf16x8, v);
+    }
+    const int r = rb + (lane & 31), c = (ks >> 3) + (lane >> 5);
+    return *reinterpret_cast<const bf16x8*>(lds + r * 64 + 8 * (c ^ ((r >> 1) & 7)));
+  }
+};
+
+// Waits until at most N of this wave's vector loads are in flight and its LDS reads are done, then for the group.
+template <int N>
+__device__ __forceinline__ void landed() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4));  // vmcnt(N) lgkmcnt(0), no expcnt
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// The kernel of the training products: a TBM x TBN tile per 256 lanes (2 x 2 waves), contraction steps of 64 in a ring
+// of 4 LDS stages filled 3 steps ahead.  These products have about one tile per CU, so one wave per SIMD has to cover
+// the load latency by itself: a step of 128 x 128 multiplies for ~0.2 us at the matrix cores' rate and its loads take
+// several times that; it measures 0.5 us, which is the rate the tiles come from L2 (16 TB/s over the chip).  The stages
+// are separate LDS objects and the step loop is unrolled over them, so that the compiler can tell a read of one stage
+// from the loads in flight into the others.  4,096 x 1,024 x 1,024 with the hidden layer's epilogue (25 MB stored):
+// 18 us, x 1,920: 26 us; the register-staged kernel with transposed copies of every activation and gradient that this
+// one replaces took 39 us on average over the three, the weight gradient 25 -> 16 us and the input gradient 35 -> 20 us
+// (1,024 x 1,024).
+template <int EPI, int TBM, int TBN, int NW, bool TA, bool TB>
+__global__ __launch_bounds__(64 * NW) void gemm_ring(const bf16* __restrict__ A, int lda, const bf16* __restrict__ B,
+                                                 int ldb, int K, EpiArgs e) {
+  constexpr int WN = NW / 2, WCOL = TBN / WN, FM = TBM / 64, FN = WCOL / 32;  // 2 x WN waves of FM x FN fragments
+  typedef Tile<TBM, TA, NW> OpA;
+  typedef Tile<TBN, TB, NW> OpB;
+  constexpr int ELEMS = (TBM + TBN) * 64, NLD = OpA::NLD + OpB::NLD;
+  __shared__ __attribute__((aligned(1024))) bf16 s0[ELEMS], s1[ELEMS], s2[ELEMS], s3[ELEMS];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = w / WN, wn = w % WN;
+  // XCD order: consecutive work-groups go to the 8 XCDs in turn; each XCD takes one contiguous eighth of the tiles
+  // (N fastest, then M, then the stretch of a split contraction), so that its L2 holds what those tiles share.
+  const uint32_t total = gridDim.x * gridDim.y * gridDim.z;
+  const uint32_t id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  const uint32_t x = id & 7u, r8 = total & 7u;
+  const uint32_t tile = x * (total >> 3) + (x < r8 ? x : r8) + (id >> 3);
+  const int nt = tile % gridDim.x, mt = tile / gridDim.x % gridDim.y, zt = tile / (gridDim.x * gridDim.y);
+  const int m0 = mt * TBM, n0 = nt * TBN;
+  // split contraction: group zt multiplies the zt-th stretch of K entries into its own partial product
+  const size_t kz = (size_t)zt * K;
+  const bf16* ap = TA ? A + kz * lda + m0 : A + (size_t)m0 * lda + kz;
+  const bf16* bp = TB ? B + kz * ldb + n0 : B + (size_t)n0 * ldb + kz;
+  if (EPI == EPI_F32) e.c += (size_t)zt * e.zstride;
+  if (EPI == EPI_HIDDEN && e.loss && tid == 0 && id == 0) *e.loss = 0.0f;
+  auto load = [&](bf16* s, int t, auto clamp) {
+    OpA::template load<decltype(clamp)::value>(s, ap, lda, 64 * t, K, w, lane);
+    OpB::template load<decltype(clamp)::value>(s + TBM * 64, bp, ldb, 64 * t, K, w, lane);
   };
   f32x16 acc[FM][FN];
 #pragma unroll
@@ -107,70 +224,64 @@ __global__ __launch_bounds__(256) void gemm_tn(const bf16* __restrict__ A, int l
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  const int nk = K / TBK;
-  gload(0);
-  sstore(0);
-  __syncthreads();
-  // MFMA 32x32x16 operand layout: lane l supplies row (l & 31) of its 32-row block and k = 8*(l >> 5) .. +7
-  const int fr = lane & 31, fk = 8 * (lane >> 5);
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < nk) gload((kt + 1) * TBK);
+  const int nk = (K + 63) / 64;
+  auto sub = [&](const bf16* s, int ks) {  // 16 contraction entries
+    bf16x8 a[FM], b[FN];
 #pragma unroll
-    for (int ks = 0; ks < TBK; ks += 16) {
-      bf16x8 a[FM], b[FN];
+    for (int i = 0; i < FM; ++i) a[i] = OpA::frag(s, wm * (TBM / 2) + i * 32, ks, lane);
 #pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const int r = wm * (TBM / 2) + i * 32 + fr;
-        a[i] = *reinterpret_cast<const bf16x8*>(&As[cur][r * LDKT + slot(r, (ks + fk) / 8)]);
-      }
+    for (int j = 0; j < FN; ++j) b[j] = OpB::frag(s + TBM * 64, wn * WCOL + j * 32, ks, lane);
 #pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int r = wn * (TBN / 2) + j * 32 + fr;
-        b[j] = *reinterpret_cast<const bf16x8*>(&Bs[cur][r * LDKT + slot(r, (ks + fk) / 8)]);
-      }
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+      for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+  };
+  // One step: this wave's loads of stage t have landed, then everyone's have (and everyone is done with stage t - 1,
+  // whose buffer `next` takes step t + 3).  The loads of steps t + 1 and t + 2 stay in flight.
+  auto step = [&](const bf16* cur, bf16* next, int t) {
+    landed<2 * NLD>();
+    load(next, t + 3, std::false_type());
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    for (int ks = 0; ks < 64; ks += 16) sub(cur, ks);
+  };
+  // The last steps, and contractions of few steps.
+  auto tail = [&](const bf16* cur, bf16* next, int t) {
+    const int ahead = nk - 1 - t;  // later steps whose loads may still be in flight: 2 at most
+    if (ahead >= 2)
+      landed<2 * NLD>();
+    else if (ahead == 1)
+      landed<NLD>();
+    else
+      landed<0>();
+    if (ahead >= 3) load(next, t + 3, std::true_type());
+    sub(cur, 0);
+    sub(cur, 16);
+    if (K - 64 * t > 32) {
+      sub(cur, 32);
+      sub(cur, 48);
     }
-    if (kt + 1 < nk) sstore(cur ^ 1);
-    __syncthreads();
+  };
+  load(s0, 0, std::true_type());  // contractions of fewer than 3 steps load entries of their last one again
+  load(s1, 1, std::true_type());
+  load(s2, 2, std::true_type());
+  int t = 0;
+  for (; t + 7 < nk; t += 4) {
+    step(s0, s3, t);
+    step(s1, s0, t + 1);
+    step(s2, s1, t + 2);
+    step(s3, s2, t + 3);
+  }
+  for (; t < nk; t += 4) {
+    tail(s0, s3, t);
+    if (t + 1 >= nk) break;
+    tail(s1, s0, t + 1);
+    if (t + 2 >= nk) break;
+    tail(s2, s1, t + 2);
+    if (t + 3 >= nk) break;
+    tail(s3, s2, t + 3);
   }
 
-  // Accumulator layout: register r of lane l holds row 8*(r>>2) + 4*(l>>5) + (r&3), column l & 31.
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int col = n0 + wn * (TBN / 2) + j * 32 + (lane & 31);
-      const float bias = (EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_INF || EPI == EPI_OUT) ? e.bias[col] : 0.0f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = m0 + wm * (TBM / 2) + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const size_t o = (size_t)row * e.ldc + col;
-        const float v = acc[i][j][r];
-        if (EPI == EPI_F32) {
-          e.c[o] = v;
-        } else if (EPI == EPI_OUT) {
-          e.c[o] = v + bias;
-        } else if (EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_INF) {
-          const float z = v + bias;
-          const bf16 a = (bf16)(z * sigmoid(z));
-          if (EPI == EPI_HIDDEN) {
-            e.c[o] = z;
-            e.actT[(size_t)col * e.ldt + row] = a;
-          }
-          e.act[o] = a;
-        } else {  // EPI_DHIDDEN
-          const float z = e.z[o];
-          const float s = sigmoid(z);
-          const bf16 g = (bf16)(v * (s * (1.0f + z * (1.0f - s))));
-          e.act[o] = g;
-          e.actT[(size_t)col * e.ldt + row] = g;
-        }
-      }
-    }
+  epilogue<EPI, NW, FM, FN>(e, acc, m0 + wm * (TBM / 2) + (lane & 31), n0 + wn * WCOL + 4 * (lane >> 5));
 }
 
 // The large-product kernel: 256 x 256 block tile, K-step 64, NW waves as 2 x (NW/2), each computing 128 rows x
@@ -216,6 +327,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_tn_dl(const bf16* __restrict__ A
                                        (lbf16*)&lds[buf][1][(NW * i + w) * 512], 16, 0, 0);
     }
   };
+  if (EPI == EPI_HIDDEN && e.loss && tid == 0 && blockIdx.x == 0 && blockIdx.y == 0) *e.loss = 0.0f;
   f32x16 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -256,82 +368,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_tn_dl(const bf16* __restrict__ A
     }
   }
 
-  // The product is formed as C^T = B A^T, so register r of lane l holds C[m][n] with m = lane & 31 of the fragment's
-  // rows and n = 8*(r>>2) + 4*(l>>5) + (r&3) of its columns: each lane owns 4 runs of 4 consecutive columns of one
-  // row, stored as one 16-byte (fp32) or 8-byte (bf16) write each.
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int row = m0 + wm * 128 + i * 32 + (lane & 31);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int col = n0 + wn * WCOL + j * 32 + 8 * q + 4 * (lane >> 5);
-        const size_t o = (size_t)row * e.ldc + col;
-        f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-        if (EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_INF || EPI == EPI_OUT)
-          v = v + *reinterpret_cast<const f32x4*>(e.bias + col);
-        if (EPI == EPI_F32 || EPI == EPI_OUT) {
-          *reinterpret_cast<f32x4*>(e.c + o) = v;
-        } else if (EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_INF) {
-          bf16x4 a;
-#pragma unroll
-          for (int t = 0; t < 4; ++t) a[t] = (bf16)(v[t] * sigmoid(v[t]));
-          if (EPI == EPI_HIDDEN) {
-            *reinterpret_cast<f32x4*>(e.c + o) = v;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) e.actT[(size_t)(col + t) * e.ldt + row] = a[t];
-          }
-          *reinterpret_cast<bf16x4*>(e.act + o) = a;
-        } else {  // EPI_DHIDDEN
-          const f32x4 z = *reinterpret_cast<const f32x4*>(e.z + o);
-          bf16x4 g;
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const float sg = sigmoid(z[t]);
-            g[t] = (bf16)(v[t] * (sg * (1.0f + z[t] * (1.0f - sg))));
-          }
-          *reinterpret_cast<bf16x4*>(e.act + o) = g;
-#pragma unroll
-          for (int t = 0; t < 4; ++t) e.actT[(size_t)(col + t) * e.ldt + row] = g[t];
-        }
-      }
-    }
-}
-
-// Output-layer loss: L = sum_{m,n} wgt[n] (y - t)^2 / M.  dY = 2 wgt[n] (y - t) / M (bf16, both layouts);
-// loss partial sums are accumulated into *loss (fp32 atomics).  A 64 x 64 tile per 256-lane group: rows of dY read
-// and written along n, the transposed copy written along m through LDS, so that every store is coalesced.
-__global__ __launch_bounds__(256) void mse_grad(const float* __restrict__ y, const float* __restrict__ t,
-                                                const float* __restrict__ wgt, int M, int N, bf16* __restrict__ dy,
-                                                bf16* __restrict__ dyT, float* __restrict__ loss) {
-  __shared__ bf16 tile[64][66];
-  const int n0 = blockIdx.x * 64, m0 = blockIdx.y * 64;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  float l = 0.0f;
-  for (int r = ty; r < 64; r += 4) {  // lanes along n
-    const int m = m0 + r, n = n0 + tx;
-    bf16 g = (bf16)0.0f;
-    if (m < M && n < N) {
-      const size_t idx = (size_t)m * N + n;
-      const float d = y[idx] - t[idx];
-      const float wd = wgt[n] * d;
-      l += wd * d;
-      g = (bf16)(2.0f * wd / (float)M);
-      dy[idx] = g;
-    }
-    tile[r][tx] = g;
-  }
-  __syncthreads();
-  for (int r = ty; r < 64; r += 4) {  // lanes along m
-    const int n = n0 + r, m = m0 + tx;
-    if (m < M && n < N) dyT[(size_t)n * M + m] = tile[tx][r];
-  }
-  // wave reduction, one atomic per wave
-  for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
-  if ((threadIdx.x & 63) == 0 && l != 0.0f) atomicAdd(loss, l / (float)M);
+  epilogue<EPI, NW, FM, FN>(e, acc, m0 + wm * 128 + (lane & 31), n0 + wn * WCOL + 4 * (lane >> 5));
 }
 
 // Sum of the S partial products of a split contraction, in split order: out[i] = sum_z part[z * n + i].
@@ -343,58 +380,113 @@ __global__ void sum_splits(const float* __restrict__ part, size_t n, int S, floa
   out[i] = v;
 }
 
-// Bias gradient: db[n] = sum_m G^T[n][m] (fp32 sum of the bf16 gradient the weight product also sees).
-__global__ __launch_bounds__(256) void row_sums(const bf16* __restrict__ gT, int M, float* __restrict__ db) {
-  const int n = blockIdx.x;
-  float s = 0.0f;
-  for (int m = threadIdx.x; m < M; m += 256) s += (float)gT[(size_t)n * M + m];
-  __shared__ float red[256];
-  red[threadIdx.x] = s;
+// Bias gradient: db[n] = sum_m G[m][n] (fp32 sum of the bf16 gradient the weight product also sees), NC = 8 columns per
+// group of 256.  Partial sum i of a column holds the rows m = i, i + 256, ..., one per lane, and the 256 partials are
+// added in a binary tree.  A group's rows are 16 bytes of a line: `group` deals 8 neighbouring groups to one XCD, whose
+// L2 then fetches each line once (4,096 x 1,024: 32 columns per group took 12 us, on 32 CUs).  Returns the sum of column
+// 8 * (its group) + threadIdx.x to the threads 0..7, with that column in *c.
+constexpr int NC = 8;
+__device__ __forceinline__ float column_sum(const bf16* __restrict__ g, int M, int ld, int id, int* c) {
+  __shared__ float red[256][NC + 1];
+  const int ngroups = ld / NC;  // a multiple of 16
+  const int group = (id & 7) * (ngroups >> 3) + (id >> 3), t = threadIdx.x;
+  const bf16* gp = g + (size_t)t * ld + group * NC;
+  float s[NC] = {};
+  auto add = [&](const bf16x8 v) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i) s[i] += (float)v[i];
+  };
+  int m = 0;
+  for (; m + 2048 <= M; m += 2048) {
+    bf16x8 v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = *reinterpret_cast<const bf16x8*>(gp + (size_t)(m + 256 * j) * ld);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) add(v[j]);
+  }
+  for (; m + t < M; m += 256) add(*reinterpret_cast<const bf16x8*>(gp + (size_t)m * ld));
+#pragma unroll
+  for (int i = 0; i < NC; ++i) red[t][i] = s[i];
   __syncthreads();
   for (int h = 128; h > 0; h >>= 1) {
-    if ((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+    for (int i = t >> 3; i < h; i += 32) red[i][t & 7] += red[i + h][t & 7];
     __syncthreads();
   }
-  if (threadIdx.x == 0) db[n] = red[0];
+  *c = group * NC + (t & 7);
+  return red[0][t & 7];
 }
 
-// Adam on FP32 master weights; refreshes the BF16 copies W [rows x cols] and W^T [cols x rows] (if wT != null).
-__global__ void adam_update(float* __restrict__ w, float* __restrict__ m1, float* __restrict__ m2,
-                            const float* __restrict__ g, size_t n, int cols, float lr, float b1, float b2, float eps,
-                            float bc1, float bc2, bf16* __restrict__ wb, bf16* __restrict__ wT, int rows) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float a = b1 * m1[i] + (1.0f - b1) * gi;
-  const float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
-  m1[i] = a;
-  m2[i] = b;
-  const float wi = w[i] - lr * (a / bc1) / (sqrtf(b / bc2) + eps);
-  w[i] = wi;
-  if (wb) {
-    const bf16 h = (bf16)wi;
-    wb[i] = h;
-    if (wT) {
-      const size_t r = i / cols, c = i - r * cols;
-      wT[c * rows + r] = h;
+__global__ __launch_bounds__(256) void column_sums(const bf16* __restrict__ g, int M, int ld, float* __restrict__ db) {
+  int c;
+  const float v = column_sum(g, M, ld, blockIdx.x, &c);
+  if (threadIdx.x < NC) db[c] = v;
+}
+
+// Adam on FP32 master weights (n entries, a multiple of 4) and biases (nb entries, a multiple of 64); refreshes the
+// BF16 copy of the weights.  Weight gradient: gw, or with S > 1 the sum of the S partial products in part, in split
+// order, which is stored to gw.  Bias gradient: gb, or with g the column sums of g [M x nb], which are stored to gb; the
+// groups that form them come first and run while the others update the weights.
+struct AdamArgs {
+  float *w, *m1, *m2, *gw;
+  const float* part;
+  size_t n;
+  bf16* wb;
+  float *b, *mb1, *mb2, *gb;
+  const bf16* g;
+  int M, nb;
+  float lr, beta1, beta2, eps, bc1, bc2;
+};
+__device__ __forceinline__ float adam1(const AdamArgs& a, float g, float& m1, float& m2, float w) {
+  m1 = a.beta1 * m1 + (1.0f - a.beta1) * g;
+  m2 = a.beta2 * m2 + (1.0f - a.beta2) * g * g;
+  return w - a.lr * (m1 / a.bc1) / (sqrtf(m2 / a.bc2) + a.eps);
+}
+template <int S>
+__global__ __launch_bounds__(256) void adam_update(AdamArgs a) {
+  const int ngb = a.nb / NC;
+  if ((int)blockIdx.x < ngb) {  // biases
+    int i = blockIdx.x * NC + (threadIdx.x & 7);
+    const float v = a.g ? column_sum(a.g, a.M, a.nb, blockIdx.x, &i) : a.gb[i];
+    if (threadIdx.x < NC) {
+      a.gb[i] = v;
+      a.b[i] = adam1(a, v, a.mb1[i], a.mb2[i], a.b[i]);
     }
+    return;
   }
+  const size_t i = ((size_t)(blockIdx.x - ngb) * 256 + threadIdx.x) * 4;
+  if (i >= a.n) return;
+  auto at = [&](float* p) { return reinterpret_cast<f32x4*>(p + i); };
+  f32x4 m1 = *at(a.m1), m2 = *at(a.m2), w = *at(a.w), g;
+  if constexpr (S > 1) {
+    f32x4 part[S];
+#pragma unroll
+    for (int z = 0; z < S; ++z) part[z] = *reinterpret_cast<const f32x4*>(a.part + (size_t)z * a.n + i);
+    g = part[0];
+#pragma unroll
+    for (int z = 1; z < S; ++z) g = g + part[z];
+    *at(a.gw) = g;
+  } else {
+    g = *at(a.gw);
+  }
+  bf16x4 h;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    float p = m1[t], q = m2[t];
+    w[t] = adam1(a, g[t], p, q, w[t]);
+    m1[t] = p;
+    m2[t] = q;
+    h[t] = (bf16)w[t];
+  }
+  *at(a.m1) = m1;
+  *at(a.m2) = m2;
+  *at(a.w) = w;
+  *reinterpret_cast<bf16x4*>(a.wb + i) = h;
 }
 
-// FP32 -> BF16 copies of a weight matrix in both layouts.
-__global__ void to_bf16(const float* __restrict__ w, size_t n, int cols, int rows, bf16* __restrict__ wb,
-                        bf16* __restrict__ wT) {
+// FP32 -> BF16 copy of a weight matrix.
+__global__ void to_bf16(const float* __restrict__ w, size_t n, bf16* __restrict__ wb) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const bf16 h = (bf16)w[i];
-  wb[i] = h;
-  const size_t r = i / cols, c = i - r * cols;
-  wT[c * rows + r] = h;
-}
-
-__global__ void fill_f32(float* p, size_t n, float v) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
+  if (i < n) wb[i] = (bf16)w[i];
 }
 
 }  // namespace mlp
@@ -415,23 +507,24 @@ int dev_alloc(cloudsc_mlp* m, size_t bytes, void** p) {
   return CLOUDSC_OK;
 }
 
-// Tile choice: the largest tile that divides M and N and still gives at least one group per CU (256 CUs).
-template <int EPI>
+// Tile choice: 256 x 256 where that gives a tile for every CU (256), else 128 x 128 where that gives one for every
+// other CU, else 64 x 64.
+template <int EPI, bool TA = false, bool TB = false>
 hipError_t gemm(const bf16* A, int lda, const bf16* B, int ldb, int M, int N, int K, const mlp::EpiArgs& e,
-                hipStream_t s) {
+                hipStream_t s, int splits = 1) {
   const long groups256 = (M % 256 == 0 && N % 256 == 0) ? (long)(M / 256) * (N / 256) : 0;
-  const long groups256x128 = (M % 256 == 0) ? (long)(M / 256) * (N / 128) : 0;
-  const bool k64 = K % 64 == 0;
-  if (groups256 >= 256 && k64) {
-    hipLaunchKernelGGL((mlp::gemm_tn_dl<EPI, 8>), dim3(N / 256, M / 256), dim3(512), 0, s, A, lda,
-                       B, ldb, K, e);
-  } else if (groups256x128 >= 256 && k64) {
-    hipLaunchKernelGGL((mlp::gemm_tn<EPI, 256, 128, 64>), dim3(N / 128, M / 256), dim3(256), 0, s, A, lda, B, ldb, K,
-                       e);
-  } else {
-    hipLaunchKernelGGL((mlp::gemm_tn<EPI, 128, 128, 32>), dim3(N / 128, M / 128), dim3(256), 0, s, A, lda, B, ldb, K,
-                       e);
+  if constexpr (!TA && !TB && EPI != mlp::EPI_LOSS) {  // (the loss epilogue does not fit that tile's registers)
+    if (groups256 >= 256 && K % 64 == 0 && splits == 1) {
+      hipLaunchKernelGGL((mlp::gemm_tn_dl<EPI, 8>), dim3(N / 256, M / 256), dim3(512), 0, s, A, lda, B, ldb, K, e);
+      return hipGetLastError();
+    }
   }
+  if ((long)(M / 128) * (N / 128) * splits >= 128)
+    hipLaunchKernelGGL((mlp::gemm_ring<EPI, 128, 128, 8, TA, TB>), dim3(N / 128, M / 128, splits), dim3(512), 0, s, A,
+                       lda, B, ldb, K, e);
+  else
+    hipLaunchKernelGGL((mlp::gemm_ring<EPI, 64, 64, 4, TA, TB>), dim3(N / 64, M / 64, splits), dim3(256), 0, s, A, lda, B,
+                       ldb, K, e);
   return hipGetLastError();
 }
 
@@ -446,8 +539,10 @@ int check_batch(const cloudsc_mlp* m, int M) {
 }  // namespace
 
 namespace mlp {
-// Forward pass; train = keep Z and the transposed activations for the backward pass.
-hipError_t forward(cloudsc_mlp* m, const bf16* x, int M, float* y, bool train, hipStream_t s) {
+// Forward pass; with loss, Z and the activations are kept for the backward pass, and the loss against target t with
+// weights wgt and its gradient (into g0) are formed in the output layer's epilogue.
+hipError_t forward(cloudsc_mlp* m, const bf16* x, int M, float* y, const float* t, const float* wgt, hipStream_t s) {
+  const bool train = t != nullptr;
   hipError_t e = hipSuccess;
   const bf16* in = x;
   int ldin = m->din[0];
@@ -458,8 +553,7 @@ hipError_t forward(cloudsc_mlp* m, const bf16* x, int M, float* y, bool train, h
       ea.c = m->z[l];
       ea.ldc = m->dout[l];
       ea.act = m->a[l];
-      ea.actT = m->aT[l];
-      ea.ldt = M;
+      if (train && l == 0) ea.loss = m->loss;  // cleared here
       e = train ? gemm<mlp::EPI_HIDDEN>(in, ldin, m->wb[l], m->din[l], M, m->dout[l], m->din[l], ea, s)
                 : gemm<mlp::EPI_HIDDEN_INF>(in, ldin, m->wb[l], m->din[l], M, m->dout[l], m->din[l], ea, s);
       in = m->a[l];
@@ -467,7 +561,13 @@ hipError_t forward(cloudsc_mlp* m, const bf16* x, int M, float* y, bool train, h
     } else {
       ea.c = y;
       ea.ldc = m->dout[l];
-      e = gemm<mlp::EPI_OUT>(in, ldin, m->wb[l], m->din[l], M, m->dout[l], m->din[l], ea, s);
+      ea.act = m->g0;
+      ea.z = t;
+      ea.wgt = wgt;
+      ea.loss = m->loss;
+      ea.batch = (float)M;
+      e = train ? gemm<mlp::EPI_LOSS>(in, ldin, m->wb[l], m->din[l], M, m->dout[l], m->din[l], ea, s)
+                : gemm<mlp::EPI_OUT>(in, ldin, m->wb[l], m->din[l], M, m->dout[l], m->din[l], ea, s);
     }
   }
   return e;
@@ -476,57 +576,98 @@ hipError_t forward(cloudsc_mlp* m, const bf16* x, int M, float* y, bool train, h
 
 namespace {
 
-// dW = G^T X over the batch (C[dout x din], contraction over M columns).  With few output tiles (one 128x128 tile
-// per CU or less) the contraction is split in S stretches over the grid's z dimension, each into its own partial
-// product in the workspace, which sum_splits then adds in split order (deterministic).
-hipError_t weight_gradient(cloudsc_mlp* m, const bf16* gT, const bf16* xT, int dout, int din, int M,
-                           const mlp::EpiArgs& ew, hipStream_t s) {
+struct AdamStep {
+  float lr, beta1, beta2, eps, bc1, bc2;
+};
+
+AdamStep next_step(const cloudsc_mlp* m, float lr, float beta1, float beta2, float eps) {
+  const float n = (float)(m->step + 1);
+  return AdamStep{lr, beta1, beta2, eps, 1.0f - std::pow(beta1, n), 1.0f - std::pow(beta2, n)};
+}
+
+// Adam on layer l; S > 1: its weight gradient is still in S partial products in the workspace; g: its bias gradient is
+// still to be summed over the M rows of g.
+void adam_layer(cloudsc_mlp* m, int l, int S, const bf16* g, int M, const AdamStep& a, hipStream_t s) {
+  const size_t nw = (size_t)m->din[l] * m->dout[l];
+  const mlp::AdamArgs p{m->w[l],  m->mw[l], m->vw[l], m->gw[l],   m->ws, nw,      m->wb[l], m->b[l], m->mb[l],
+                        m->vb[l], m->gb[l], g, M, m->dout[l], a.lr, a.beta1, a.beta2, a.eps, a.bc1, a.bc2};
+  static_assert(mlp::MAX_SPLIT == 4, "splits are 1, 2 or 4");
+  const dim3 grid(m->dout[l] / mlp::NC + blocks(nw / 4, 256));
+  if (S == 4)
+    hipLaunchKernelGGL(mlp::adam_update<4>, grid, dim3(256), 0, s, p);
+  else if (S == 2)
+    hipLaunchKernelGGL(mlp::adam_update<2>, grid, dim3(256), 0, s, p);
+  else
+    hipLaunchKernelGGL(mlp::adam_update<1>, grid, dim3(256), 0, s, p);
+}
+
+// dW = G^T X over the batch (C[dout x din], contraction over M rows).  With few output tiles (one 128x128 tile per CU or
+// less) the contraction is split in S stretches over the grid's z dimension, each into its own partial product in the
+// workspace; they are added in split order (deterministic) by sum_splits or by Adam.  Returns S in *splits.
+hipError_t weight_gradient(cloudsc_mlp* m, const bf16* g, const bf16* x, int dout, int din, int M, float* gw,
+                           int* splits, hipStream_t s) {
   const long tiles = (long)(dout / mlp::BM) * (din / mlp::BN);
   int S = 1;
   while (S < mlp::MAX_SPLIT && tiles * S < 256 && (M / (2 * S)) % mlp::BK == 0 && M / (2 * S) >= 512) S *= 2;
-  if (S == 1 || dout % mlp::BM || din % mlp::BN || (size_t)S * dout * din > m->ws_elems)
-    return gemm<mlp::EPI_F32>(gT, M, xT, M, dout, din, M, ew, s);
+  if ((size_t)S * dout * din > m->ws_elems) S = 1;
+  *splits = S;
   mlp::EpiArgs ep{};
-  ep.c = m->ws;
+  ep.c = S > 1 ? m->ws : gw;
   ep.ldc = din;
   ep.zstride = (long)dout * din;
-  hipLaunchKernelGGL((mlp::gemm_tn<mlp::EPI_F32, 128, 128, 32>), dim3(din / 128, dout / 128, S), dim3(256), 0, s, gT,
-                     M, xT, M, M / S, ep);
-  const size_t n = (size_t)dout * din;
-  hipLaunchKernelGGL(mlp::sum_splits, dim3(blocks(n, 256)), dim3(256), 0, s, m->ws, n, S, ew.c);
-  return hipGetLastError();
+  return gemm<mlp::EPI_F32, true, true>(g, dout, x, din, dout, din, M / S, ep, s, S);
 }
 
-// Backward pass from the output gradient (g0, g0T hold dY and dY^T); fills gw, gb.
-hipError_t backward(cloudsc_mlp* m, const bf16* xT, int M, hipStream_t s) {
+// Backward pass from the output gradient in g0; fills gw, gb.  With adam, each layer is updated as soon as its weights
+// have been read (its input gradient formed).
+hipError_t backward(cloudsc_mlp* m, const bf16* x, int M, const AdamStep* adam, hipStream_t s) {
   hipError_t e = hipSuccess;
-  bf16 *g = m->g0, *gT = m->g0T, *gn = m->g1, *gnT = m->g1T;
+  bf16 *g = m->g0, *gn = m->g1;
   for (int l = m->nl - 1; l >= 0 && e == hipSuccess; --l) {
-    // dW_l = G^T * X_l : C[dout x din] = gT[dout x M] * (X_l^T [din x M])^T
-    const bf16* xlT = (l == 0) ? xT : m->aT[l - 1];
-    mlp::EpiArgs ew{};
-    ew.c = m->gw[l];
-    ew.ldc = m->din[l];
-    e = weight_gradient(m, gT, xlT, m->dout[l], m->din[l], M, ew, s);
+    const int dout = m->dout[l], din = m->din[l];
+    int S = 1;
+    e = weight_gradient(m, g, l == 0 ? x : m->a[l - 1], dout, din, M, m->gw[l], &S, s);
     if (e != hipSuccess) break;
-    hipLaunchKernelGGL(mlp::row_sums, dim3(m->dout[l]), dim3(256), 0, s, gT, M, m->gb[l]);
-    if (l == 0) break;
-    // dX_l = G * W_l, then times silu'(Z_{l-1}) -> gradient of the previous layer
-    mlp::EpiArgs ed{};
-    ed.ldc = m->din[l];
-    ed.act = gn;
-    ed.actT = gnT;
-    ed.ldt = M;
-    ed.z = m->z[l - 1];
-    e = gemm<mlp::EPI_DHIDDEN>(g, m->dout[l], m->wT[l], m->dout[l], M, m->din[l], m->dout[l], ed, s);
+    if (!adam) {
+      hipLaunchKernelGGL(mlp::column_sums, dim3(dout / mlp::NC), dim3(256), 0, s, g, M, dout, m->gb[l]);
+      const size_t n = (size_t)dout * din;
+      if (S > 1) hipLaunchKernelGGL(mlp::sum_splits, dim3(blocks(n, 256)), dim3(256), 0, s, m->ws, n, S, m->gw[l]);
+    }
+    if (l > 0) {  // dX_l = G * W_l, then times silu'(Z_{l-1}) -> gradient of the previous layer
+      mlp::EpiArgs ed{};
+      ed.ldc = din;
+      ed.act = gn;
+      ed.z = m->z[l - 1];
+      e = gemm<mlp::EPI_DHIDDEN, false, true>(g, dout, m->wb[l], din, M, din, dout, ed, s);
+    }
+    if (adam && e == hipSuccess) adam_layer(m, l, S, g, M, *adam, s);
     std::swap(g, gn);
-    std::swap(gT, gnT);
   }
   if (e == hipSuccess) e = hipGetLastError();
   return e;
 }
 
+// Forward, loss and backward of one batch; with adam, the parameter update too.
+int train_batch(cloudsc_mlp* m, const bf16* x, const float* t, const float* wgt, int M, const AdamStep* adam,
+                hipStream_t s) {
+  hipError_t e = mlp::forward(m, x, M, m->y, t, wgt, s);
+  if (e == hipSuccess) e = backward(m, x, M, adam, s);
+  if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_mlp_gradients", e);
+  return CLOUDSC_OK;
+}
+
 }  // namespace
+
+namespace mlp {
+int train_step(cloudsc_mlp* m, const bf16* x, const float* t, const float* wgt, int M, float lr, hipStream_t s) {
+  const int rc = check_batch(m, M);
+  if (rc) return rc;
+  const AdamStep a = next_step(m, lr, 0.9f, 0.999f, 1e-8f);
+  const int e = train_batch(m, x, t, wgt, M, &a, s);
+  if (!e) m->step += 1;
+  return e;
+}
+}  // namespace mlp
 
 extern "C" {
 
@@ -549,17 +690,17 @@ int cloudsc_mlp_create(cloudsc_mlp_t** out, int n_in, int n_hidden, int n_hidden
   auto F = [&](size_t n, float** p) { return dev_alloc(m, n * sizeof(float), (void**)p); };
   auto H = [&](size_t n, bf16** p) { return dev_alloc(m, n * sizeof(bf16), (void**)p); };
   m->w.resize(m->nl); m->b.resize(m->nl); m->mw.resize(m->nl); m->vw.resize(m->nl); m->mb.resize(m->nl);
-  m->vb.resize(m->nl); m->gw.resize(m->nl); m->gb.resize(m->nl); m->wb.resize(m->nl); m->wT.resize(m->nl);
+  m->vb.resize(m->nl); m->gw.resize(m->nl); m->gb.resize(m->nl); m->wb.resize(m->nl);
   for (int l = 0; l < m->nl && !rc; ++l) {
     const size_t nw = (size_t)m->din[l] * m->dout[l], nb = m->dout[l];
     rc = F(nw, &m->w[l]) || F(nb, &m->b[l]) || F(nw, &m->mw[l]) || F(nw, &m->vw[l]) || F(nb, &m->mb[l]) ||
-         F(nb, &m->vb[l]) || F(nw, &m->gw[l]) || F(nb, &m->gb[l]) || H(nw, &m->wb[l]) || H(nw, &m->wT[l]);
+         F(nb, &m->vb[l]) || F(nw, &m->gw[l]) || F(nb, &m->gb[l]) || H(nw, &m->wb[l]);
   }
-  m->z.resize(m->nl - 1); m->a.resize(m->nl - 1); m->aT.resize(m->nl - 1);
+  m->z.resize(m->nl - 1); m->a.resize(m->nl - 1);
   const size_t mh = (size_t)max_batch * n_hidden;
-  for (int l = 0; l < m->nl - 1 && !rc; ++l) rc = F(mh, &m->z[l]) || H(mh, &m->a[l]) || H(mh, &m->aT[l]);
+  for (int l = 0; l < m->nl - 1 && !rc; ++l) rc = F(mh, &m->z[l]) || H(mh, &m->a[l]);
   const size_t mg = (size_t)max_batch * std::max(n_hidden, n_out);
-  if (!rc) rc = H(mg, &m->g0) || H(mg, &m->g0T) || H(mg, &m->g1) || H(mg, &m->g1T);
+  if (!rc) rc = H(mg, &m->g0) || H(mg, &m->g1);
   if (!rc) rc = F((size_t)max_batch * n_out, &m->y) || F(1, &m->loss);
   size_t wmax = 0;
   for (int l = 0; l < m->nl; ++l) wmax = std::max(wmax, (size_t)m->din[l] * m->dout[l]);
@@ -590,8 +731,7 @@ int cloudsc_mlp_create(cloudsc_mlp_t** out, int n_in, int n_hidden, int n_hidden
     if (e == hipSuccess) e = hipMemset(m->mb[l], 0, m->dout[l] * sizeof(float));
     if (e == hipSuccess) e = hipMemset(m->vb[l], 0, m->dout[l] * sizeof(float));
     if (e == hipSuccess) {
-      hipLaunchKernelGGL(mlp::to_bf16, dim3(blocks(nw, 256)), dim3(256), 0, 0, m->w[l], nw, m->din[l], m->dout[l],
-                         m->wb[l], m->wT[l]);
+      hipLaunchKernelGGL(mlp::to_bf16, dim3(blocks(nw, 256)), dim3(256), 0, 0, m->w[l], nw, m->wb[l]);
       e = hipGetLastError();
     }
   }
@@ -625,7 +765,7 @@ int cloudsc_mlp_forward(cloudsc_mlp_t* m, const uint16_t* x, int M, float* y, vo
   if (!m || !x || !y) return fail(CLOUDSC_ENULL, "cloudsc_mlp_forward: NULL argument");
   int rc = check_batch(m, M);
   if (rc) return rc;
-  hipError_t e = mlp::forward(m, (const bf16*)x, M, y, false, (hipStream_t)stream);
+  hipError_t e = mlp::forward(m, (const bf16*)x, M, y, nullptr, nullptr, (hipStream_t)stream);
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_mlp_forward", e);
   return CLOUDSC_OK;
 }
@@ -635,33 +775,15 @@ int cloudsc_mlp_gradients(cloudsc_mlp_t* m, const uint16_t* x, const uint16_t* x
   if (!m || !x || !xT || !t || !wgt) return fail(CLOUDSC_ENULL, "cloudsc_mlp_gradients: NULL argument");
   int rc = check_batch(m, M);
   if (rc) return rc;
-  hipStream_t s = (hipStream_t)stream;
-  hipError_t e = mlp::forward(m, (const bf16*)x, M, m->y, true, s);
-  if (e == hipSuccess) {
-    const int n = m->dout[m->nl - 1];
-    hipLaunchKernelGGL(mlp::fill_f32, dim3(1), dim3(64), 0, s, m->loss, (size_t)1, 0.0f);
-    hipLaunchKernelGGL(mlp::mse_grad, dim3((n + 63) / 64, (M + 63) / 64), dim3(256), 0, s, m->y, t, wgt, M, n, m->g0,
-                       m->g0T, m->loss);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = backward(m, (const bf16*)xT, M, s);
-  if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_mlp_gradients", e);
-  return CLOUDSC_OK;
+  return train_batch(m, (const bf16*)x, t, wgt, M, nullptr, (hipStream_t)stream);
 }
 
 int cloudsc_mlp_adam(cloudsc_mlp_t* m, float lr, float beta1, float beta2, float eps, void* stream) {
   if (!m) return fail(CLOUDSC_ENULL, "cloudsc_mlp_adam: NULL model");
   hipStream_t s = (hipStream_t)stream;
+  const AdamStep a = next_step(m, lr, beta1, beta2, eps);
   m->step += 1;
-  const float bc1 = 1.0f - std::pow(beta1, (float)m->step), bc2 = 1.0f - std::pow(beta2, (float)m->step);
-  for (int l = 0; l < m->nl; ++l) {
-    const size_t nw = (size_t)m->din[l] * m->dout[l];
-    hipLaunchKernelGGL(mlp::adam_update, dim3(blocks(nw, 256)), dim3(256), 0, s, m->w[l], m->mw[l], m->vw[l],
-                       m->gw[l], nw, m->din[l], lr, beta1, beta2, eps, bc1, bc2, m->wb[l], m->wT[l], m->dout[l]);
-    hipLaunchKernelGGL(mlp::adam_update, dim3(blocks(m->dout[l], 256)), dim3(256), 0, s, m->b[l], m->mb[l],
-                       m->vb[l], m->gb[l], (size_t)m->dout[l], 1, lr, beta1, beta2, eps, bc1, bc2, (bf16*)nullptr,
-                       (bf16*)nullptr, 1);
-  }
+  for (int l = 0; l < m->nl; ++l) adam_layer(m, l, 1, nullptr, 0, a, s);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_mlp_adam", e);
   return CLOUDSC_OK;
@@ -669,9 +791,8 @@ int cloudsc_mlp_adam(cloudsc_mlp_t* m, float lr, float beta1, float beta2, float
 
 int cloudsc_mlp_train_step(cloudsc_mlp_t* m, const uint16_t* x, const uint16_t* xT, const float* t, const float* wgt,
                            int M, float lr, void* stream) {
-  int rc = cloudsc_mlp_gradients(m, x, xT, t, wgt, M, stream);
-  if (rc) return rc;
-  return cloudsc_mlp_adam(m, lr, 0.9f, 0.999f, 1e-8f, stream);
+  if (!m || !x || !xT || !t || !wgt) return fail(CLOUDSC_ENULL, "cloudsc_mlp_gradients: NULL argument");
+  return mlp::train_step(m, (const bf16*)x, t, wgt, M, lr, (hipStream_t)stream);
 }
 
 // Host copies of one layer's parameters (which: 0 = W [dout x din] fp32, 1 = b, 2 = dW, 3 = db, 4 = last output Y
@@ -699,8 +820,7 @@ int cloudsc_mlp_param(cloudsc_mlp_t* m, int layer, int which, float* host, size_
     e = set ? hipMemcpy(p, host, n * sizeof(float), hipMemcpyHostToDevice)
             : hipMemcpy(host, p, n * sizeof(float), hipMemcpyDeviceToHost);
   if (e == hipSuccess && set && which == 0) {
-    hipLaunchKernelGGL(mlp::to_bf16, dim3(blocks(nw, 256)), dim3(256), 0, 0, m->w[layer], nw, m->din[layer],
-                       m->dout[layer], m->wb[layer], m->wT[layer]);
+    hipLaunchKernelGGL(mlp::to_bf16, dim3(blocks(nw, 256)), dim3(256), 0, 0, m->w[layer], nw, m->wb[layer]);
     e = hipDeviceSynchronize();
   }
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_mlp_param", e);

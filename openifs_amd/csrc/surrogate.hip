@@ -98,11 +98,11 @@ __device__ __forceinline__ float target(const KPtrs<float>& p, const Dims& d, in
   }
 }
 
-// Feature matrix X [M x nin] (bf16, standardised) and optionally X^T [nin x M] for columns col0 .. col0+M-1.
+// Feature matrix X [M x nin] (bf16, standardised) for columns col0 .. col0+M-1.
 // Block: 256 threads, tile of 64 columns x 64 matrix entries; columns beyond NGPTOT and padding entries are 0.
 __global__ __launch_bounds__(256) void features(KPtrs<float> p, Dims d, int col0, int M, int nin,
                                                 const float* __restrict__ mu, const float* __restrict__ rsd,
-                                                bf16* __restrict__ X, bf16* __restrict__ XT) {
+                                                bf16* __restrict__ X) {
   __shared__ float tile[TILE][TILE + 1];
   const int c0 = blockIdx.x * TILE, e0 = blockIdx.y * TILE;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
@@ -121,11 +121,6 @@ __global__ __launch_bounds__(256) void features(KPtrs<float> p, Dims d, int col0
     const int c = c0 + i, e = e0 + tx;
     if (c < M && e < nin) X[(size_t)c * nin + e] = (bf16)tile[tx][i];
   }
-  if (XT)
-    for (int i = ty; i < TILE; i += 4) {  // write X^T rows: lanes over columns
-      const int e = e0 + i, c = c0 + tx;
-      if (c < M && e < nin) XT[(size_t)e * M + c] = (bf16)tile[i][tx];
-    }
 }
 
 // Target matrix T [M x nout] (fp32, standardised) for columns col0 .. col0+M-1.
@@ -366,7 +361,7 @@ struct cloudsc_surrogate {
   int klev = 0, nin = 0, nout = 0, max_batch = 0;
   float *mu_x = nullptr, *sd_x = nullptr, *rsd_x = nullptr, *mu_y = nullptr, *sd_y = nullptr, *rsd_y = nullptr;
   float* wgt = nullptr;  // per output entry: 1 for the 6*KLEV targets, 0 for padding
-  bf16 *X = nullptr, *XT = nullptr;
+  bf16* X = nullptr;
   float *T = nullptr, *Y = nullptr, *loss_acc = nullptr;
   // hybrid: selection list and the compact field set
   int* list = nullptr;
@@ -425,8 +420,8 @@ hipError_t predict(cloudsc_surrogate* s, const cloudsc_params_t* q, const KPtrs<
     const int n = std::min(s->max_batch, d.ngptot - c0);
     const int M = surr::pad128(n);
     hipLaunchKernelGGL(surr::features, dim3(nblk(M, surr::TILE), nblk(s->nin, surr::TILE)), dim3(256), 0, st, p, d,
-                       c0, M, s->nin, s->mu_x, s->rsd_x, s->X, (bf16*)nullptr);
-    e = mlp::forward(s->net, s->X, M, s->Y, false, st);
+                       c0, M, s->nin, s->mu_x, s->rsd_x, s->X);
+    e = mlp::forward(s->net, s->X, M, s->Y, nullptr, nullptr, st);
     if (e != hipSuccess) break;
     hipLaunchKernelGGL(surr::outputs, dim3(nblk(M, surr::TILE), nblk(surr::NT * d.klev, surr::TILE)), dim3(256), 0,
                        st, p, d, c0, n, s->nout, s->mu_y, s->sd_y, s->Y, (float)q->rtt, (float)q->rlvtt,
@@ -472,7 +467,6 @@ int cloudsc_surrogate_create(cloudsc_surrogate_t** out, int klev, int n_hidden, 
     rc = F(s->nin, &s->mu_x) || F(s->nin, &s->sd_x) || F(s->nin, &s->rsd_x) || F(s->nout, &s->mu_y) ||
          F(s->nout, &s->sd_y) || F(s->nout, &s->rsd_y) || F(s->nout, &s->wgt) ||
          salloc(s, (size_t)max_batch * s->nin * sizeof(bf16), (void**)&s->X) ||
-         salloc(s, (size_t)max_batch * s->nin * sizeof(bf16), (void**)&s->XT) ||
          F((size_t)max_batch * s->nout, &s->T) || F((size_t)max_batch * s->nout, &s->Y) || F(1, &s->loss_acc) ||
          salloc(s, sizeof(int), (void**)&s->count);
   if (rc) {
@@ -609,12 +603,12 @@ int cloudsc_surrogate_train(cloudsc_surrogate_t* s, float lr, int batch, float* 
   hipError_t e = hipGetLastError();
   for (int c0 = 0; c0 + M <= ngptot && e == hipSuccess; c0 += M, ++nb) {
     hipLaunchKernelGGL(surr::features, dim3(nblk(M, surr::TILE), nblk(s->nin, surr::TILE)), dim3(256), 0, st, p, d,
-                       c0, M, s->nin, s->mu_x, s->rsd_x, s->X, s->XT);
+                       c0, M, s->nin, s->mu_x, s->rsd_x, s->X);
     hipLaunchKernelGGL(surr::targets, dim3(nblk(M, surr::TILE), nblk(s->nout, surr::TILE)), dim3(256), 0, st, p, d,
                        c0, M, s->nout, s->mu_y, s->rsd_y, s->T);
     e = hipGetLastError();
     if (e != hipSuccess) break;
-    rc = cloudsc_mlp_train_step(s->net, (const uint16_t*)s->X, (const uint16_t*)s->XT, s->T, s->wgt, M, lr, stream);
+    rc = mlp::train_step(s->net, s->X, s->T, s->wgt, M, lr, st);
     if (rc) return rc;
     hipLaunchKernelGGL(surr::add_scalar, dim3(1), dim3(64), 0, st, s->loss_acc, s->net->loss);
     e = hipGetLastError();
