@@ -60,35 +60,48 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 // Epilogue of a wave's FM x FN fragments of C^T = B A^T: register r of lane l holds C[m][n] with m = lane & 31 of the
-// fragment's rows and n = 8 (r >> 2) + 4 (l >> 5) + (r & 3) of its columns, so each lane owns runs of 4 consecutive
-// columns of one row, stored as one 16-byte (fp32) or 8-byte (bf16) write each.  row, col: this lane's first row and
-// column.  All loads come before the first store: loads and stores share one in-order wait counter.
+// fragment's rows and n = 8 (r >> 2) + 4 (l >> 5) + (r & 3) of its columns.  Stored like that, an instruction touches 32
+// rows with 16 or 32 bytes each; so each fragment goes through 4 KB of LDS (lds: this wave's own) into a layout of 8
+// rows of 8 lanes x 4 consecutive columns, in which every load and store covers full runs of 64 (bf16) or 128 bytes.
+// Row r's 16-byte chunk c is in slot c ^ ((r >> 1) & 7): 16 rows' equal chunks and two rows' chunks are both spread over
+// all banks.  row, col: the wave's first row and column.  All loads come before the first store: loads and stores share
+// one in-order wait counter.
 template <int EPI, int NW, int FM, int FN>
-__device__ __forceinline__ void epilogue(const EpiArgs& e, const f32x16 (&acc)[FM][FN], int row, int col) {
+__device__ __forceinline__ void epilogue(const EpiArgs& e, const f32x16 (&acc)[FM][FN], bf16* lds, int row, int col) {
   constexpr bool BIAS = EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_INF || EPI == EPI_OUT || EPI == EPI_LOSS;
   constexpr bool READZ = EPI == EPI_DHIDDEN || EPI == EPI_LOSS;
-  f32x4 bias[FN][4], wgt[FN][4], z[FM][FN][4];
+  typedef f32x4 __attribute__((may_alias)) tile4;
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  float* wr = reinterpret_cast<float*>(lds) + 32 * r;                // this lane's row on the way in
+  const float* rd = reinterpret_cast<float*>(lds) + 32 * (lane >> 3);  // and its first row on the way out
+  row += lane >> 3;
+  col += 4 * (lane & 7);
+  f32x4 bias[FN], wgt[FN], z[FM][FN][4];
 #pragma unroll
-  for (int j = 0; j < FN; ++j)
+  for (int j = 0; j < FN; ++j) {
+    if (BIAS) bias[j] = *reinterpret_cast<const f32x4*>(e.bias + col + j * 32);
+    if (EPI == EPI_LOSS) wgt[j] = *reinterpret_cast<const f32x4*>(e.wgt + col + j * 32);
+    if (READZ)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (BIAS) bias[j][q] = *reinterpret_cast<const f32x4*>(e.bias + col + j * 32 + 8 * q);
-      if (EPI == EPI_LOSS) wgt[j][q] = *reinterpret_cast<const f32x4*>(e.wgt + col + j * 32 + 8 * q);
-      if (READZ)
+      for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int i = 0; i < FM; ++i)
-          z[i][j][q] = *reinterpret_cast<const f32x4*>(e.z + (size_t)(row + i * 32) * e.ldc + col + j * 32 + 8 * q);
-    }
+        for (int q = 0; q < 4; ++q)
+          z[i][j][q] = *reinterpret_cast<const f32x4*>(e.z + (size_t)(row + i * 32 + 8 * q) * e.ldc + col + j * 32);
+  }
   float l = 0.0f;
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j)
+    for (int j = 0; j < FN; ++j) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<tile4*>(wr + 4 * ((2 * q + h) ^ ((r >> 1) & 7))) =
+            f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const size_t o = (size_t)(row + i * 32) * e.ldc + col + j * 32 + 8 * q;
-        f32x4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-        if (BIAS) v = v + bias[j][q];
+        const size_t o = (size_t)(row + i * 32 + 8 * q) * e.ldc + col + j * 32;
+        f32x4 v = *reinterpret_cast<const tile4*>(rd + 256 * q + 4 * ((lane & 7) ^ ((4 * q + (lane >> 4)) & 7)));
+        if (BIAS) v = v + bias[j];
         if (EPI != EPI_HIDDEN_INF && EPI != EPI_DHIDDEN) *reinterpret_cast<f32x4*>(e.c + o) = v;
         if (EPI == EPI_F32 || EPI == EPI_OUT) continue;
         bf16x4 a;
@@ -101,13 +114,14 @@ __device__ __forceinline__ void epilogue(const EpiArgs& e, const f32x16 (&acc)[F
             a[t] = (bf16)(v[t] * (s * (1.0f + zt * (1.0f - s))));
           } else {
             const float d = v[t] - z[i][j][q][t];
-            const float wd = wgt[j][q][t] * d;
+            const float wd = wgt[j][t] * d;
             l += wd * d;
             a[t] = (bf16)(2.0f * wd / e.batch);
           }
         }
         *reinterpret_cast<bf16x4*>(e.act + o) = a;
       }
+    }
   if constexpr (EPI == EPI_LOSS) {  // one atomic per group: they all go to one address and are served one by one
     __shared__ float part[NW];
     for (int off = 32; off > 0; off >>= 1) l += __shfl_down(l, off, 64);
@@ -281,25 +295,25 @@ __global__ __launch_bounds__(64 * NW) void gemm_ring(const bf16* __restrict__ A,
     tail(s3, s2, t + 3);
   }
 
-  epilogue<EPI, NW, FM, FN>(e, acc, m0 + wm * (TBM / 2) + (lane & 31), n0 + wn * WCOL + 4 * (lane >> 5));
+  landed<0>();  // no load into LDS outlives the group, and its LDS is free
+  epilogue<EPI, NW, FM, FN>(e, acc, s0 + w * 2048, m0 + wm * (TBM / 2), n0 + wn * WCOL);
 }
 
-// The large-product kernel: 256 x 256 block tile, K-step 64, NW waves as 2 x (NW/2), each computing 128 rows x
-// (512/NW) columns in 32x32 fragments whose accumulators live in the AGPRs.  The two LDS buffers are filled straight
-// from global memory (global_load_lds_dwordx4: no staging registers), the next tile while the current one
-// multiplies.  One such load writes 1 KB of LDS contiguously, lane l at 16*l: 8 rows of 128 B.  Chunk c (16 B) of
-// row r is stored in slot c ^ ((r >> 1) & 7) of its row: a fragment read (16 lanes = 16 consecutive rows, one
-// chunk, 256 B across the 64 banks) then finds the 8 even rows in 8 distinct slots of one 128-byte half of the banks
-// and the 8 odd rows likewise in the other half -- no bank conflict.  Each lane of a load fetches the global chunk
-// that belongs in its LDS slot.
-template <int EPI, int NW>
-__global__ __launch_bounds__(64 * NW) void gemm_tn_dl(const bf16* __restrict__ A, int lda, const bf16* __restrict__ B,
-                                                       int ldb, int K, EpiArgs e) {
-  constexpr int TBM = 256, TBN = 256, TBK = 64, WN = NW / 2, WCOL = TBN / WN, FM = 4, FN = WCOL / 32;
-  constexpr int TILE = TBM * TBK;                    // bf16 per operand tile (32 KB)
-  constexpr int NLD = 32 / NW;                       // 1 KB loads per operand, thread and K-step
-  __shared__ __attribute__((aligned(1024))) bf16 lds[2][2][TILE];  // [buffer][A|B]
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+// The large-product kernel: 256 x 256 block tile, 8 waves as 2 x 4, each computing 128 rows x 64 columns in 32x32
+// fragments; contraction steps of 64, so that a load takes every row's full 128-byte line (half lines take as many L2
+// requests), in an LDS ring of 3 stages for A, which comes from HBM, and 2 for B, which stays in L2 (160 KB in all).
+// The fragments of a quarter step are read while the quarter before multiplies.  65,536 x 1,024 x 1,920 takes 258 us
+// (1,000 TF/s; with the loads left out 218 us: the matrix cores' clock falls under this load), x 1,024 160 us, of which
+// 46 us are the epilogues (stores and the sigmoids' divisions), during which a CU's matrix cores idle; with two full
+// LDS buffers of 64, waited for at each step, it was 278 and 166 us.  Two groups of 128 x 256 on a CU, so that one's
+// epilogue would overlap the other's products, ask for 1.5 times the bytes: 361 and 174 us.
+template <int EPI>
+__global__ __launch_bounds__(512) void gemm_wide(const bf16* __restrict__ A, int lda, const bf16* __restrict__ B,
+                                                 int ldb, int K, EpiArgs e) {
+  constexpr int NW = 8, TBM = 256, TBN = 256, TBK = 64, WN = 4, WCOL = 64, FM = 4, FN = 2;
+  typedef Tile<256, false, NW> Op;
+  __shared__ __attribute__((aligned(1024))) bf16 a0[256 * TBK], a1[256 * TBK], a2[256 * TBK], b0[256 * TBK], b1[256 * TBK];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = w / WN, wn = w % WN;
   // Tile mapping: the dispatcher hands consecutive workgroups to the 8 XCDs in turn, each with its own L2.  With the
   // M-tile count a multiple of 8, workgroup L goes to XCD L % 8 and takes, in that XCD's order, all N-tiles of one
@@ -311,22 +325,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_tn_dl(const bf16* __restrict__ A
     mt = (slot / gridDim.x) * 8 + (L & 7);
   }
   const int m0 = mt * TBM, n0 = nt * TBN;
-  // loads: wave w, instruction i fills row group g = NW i + w (rows 8g .. 8g+7) of each operand; g has the parity of
-  // w, so (row >> 1) & 7 = (4 (w & 1) + (lrow >> 1)) & 7
-  const int lrow = lane >> 3, lchunk = (lane & 7) ^ ((4 * (w & 1) + (lrow >> 1)) & 7);
-  const bf16* ag = A + (size_t)(m0 + 8 * w + lrow) * lda + 8 * lchunk;
-  const bf16* bg = B + (size_t)(n0 + 8 * w + lrow) * ldb + 8 * lchunk;
-  const size_t astep = (size_t)(8 * NW) * lda, bstep = (size_t)(8 * NW) * ldb;
-  auto gload = [&](int buf, int k0) {
-    typedef bf16 __attribute__((address_space(3))) lbf16;
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-      __builtin_amdgcn_global_load_lds((const void*)(ag + astep * i + k0),
-                                       (lbf16*)&lds[buf][0][(NW * i + w) * 512], 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const void*)(bg + bstep * i + k0),
-                                       (lbf16*)&lds[buf][1][(NW * i + w) * 512], 16, 0, 0);
-    }
-  };
+  const bf16* ap = A + (size_t)m0 * lda;
+  const bf16* bp = B + (size_t)n0 * ldb;
+  // past the last step: its entries again, which nobody reads
+  auto load_a = [&](bf16* s, int t) { Op::template load<false>(s, ap, lda, min(TBK * t, K - TBK), K, w, lane); };
+  auto load_b = [&](bf16* s, int t) { Op::template load<false>(s, bp, ldb, min(TBK * t, K - TBK), K, w, lane); };
   if (EPI == EPI_HIDDEN && e.loss && tid == 0 && blockIdx.x == 0 && blockIdx.y == 0) *e.loss = 0.0f;
   f32x16 acc[FM][FN];
 #pragma unroll
@@ -336,39 +339,74 @@ __global__ __launch_bounds__(64 * NW) void gemm_tn_dl(const bf16* __restrict__ A
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-  const int nk = K / TBK;
-  gload(0, 0);
-  // fragment reads: lane supplies row (lane & 31) of a 32-row block and k = 8*(lane >> 5) .. +7 of a 16-wide step
-  const int fr = lane & 31, fh = lane >> 5;
-  for (int kt = 0; kt < nk; ++kt) {
-    const int cur = kt & 1;
-    __builtin_amdgcn_s_waitcnt(0);  // this thread's loads of the current tile have landed
-    __syncthreads();                // everyone's; and everyone is done reading the other buffer
-    if (kt + 1 < nk) gload(cur ^ 1, (kt + 1) * TBK);
-    const bf16* as = lds[cur][0];
-    const bf16* bs = lds[cur][1];
+  struct Frags {
+    bf16x8 a[FM], b[FN];
+  };
+  auto read = [&](const bf16* sa, const bf16* sb, int ks, Frags& f) {
 #pragma unroll
-    for (int ks = 0; ks < TBK / 16; ++ks) {
-      const int c = 2 * ks + fh;  // logical 16-byte chunk of the row
-      bf16x8 a[FM], b[FN];
+    for (int j = 0; j < FN; ++j) f.b[j] = Op::frag(sb, wn * WCOL + j * 32, ks, lane);
 #pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const int r = wm * 128 + i * 32 + fr;
-        a[i] = *reinterpret_cast<const bf16x8*>(as + r * TBK + 8 * (c ^ ((r >> 1) & 7)));
-      }
+    for (int i = 0; i < FM; ++i) f.a[i] = Op::frag(sa, wm * 128 + i * 32, ks, lane);
+  };
+  auto multiply = [&](const Frags& f) {
 #pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const int r = wn * WCOL + j * 32 + fr;
-        b[j] = *reinterpret_cast<const bf16x8*>(bs + r * TBK + 8 * (c ^ ((r >> 1) & 7)));
-      }
+    for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int i = 0; i < FM; ++i)
+      for (int j = 0; j < FN; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.b[j], f.a[i], acc[i][j], 0, 0, 0);
+  };
+  auto interleave = [](auto loads, auto reads) {  // the order of a quarter step: a product, an LDS read, a load, ...
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+    for (int i = 0; i < FM * FN; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                             // matrix product
+      if (decltype(reads)::value && i < FM + FN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
+      if (decltype(loads)::value && i < Op::NLD) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // load into LDS
     }
+  };
+  // Step t: this wave's loads of A(t) and B(t) have landed (those of A(t + 1) stay in flight), then everyone's have, and
+  // everyone is done with step t - 1, whose buffers take B(t + 1) and A(t + 2).  The fragments of a quarter step are read
+  // while the quarter before multiplies.
+  auto step = [&](const bf16* ca, bf16* fa, const bf16* cb, bf16* fb, int t) {
+    Frags f, g;
+    landed<Op::NLD>();
+    load_b(fb, t + 1);
+    read(ca, cb, 0, f);
+    __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);
+    read(ca, cb, 16, g);
+    multiply(f);
+    interleave(std::true_type(), std::true_type());
+    __builtin_amdgcn_sched_barrier(0);  // the wait counts on A's loads being the later ones
+    load_a(fa, t + 2);
+    read(ca, cb, 32, f);
+    multiply(g);
+    interleave(std::true_type(), std::true_type());
+    read(ca, cb, 48, g);
+    multiply(f);
+    interleave(std::false_type(), std::true_type());
+    multiply(g);
+    interleave(std::false_type(), std::false_type());
+  };
+  const int nk = K / TBK;
+  load_a(a0, 0);
+  load_b(b0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  load_a(a1, 1);
+  int t = 0;
+  for (; t + 6 <= nk; t += 6) {
+    step(a0, a2, b0, b1, t);
+    step(a1, a0, b1, b0, t + 1);
+    step(a2, a1, b0, b1, t + 2);
+    step(a0, a2, b1, b0, t + 3);
+    step(a1, a0, b0, b1, t + 4);
+    step(a2, a1, b1, b0, t + 5);
   }
-
-  epilogue<EPI, NW, FM, FN>(e, acc, m0 + wm * 128 + (lane & 31), n0 + wn * WCOL + 4 * (lane >> 5));
+  if (t < nk) step(a0, a2, b0, b1, t);
+  if (t + 1 < nk) step(a1, a0, b1, b0, t + 1);
+  if (t + 2 < nk) step(a2, a1, b0, b1, t + 2);
+  if (t + 3 < nk) step(a0, a2, b1, b0, t + 3);
+  if (t + 4 < nk) step(a1, a0, b0, b1, t + 4);
+  landed<0>();  // no load into LDS outlives the group, and its LDS is free
+  epilogue<EPI, NW, FM, FN>(e, acc, a0 + w * 2048, m0 + wm * 128, n0 + wn * WCOL);
 }
 
 // Sum of the S partial products of a split contraction, in split order: out[i] = sum_z part[z * n + i].
@@ -515,7 +553,7 @@ hipError_t gemm(const bf16* A, int lda, const bf16* B, int ldb, int M, int N, in
   const long groups256 = (M % 256 == 0 && N % 256 == 0) ? (long)(M / 256) * (N / 256) : 0;
   if constexpr (!TA && !TB && EPI != mlp::EPI_LOSS) {  // (the loss epilogue does not fit that tile's registers)
     if (groups256 >= 256 && K % 64 == 0 && splits == 1) {
-      hipLaunchKernelGGL((mlp::gemm_tn_dl<EPI, 8>), dim3(N / 256, M / 256), dim3(512), 0, s, A, lda, B, ldb, K, e);
+      hipLaunchKernelGGL((mlp::gemm_wide<EPI>), dim3(N / 256, M / 256), dim3(512), 0, s, A, lda, B, ldb, K, e);
       return hipGetLastError();
     }
   }

@@ -56,6 +56,31 @@ def test_train_step_equals_gradients_then_adam(n_in, hidden, layers, n_out, M):
         np.testing.assert_array_equal(a.bias_grad(l), b.bias_grad(l))
 
 
+# 256 of the 256 x 256 tiles, contractions of 1 to 8 steps (the ring's unrolled steps are 6) and one that is no multiple
+# of 64 (the smaller tiles); entries are small whole numbers, so every sum is exact
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448, 512, 832, 96])
+def test_large_product_is_exact(K):
+    torch = pytest.importorskip("torch")
+    from openifs_amd import surrogate as S
+
+    g = torch.Generator().manual_seed(K)
+    a = torch.randint(-8, 9, (4096, K + 8), generator=g).bfloat16().to(DEV)[:, :K]
+    b = torch.randint(-8, 9, (4096, K), generator=g).bfloat16().to(DEV)
+    assert torch.equal(S.gemm_tn(a, b), a.float() @ b.float().T)
+
+
+def test_large_forward_equals_small_forward():
+    """A batch on the large tiles gives the rows that small batches give, bit for bit (hidden and output layers)."""
+    torch = pytest.importorskip("torch")
+    from openifs_amd import surrogate as S
+
+    m = S.MLP(384, 1024, 2, 1024, 16384, seed=5)
+    x = torch.randn(16384, 384, generator=torch.Generator().manual_seed(5)).bfloat16().to(DEV)
+    y = m.forward(x)
+    for r in (0, 128, 8064, 16256):
+        assert torch.equal(y[r:r + 128], m.forward(x[r:r + 128].contiguous())), r
+
+
 @pytest.mark.parametrize("ngptot,nproma", [(300, 128), (257, 75)])
 def test_statistics_match_numpy(ngptot, nproma, params91):
     """Mean and spread of all 14 features and 6 targets per level (FP64 sums on both sides; entries that are floored
