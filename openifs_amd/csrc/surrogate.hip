@@ -252,63 +252,204 @@ __global__ __launch_bounds__(256) void targets(KPtrs<float> p, Dims d, int col0,
   }
 }
 
-// Network output Y [M x nout] (standardised) -> CLOUDSC outputs of columns col0 .. col0+M-1.
-__global__ __launch_bounds__(256) void outputs(KPtrs<float> p, Dims d, int col0, int M, int nout,
-                                               const float* __restrict__ mu, const float* __restrict__ sd,
-                                               const float* __restrict__ Y, float rtt, float rlvtt, float rlstt,
-                                               int ncldtop) {
+// Where a tendency goes: as Src, t = 0 .. 4.
+struct Dst {
+  float* p;
+  int s, n;
+};
+__device__ __forceinline__ Dst tendency_dst(const KPtrs<float>& p, int t) {
+  float* q = p.tloc_cld;
+  q = t == 0 ? p.tloc_t : q;
+  q = t == 1 ? p.tloc_q : q;
+  q = t == 2 ? p.tloc_a : q;
+  return Dst{q, t >= 3 ? t - 3 : 0, t >= 3 ? 5 : 1};
+}
+
+constexpr int NP_C = 128;  // NPROMA of the compact field set of the hybrid entry
+
+// Network output Y [M x nout] (standardised) -> tendencies and precipitation fluxes of columns col0 .. col0+M-1, by the
+// transpose of `features` the other way.  MERGE: a column with rank[column] >= 0 takes that column of the compact field
+// set pc (the plain kernel's results) instead.  Writing the plain results over the network's afterwards touched every
+// line a rerun column is in a second time, for 4 of its bytes: 780 us for 3 % of 262,144 columns x L137.  65,536 columns
+// (630 MB): 146 us; with the diagnostics below, 11 of the 22 fields written, stored per entry here, 285 us.
+template <bool MERGE>
+__global__ __launch_bounds__(256) void outputs(KPtrs<float> p, KPtrs<float> pc, const int* __restrict__ rank, Dims d,
+                                               int col0, int M, int nout, const float* __restrict__ mu,
+                                               const float* __restrict__ sd, const float* __restrict__ Y, float rtt,
+                                               float rlvtt, float rlstt) {
   __shared__ float tile[TILE][TILE + 1];
   const int c0 = blockIdx.x * TILE, e0 = blockIdx.y * TILE;
   const int tx = threadIdx.x & 63, ty = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int ntk = NT * d.klev, L = d.klev, np = d.nproma;
+  const int L = d.klev, np = d.nproma, ntk = NT * L;
   {
-    const int e = e0 + tx;
-    const float s = e < ntk ? sd[e] : 0.0f, m = e < ntk ? mu[e] : 0.0f;
-#pragma unroll 8
-    for (int i = ty; i < TILE; i += 4) {  // read Y rows: lanes over entries
-      const int c = c0 + i;
-      tile[tx][i] = (c < M && e < ntk) ? Y[(size_t)c * nout + e] * s + m : 0.0f;
-    }
+    const int e = min(e0 + tx, ntk - 1);
+    const float s = sd[e], m = mu[e];
+    float y[ENT];
+#pragma unroll
+    for (int i = 0; i < ENT; ++i) y[i] = Y[(size_t)min(c0 + ENT * ty + i, M - 1) * nout + e];  // lanes over entries
+#pragma unroll
+    for (int i = 0; i < ENT; ++i) tile[tx][ENT * ty + i] = y[i] * s + m;
   }
   __syncthreads();
-  if (c0 + tx >= M || col0 + c0 + tx >= d.ngptot) return;
-  const Col c = column(col0 + c0 + tx, np);
-  for (int i = ty; i < TILE; i += 4) {  // write fields: lanes over columns
-    const int e = e0 + i;
-    if (e >= ntk) break;
-    const int t = e / L, k = e - t * L;
-    const float v = tile[i][tx];
-    const size_t i2 = fidx(c, k, 0, 1, L, np);
-    switch (t) {
-      case 0: p.tloc_t[i2] = v; break;
-      case 1: p.tloc_q[i2] = v; break;
-      case 2: p.tloc_a[i2] = v; break;
-      case 3: case 4:
-        p.tloc_cld[fidx(c, k, t - 3, 5, L, np)] = v;
-        p.tloc_cld[fidx(c, k, t - 1, 5, L, np)] = 0.0f;  // rain and snow tendencies are not predicted
-        break;
-      default: {
-        const float pr = fmaxf(v, 0.0f);
-        const bool liquid = p.pt[i2] > rtt;
-        const float fl = liquid ? pr : 0.0f, fs = liquid ? 0.0f : pr;
-        const size_t h = fidx(c, k + 1, 0, 1, L + 1, np);
-        p.pfplsl[h] = fl;
-        p.pfplsn[h] = fs;
-        p.pfhpsl[h] = -rlvtt * fl;
-        p.pfhpsn[h] = -rlstt * fs;
-        if (k >= ncldtop - 1) p.pcovptot[i2] = 0.0f;  // the plain kernel's write set
-        float* ddh[10] = {p.pfsqlf, p.pfsqif, p.pfcqnng, p.pfcqlng, p.pfsqrf,
-                          p.pfsqsf, p.pfcqrng, p.pfcqsng, p.pfsqltur, p.pfsqitur};
-        for (int j = 0; j < 10; ++j) ddh[j][h] = 0.0f;
-        if (k == 0) {
-          const size_t h0 = fidx(c, 0, 0, 1, L + 1, np);
-          p.pfplsl[h0] = 0.0f;
-          p.pfplsn[h0] = 0.0f;
-          p.pfhpsl[h0] = 0.0f;
-          p.pfhpsn[h0] = 0.0f;
-          for (int j = 0; j < 10; ++j) ddh[j][h0] = 0.0f;
-          p.prainfrac_toprfz[fidx(c, 0, 0, 1, 1, np)] = 0.0f;
+  const int eb = e0 + ENT * ty, col = col0 + c0 + tx;
+  if (eb >= ntk || c0 + tx >= M || col >= d.ngptot) return;
+  const Col c = column(col, np);
+  const int r = MERGE ? rank[col] : -1;
+  const Col q = column(r < 0 ? 0 : r, NP_C);
+  float v[ENT];
+#pragma unroll
+  for (int i = 0; i < ENT; ++i) v[i] = tile[ENT * ty + i][tx];
+  if (eb < 5 * L) {  // tendencies
+    const int t0 = eb / L, k0 = eb - t0 * L;
+    float w[ENT];  // rain and snow, which the network does not predict, go with cloud liquid and ice
+#pragma unroll
+    for (int i = 0; i < ENT; ++i) w[i] = 0.0f;
+    if (MERGE && r >= 0) {
+      int t = t0, k = k0;
+      Dst x = tendency_dst(pc, t);
+      size_t o = fidx(q, k, x.s, x.n, L, NP_C);
+#pragma unroll
+      for (int i = 0; i < ENT; ++i) {
+        if (eb + i < 5 * L) {
+          v[i] = x.p[o];
+          if (t >= 3) w[i] = x.p[o + (size_t)2 * L * NP_C];
         }
+        if (k + 1 < L) {
+          ++k;
+          o += NP_C;
+        } else if (t + 1 < 5) {
+          k = 0;
+          x = tendency_dst(pc, ++t);
+          o = fidx(q, 0, x.s, x.n, L, NP_C);
+        }
+      }
+    }
+    int t = t0, k = k0;
+    Dst x = tendency_dst(p, t);
+    size_t o = fidx(c, k, x.s, x.n, L, np);
+#pragma unroll
+    for (int i = 0; i < ENT; ++i) {
+      if (eb + i < 5 * L) {
+        x.p[o] = v[i];
+        if (t >= 3) x.p[o + (size_t)2 * L * np] = w[i];
+      }
+      if (k + 1 < L) {
+        ++k;
+        o += np;
+      } else if (t + 1 < 5) {
+        k = 0;
+        x = tendency_dst(p, ++t);
+        o = fidx(c, 0, x.s, x.n, L, np);
+      }
+    }
+  }
+  if (eb + ENT > 5 * L) {  // precipitation at the lower half level, as rain above freezing, else as snow
+    const int kb = eb - 5 * L;
+    float t[ENT], hl[ENT], hs[ENT], fs[ENT], top[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < ENT; ++i) t[i] = p.pt[fidx(c, min(max(kb + i, 0), L - 1), 0, 1, L, np)];
+#pragma unroll
+    for (int i = 0; i < ENT; ++i) {
+      const float pr = fmaxf(v[i], 0.0f);
+      const bool liquid = t[i] > rtt;
+      v[i] = liquid ? pr : 0.0f;
+      fs[i] = liquid ? 0.0f : pr;
+      hl[i] = -rlvtt * v[i];
+      hs[i] = -rlstt * fs[i];
+    }
+    if (MERGE && r >= 0) {
+#pragma unroll
+      for (int i = 0; i < ENT; ++i) {
+        const size_t h = fidx(q, min(max(kb + i, 0), L - 1) + 1, 0, 1, L + 1, NP_C);
+        v[i] = pc.pfplsl[h];
+        fs[i] = pc.pfplsn[h];
+        hl[i] = pc.pfhpsl[h];
+        hs[i] = pc.pfhpsn[h];
+      }
+      const size_t h = fidx(q, 0, 0, 1, L + 1, NP_C);
+      top[0] = pc.pfplsl[h];
+      top[1] = pc.pfplsn[h];
+      top[2] = pc.pfhpsl[h];
+      top[3] = pc.pfhpsn[h];
+    }
+    auto store = [&](int k, float a, float b, float e, float f) {
+      const size_t h = fidx(c, k, 0, 1, L + 1, np);
+      p.pfplsl[h] = a;
+      p.pfplsn[h] = b;
+      p.pfhpsl[h] = e;
+      p.pfhpsn[h] = f;
+    };
+#pragma unroll
+    for (int i = 0; i < ENT; ++i)
+      if (kb + i >= 0 && kb + i < L) store(kb + i + 1, v[i], fs[i], hl[i], hs[i]);
+    if (kb <= 0) store(0, top[0], top[1], top[2], top[3]);
+  }
+}
+
+// The outputs that the network does not predict: 0 (MERGE: or the compact set's, as above) in the ten flux diagnostics,
+// in PCOVPTOT from NCLDTOP on (the plain kernel's write set) and in PRAINFRAC_TOPRFZ.  A lane takes W consecutive columns
+// (4 where NPROMA and the arrays' addresses allow 16-byte stores) of array blockIdx.y over LEV levels, 8 at a time, so
+// that a rerun column's words are in flight together.  1.6 GB for 262,144 columns: 329 us with 3 % of them merged.
+constexpr int LEV = 32;
+template <bool MERGE, int W>
+__global__ __launch_bounds__(256) void diagnostics(KPtrs<float> p, KPtrs<float> pc, const int* __restrict__ rank, Dims d,
+                                                   int ncldtop) {
+  const int a = blockIdx.y, np = d.nproma;
+  auto array = [&](const KPtrs<float>& g) {
+    float* q = g.prainfrac_toprfz;  // 11
+    q = a == 0 ? g.pfsqlf : q;
+    q = a == 1 ? g.pfsqif : q;
+    q = a == 2 ? g.pfcqnng : q;
+    q = a == 3 ? g.pfcqlng : q;
+    q = a == 4 ? g.pfsqrf : q;
+    q = a == 5 ? g.pfsqsf : q;
+    q = a == 6 ? g.pfcqrng : q;
+    q = a == 7 ? g.pfcqsng : q;
+    q = a == 8 ? g.pfsqltur : q;
+    q = a == 9 ? g.pfsqitur : q;
+    q = a == 10 ? g.pcovptot : q;
+    return q;
+  };
+  const int R = a < 10 ? d.klev + 1 : (a == 10 ? d.klev : 1);  // levels
+  const int klo = a == 10 ? ncldtop - 1 : 0;
+  const int k0 = max(klo, (int)blockIdx.z * LEV), k1 = min(R, (int)(blockIdx.z + 1) * LEV);
+  const int col = (blockIdx.x * 256 + threadIdx.x) * W;
+  if (col >= d.ngptot) return;
+  const int live = min(W, d.ngptot - col);
+  const Col c = column(col, np);
+  float* out = array(p) + c.blk * R * np + c.jl;
+  int r[W];
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    r[i] = MERGE && i < live ? rank[col + i] : -1;
+    any |= r[i] >= 0;
+  }
+  const float* comp = array(pc);
+  constexpr int U = 8;
+  for (int k = k0; k < k1; k += U) {
+    typedef float fw __attribute__((ext_vector_type(W)));
+    float v[U][W] = {};
+    if (MERGE && any) {
+#pragma unroll
+      for (int i = 0; i < W; ++i)
+        if (r[i] >= 0) {
+          const Col q = column(r[i], NP_C);
+#pragma unroll
+          for (int u = 0; u < U; ++u) v[u][i] = comp[fidx(q, min(k + u, R - 1), 0, 1, R, NP_C)];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (k + u >= k1) break;
+      float* o = out + (size_t)(k + u) * np;
+      if (live == W) {
+        fw x;
+#pragma unroll
+        for (int i = 0; i < W; ++i) x[i] = v[u][i];
+        *reinterpret_cast<fw*>(o) = x;
+      } else {
+        for (int i = 0; i < live; ++i) o[i] = v[u][i];
       }
     }
   }
@@ -363,7 +504,8 @@ __global__ void fill_f32(float* p, float v) {
   if (threadIdx.x == 0 && blockIdx.x == 0) p[0] = v;
 }
 
-// Gate score and rerun selection.  Score: max over levels with T < 238 K of q / qsat_mix (FOEEWM with FOEALFA,
+// Gate score and rerun selection (262,144 columns x L137, 430 MB: 169 us loading q and p only below 238 K, one level at a
+// time; 105 us with 8 levels' words in flight).  Score: max over levels with T < 238 K of q / qsat_mix (FOEEWM with FOEALFA,
 // fcttre.func.h).  With flags, each column's selection (seeded 1 % draw or score above the threshold) is stored and
 // each group of 256 columns writes how many it selected, for the compaction below.
 __global__ __launch_bounds__(256) void select_columns(KPtrs<float> p, Dims d, float frac, uint64_t seed, float thr,
@@ -374,12 +516,24 @@ __global__ __launch_bounds__(256) void select_columns(KPtrs<float> p, Dims d, fl
   if (c < d.ngptot) {
     float sc = 0.0f;
     const Col col = column(c, d.nproma);
-    for (int k = 0; k < d.klev; ++k) {
-      const size_t i = fidx(col, k, 0, 1, d.klev, d.nproma);
-      const float t = p.pt[i];
-      if (t >= 238.0f) continue;
-      sc = fmaxf(sc, p.pq[i] / qsat_mix(d.th, t, p.pap[i]));
+    size_t o = fidx(col, 0, 0, 1, d.klev, d.nproma);
+    auto level = [&](float t, float q, float pap) {
+      if (t < 238.0f) sc = fmaxf(sc, q / qsat_mix(d.th, t, pap));
+    };
+    int k = 0;
+    for (; k + 8 <= d.klev; k += 8) {  // the words of 8 levels in flight
+      float t[8], q[8], pap[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        t[i] = p.pt[o + (size_t)i * d.nproma];
+        q[i] = p.pq[o + (size_t)i * d.nproma];
+        pap[i] = p.pap[o + (size_t)i * d.nproma];
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) level(t[i], q[i], pap[i]);
+      o += (size_t)8 * d.nproma;
     }
+    for (; k < d.klev; ++k, o += d.nproma) level(p.pt[o], p.pq[o], p.pap[o]);
     if (score) score[c] = sc;
     if (flags) {
       const synth::Draw u = synth::draw(seed, 0x52455255u /* "RERU" */, (uint32_t)c, 0u);
@@ -418,10 +572,11 @@ __global__ __launch_bounds__(1024) void scan_counts(int* __restrict__ counts, in
   if (t == 1023) *total = part[1023];
 }
 
-// The selected columns in ascending order: list[offset of the group + rank within it] = column.  Ascending order
+// The selected columns in ascending order: list[offset of the group + rank within it] = column, and that place by
+// column (-1: not selected).  Ascending order
 // keeps neighbouring lanes of the gather and scatter on neighbouring blocks of the fields.
 __global__ __launch_bounds__(256) void compact_columns(const uint8_t* __restrict__ flags, const int* __restrict__ offsets,
-                                                       int ngptot, int* __restrict__ list) {
+                                                       int ngptot, int* __restrict__ list, int* __restrict__ rank_of) {
   const int c = blockIdx.x * 256 + threadIdx.x, w = threadIdx.x >> 6;
   const bool sel = c < ngptot && flags[c];
   const uint64_t b = __ballot(sel);
@@ -432,6 +587,7 @@ __global__ __launch_bounds__(256) void compact_columns(const uint8_t* __restrict
   for (int i = 0; i < w; ++i) base += wcount[i];
   const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0));
   if (sel) list[base + rank] = c;
+  if (c < ngptot) rank_of[c] = sel ? base + rank : -1;
 }
 
 // Column copies between a blocked field set (NPROMA = np_full) and a compact one (NPROMA = np_c), for one
@@ -481,14 +637,14 @@ struct cloudsc_surrogate {
   int* list = nullptr;
   int* count = nullptr;
   int list_cap = 0;
+  int* count_host = nullptr;  // pinned
+  hipEvent_t counted = nullptr;
   void* comp = nullptr;
   size_t comp_bytes = 0;
   std::vector<void*> allocs;
 };
 
 namespace {
-
-constexpr int NP_C = 128;  // NPROMA of the compact field set
 
 int salloc(cloudsc_surrogate* s, size_t bytes, void** p) {
   hipError_t e = hipMalloc(p, bytes);
@@ -522,24 +678,38 @@ surr::Sat sat_consts(const cloudsc_params_t* q) {
                    (float)q->rtt,  (float)q->rtice, (float)q->rtwat_rtice_r, (float)q->retv};
 }
 
-// Network prediction for all columns, in batches of max_batch.
+void launch_features(cloudsc_surrogate* s, const KPtrs<float>& p, const surr::Dims& d, int c0, hipStream_t st) {
+  const int M = surr::pad128(std::min(s->max_batch, d.ngptot - c0));
+  hipLaunchKernelGGL(surr::features, dim3(nblk(M, surr::TILE), nblk(s->nin, surr::TILE)), dim3(256), 0, st, p, d, c0, M,
+                     s->nin, s->mu_x, s->rsd_x, s->X);
+}
+
+// Network prediction for all columns, in batches of max_batch, the first of whose features are already there; with rank,
+// columns of rank >= 0 are taken from the compact field set pc instead.
 hipError_t predict(cloudsc_surrogate* s, const cloudsc_params_t* q, const KPtrs<float>& p, const surr::Dims& d,
-                   hipStream_t st) {
+                   const KPtrs<float>& pc, const int* rank, hipStream_t st) {
   hipError_t e = hipSuccess;
   const int ntotal = d.ngpblks * d.nproma;
   if (ntotal > d.ngptot)
     hipLaunchKernelGGL(surr::zero_padding_columns, dim3(nblk(ntotal - d.ngptot, 256)), dim3(256), 0, st,
                        p.prainfrac_toprfz, d.ngptot, ntotal);
+  uintptr_t bits = (uintptr_t)d.nproma * 4;
+  for (const float* x : {p.pfsqlf, p.pfsqif, p.pfcqnng, p.pfcqlng, p.pfsqrf, p.pfsqsf, p.pfcqrng, p.pfcqsng, p.pfsqltur,
+                         p.pfsqitur, p.pcovptot, p.prainfrac_toprfz})
+    bits |= (uintptr_t)x;
+  const bool vec = bits % 16 == 0;
+  auto* diag = rank ? (vec ? surr::diagnostics<true, 4> : surr::diagnostics<true, 1>)
+                    : (vec ? surr::diagnostics<false, 4> : surr::diagnostics<false, 1>);
+  hipLaunchKernelGGL(diag, dim3(nblk(d.ngptot, vec ? 1024 : 256), 12, nblk(d.klev + 1, surr::LEV)), dim3(256), 0, st, p,
+                     pc, rank, d, q->ncldtop);
   for (int c0 = 0; c0 < d.ngptot && e == hipSuccess; c0 += s->max_batch) {
     const int n = std::min(s->max_batch, d.ngptot - c0);
-    const int M = surr::pad128(n);
-    hipLaunchKernelGGL(surr::features, dim3(nblk(M, surr::TILE), nblk(s->nin, surr::TILE)), dim3(256), 0, st, p, d,
-                       c0, M, s->nin, s->mu_x, s->rsd_x, s->X);
-    e = mlp::forward(s->net, s->X, M, s->Y, nullptr, nullptr, st);
+    if (c0 > 0) launch_features(s, p, d, c0, st);
+    e = mlp::forward(s->net, s->X, surr::pad128(n), s->Y, nullptr, nullptr, st);
     if (e != hipSuccess) break;
-    hipLaunchKernelGGL(surr::outputs, dim3(nblk(M, surr::TILE), nblk(surr::NT * d.klev, surr::TILE)), dim3(256), 0,
-                       st, p, d, c0, n, s->nout, s->mu_y, s->sd_y, s->Y, (float)q->rtt, (float)q->rlvtt,
-                       (float)q->rlstt, q->ncldtop);
+    hipLaunchKernelGGL(rank ? surr::outputs<true> : surr::outputs<false>,
+                       dim3(nblk(n, surr::TILE), nblk(surr::NT * d.klev, surr::TILE)), dim3(256), 0, st, p, pc, rank, d,
+                       c0, n, s->nout, s->mu_y, s->sd_y, s->Y, (float)q->rtt, (float)q->rlvtt, (float)q->rlstt);
     e = hipGetLastError();
   }
   return e;
@@ -583,6 +753,9 @@ int cloudsc_surrogate_create(cloudsc_surrogate_t** out, int klev, int n_hidden, 
          salloc(s, (size_t)max_batch * s->nin * sizeof(bf16), (void**)&s->X) ||
          F((size_t)max_batch * s->nout, &s->T) || F((size_t)max_batch * s->nout, &s->Y) || F(1, &s->loss_acc) ||
          salloc(s, sizeof(int), (void**)&s->count);
+  if (!rc && (hipHostMalloc((void**)&s->count_host, sizeof(int), hipHostMallocDefault) != hipSuccess ||
+              hipEventCreateWithFlags(&s->counted, hipEventDisableTiming) != hipSuccess))
+    rc = fail(CLOUDSC_ENOMEM, "cloudsc_surrogate_create: pinned count or event");
   if (rc) {
     cloudsc_surrogate_destroy(s);
     return rc < 0 ? rc : CLOUDSC_ENOMEM;
@@ -611,6 +784,8 @@ int cloudsc_surrogate_destroy(cloudsc_surrogate_t* s) {
   for (void* p : s->allocs) (void)hipFree(p);
   if (s->list) (void)hipFree(s->list);
   if (s->comp) (void)hipFree(s->comp);
+  if (s->count_host) (void)hipHostFree(s->count_host);
+  if (s->counted) (void)hipEventDestroy(s->counted);
   delete s;
   return CLOUDSC_OK;
 }
@@ -739,7 +914,8 @@ int cloudsc_surrogate_predict_sp(cloudsc_surrogate_t* s, CLOUDSC_BLOCKED_ARGS(fl
   SURR_PTRS;
   int rc = check_fields(s, ydparams, ngptot, nproma, klev, ngpblks, p);
   if (rc) return rc;
-  hipError_t e = predict(s, ydparams, p, d, st);
+  launch_features(s, p, d, 0, st);
+  hipError_t e = predict(s, ydparams, p, d, p, nullptr, st);
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_surrogate_predict_sp", e);
   return CLOUDSC_OK;
 }
@@ -765,63 +941,71 @@ int cloudsc_hybrid_sp_c(cloudsc_surrogate_t* s, float rerun_fraction, uint64_t r
       !p.pmfu || !p.pmfd)
     return fail(CLOUDSC_ENULL, "cloudsc_hybrid_sp_c: NULL array on the default path");
   const cloudsc_params_t* q = ydparams;
-  // 1. network on every column
-  hipError_t e = predict(s, q, p, d, st);
-  if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: prediction", e);
-  // 2. columns for the plain kernel
-  // selection list (ngptot ints), per-group counts and offsets, per-column flags: one allocation
+  // 1. columns for the plain kernel
+  // selection list and ranks (2 ngptot ints), per-group counts and offsets, per-column flags: one allocation
+  hipError_t e = hipSuccess;
   const int ngroups = (int)nblk(ngptot, 256);
   if (s->list_cap < ngptot) {
     if (s->list) (void)hipFree(s->list);
     s->list = nullptr;
     s->list_cap = 0;
-    e = hipMalloc((void**)&s->list, (size_t)(ngptot + ngroups) * sizeof(int) + (size_t)ngptot);
+    e = hipMalloc((void**)&s->list, (size_t)(2L * ngptot + ngroups) * sizeof(int) + (size_t)ngptot);
     if (e != hipSuccess) return fail(CLOUDSC_ENOMEM, "cloudsc_hybrid_sp_c: hipMalloc", e);
     s->list_cap = ngptot;
   }
-  int* group_offsets = s->list + ngptot;
+  int* rank = s->list + ngptot;
+  int* group_offsets = rank + ngptot;
   uint8_t* flags = reinterpret_cast<uint8_t*>(group_offsets + ngroups);
   hipLaunchKernelGGL(surr::select_columns, dim3(ngroups), dim3(256), 0, st, p, d, rerun_fraction, rerun_seed,
                      gate_threshold, (float*)nullptr, flags, group_offsets);
   hipLaunchKernelGGL(surr::scan_counts, dim3(1), dim3(1024), 0, st, group_offsets, ngroups, s->count);
-  hipLaunchKernelGGL(surr::compact_columns, dim3(ngroups), dim3(256), 0, st, flags, group_offsets, ngptot, s->list);
-  int nsel = 0;
+  hipLaunchKernelGGL(surr::compact_columns, dim3(ngroups), dim3(256), 0, st, flags, group_offsets, ngptot, s->list, rank);
   e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(&nsel, s->count, sizeof(int), hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (e == hipSuccess) e = hipMemcpyAsync(s->count_host, s->count, sizeof(int), hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess) e = hipEventRecord(s->counted, st);
+  if (e == hipSuccess) {
+    launch_features(s, p, d, 0, st);  // runs while the host learns the count
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) e = hipEventSynchronize(s->counted);
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: selection", e);
+  const int nsel = *s->count_host;
   if (n_plain) *n_plain = nsel;
-  if (nsel == 0) return CLOUDSC_OK;
-  // 3. compact field set of the selected columns
+  if (nsel == 0) {
+    e = predict(s, q, p, d, p, nullptr, st);
+    if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: prediction", e);
+    return CLOUDSC_OK;
+  }
+  // 2. compact field set of the selected columns
+  constexpr int NP_C = surr::NP_C;
   const int ncb = (nsel + NP_C - 1) / NP_C;
   const long L = klev, c2 = (long)NP_C * L, ch = (long)NP_C * (L + 1), c1 = NP_C;
   struct Arr {
     void* full;
     int n, L;   // species, levels per species
-    bool in, out;
-    int nout;   // species written (tloc_cld: 4 of 5)
+    bool in;
   };
-  Arr arrs[] = {{(void*)p.pt, 1, (int)L, true, false, 0},        {(void*)p.pq, 1, (int)L, true, false, 0},
-                {(void*)p.tcml_t, 1, (int)L, true, false, 0},    {(void*)p.tcml_q, 1, (int)L, true, false, 0},
-                {(void*)p.tcml_a, 1, (int)L, true, false, 0},    {(void*)p.tcml_cld, 5, (int)L, true, false, 0},
-                {(void*)p.tloc_t, 1, (int)L, false, true, 1},    {(void*)p.tloc_q, 1, (int)L, false, true, 1},
-                {(void*)p.tloc_a, 1, (int)L, false, true, 1},    {(void*)p.tloc_cld, 5, (int)L, false, true, 4},
-                {(void*)p.pvfl, 1, (int)L, true, false, 0},      {(void*)p.pvfi, 1, (int)L, true, false, 0},
-                {(void*)p.pap, 1, (int)L, true, false, 0},       {(void*)p.paph, 1, (int)L + 1, true, false, 0},
-                {(void*)p.plsm, 1, 1, true, false, 0},           {(void*)p.ldcum, 1, 1, true, false, 0},
-                {(void*)p.ktype, 1, 1, true, false, 0},          {(void*)p.peis, 1, 1, true, false, 0},
-                {(void*)p.plu, 1, (int)L, true, false, 0},       {(void*)p.plude, 1, (int)L, true, true, 1},
-                {(void*)p.pludeli, 4, (int)L, true, false, 0},   {(void*)p.psnde, 2, (int)L, true, false, 0},
-                {(void*)p.pmfu, 1, (int)L, true, false, 0},      {(void*)p.pmfd, 1, (int)L, true, false, 0},
-                {(void*)p.pa, 1, (int)L, true, false, 0},        {(void*)p.pclv, 5, (int)L, true, false, 0},
-                {(void*)p.pcovptot, 1, (int)L, true, true, 1},  {(void*)p.prainfrac_toprfz, 1, 1, false, true, 1},
-                {(void*)p.pfsqlf, 1, (int)L + 1, false, true, 1}, {(void*)p.pfsqif, 1, (int)L + 1, false, true, 1},
-                {(void*)p.pfcqnng, 1, (int)L + 1, false, true, 1}, {(void*)p.pfcqlng, 1, (int)L + 1, false, true, 1},
-                {(void*)p.pfsqrf, 1, (int)L + 1, false, true, 1}, {(void*)p.pfsqsf, 1, (int)L + 1, false, true, 1},
-                {(void*)p.pfcqrng, 1, (int)L + 1, false, true, 1}, {(void*)p.pfcqsng, 1, (int)L + 1, false, true, 1},
-                {(void*)p.pfsqltur, 1, (int)L + 1, false, true, 1}, {(void*)p.pfsqitur, 1, (int)L + 1, false, true, 1},
-                {(void*)p.pfplsl, 1, (int)L + 1, false, true, 1}, {(void*)p.pfplsn, 1, (int)L + 1, false, true, 1},
-                {(void*)p.pfhpsl, 1, (int)L + 1, false, true, 1}, {(void*)p.pfhpsn, 1, (int)L + 1, false, true, 1}};
+  Arr arrs[] = {{(void*)p.pt, 1, (int)L, true},        {(void*)p.pq, 1, (int)L, true},
+                {(void*)p.tcml_t, 1, (int)L, true},    {(void*)p.tcml_q, 1, (int)L, true},
+                {(void*)p.tcml_a, 1, (int)L, true},    {(void*)p.tcml_cld, 5, (int)L, true},
+                {(void*)p.tloc_t, 1, (int)L, false},    {(void*)p.tloc_q, 1, (int)L, false},
+                {(void*)p.tloc_a, 1, (int)L, false},    {(void*)p.tloc_cld, 5, (int)L, false},
+                {(void*)p.pvfl, 1, (int)L, true},      {(void*)p.pvfi, 1, (int)L, true},
+                {(void*)p.pap, 1, (int)L, true},       {(void*)p.paph, 1, (int)L + 1, true},
+                {(void*)p.plsm, 1, 1, true},           {(void*)p.ldcum, 1, 1, true},
+                {(void*)p.ktype, 1, 1, true},          {(void*)p.peis, 1, 1, true},
+                {(void*)p.plu, 1, (int)L, true},       {(void*)p.plude, 1, (int)L, true},
+                {(void*)p.pludeli, 4, (int)L, true},   {(void*)p.psnde, 2, (int)L, true},
+                {(void*)p.pmfu, 1, (int)L, true},      {(void*)p.pmfd, 1, (int)L, true},
+                {(void*)p.pa, 1, (int)L, true},        {(void*)p.pclv, 5, (int)L, true},
+                {(void*)p.pcovptot, 1, (int)L, false},  {(void*)p.prainfrac_toprfz, 1, 1, false},
+                {(void*)p.pfsqlf, 1, (int)L + 1, false}, {(void*)p.pfsqif, 1, (int)L + 1, false},
+                {(void*)p.pfcqnng, 1, (int)L + 1, false}, {(void*)p.pfcqlng, 1, (int)L + 1, false},
+                {(void*)p.pfsqrf, 1, (int)L + 1, false}, {(void*)p.pfsqsf, 1, (int)L + 1, false},
+                {(void*)p.pfcqrng, 1, (int)L + 1, false}, {(void*)p.pfcqsng, 1, (int)L + 1, false},
+                {(void*)p.pfsqltur, 1, (int)L + 1, false}, {(void*)p.pfsqitur, 1, (int)L + 1, false},
+                {(void*)p.pfplsl, 1, (int)L + 1, false}, {(void*)p.pfplsn, 1, (int)L + 1, false},
+                {(void*)p.pfhpsl, 1, (int)L + 1, false}, {(void*)p.pfhpsn, 1, (int)L + 1, false}};
   const int narr = sizeof(arrs) / sizeof(arrs[0]);
   size_t offs[sizeof(arrs) / sizeof(arrs[0])], need = 0;
   for (int i = 0; i < narr; ++i) {
@@ -837,31 +1021,28 @@ int cloudsc_hybrid_sp_c(cloudsc_surrogate_t* s, float rerun_fraction, uint64_t r
     s->comp_bytes = need;
   }
   char* cb = (char*)s->comp;
-  auto slices = [&](bool inputs, surr::Slices& sl) {
-    sl.n = 0;
-    for (int i = 0; i < narr; ++i) {
-      const Arr& a = arrs[i];
-      if (inputs ? !a.in : !a.out) continue;
-      const int ns = inputs ? a.n : a.nout;
-      for (int sp = 0; sp < ns; ++sp) {
-        surr::Slice& x = sl.s[sl.n++];
-        x.full = (uint32_t*)a.full;
-        x.comp = (uint32_t*)(cb + offs[i]);
-        x.full_stride = (long)nproma * a.n * a.L;
-        x.comp_stride = (long)NP_C * a.n * a.L;
-        x.full_off = (long)nproma * sp * a.L;
-        x.comp_off = (long)NP_C * sp * a.L;
-        x.L = a.L;
-      }
+  surr::Slices sl;
+  auto add_slices = [&](int i) {
+    const Arr& a = arrs[i];
+    for (int sp = 0; sp < a.n; ++sp) {
+      surr::Slice& x = sl.s[sl.n++];
+      x.full = (uint32_t*)a.full;
+      x.comp = (uint32_t*)(cb + offs[i]);
+      x.full_stride = (long)nproma * a.n * a.L;
+      x.comp_stride = (long)NP_C * a.n * a.L;
+      x.full_off = (long)nproma * sp * a.L;
+      x.comp_off = (long)NP_C * sp * a.L;
+      x.L = a.L;
     }
   };
-  surr::Slices sl;
-  slices(true, sl);
+  sl.n = 0;
+  for (int i = 0; i < narr; ++i)
+    if (arrs[i].in) add_slices(i);
   const unsigned gx = std::min<unsigned>(nblk((long)nsel * (L + 1), 256), 4096u);
   hipLaunchKernelGGL(surr::copy_columns, dim3(gx, sl.n), dim3(256), 0, st, sl, s->list, nsel, nproma, NP_C, 1);
   e = hipGetLastError();
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: gather", e);
-  // 4. plain kernel on the compact set
+  // 3. plain kernel on the compact set
   auto C = [&](int i) { return (float*)(cb + offs[i]); };
   KPtrs<float> pc;
   pc.pt = C(0); pc.pq = C(1); pc.tcml_t = C(2); pc.tcml_q = C(3); pc.tcml_a = C(4); pc.tcml_cld = C(5);
@@ -875,8 +1056,12 @@ int cloudsc_hybrid_sp_c(cloudsc_surrogate_t* s, float rerun_fraction, uint64_t r
   const KDims kd{nsel, NP_C, klev, ncb, 1, NP_C};
   e = cloudsc_gpu::launch_cloudsc<float, float>(*q, (double)ptsphy, pc, kd, 0, st);
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: plain kernel", e);
-  // 5. scatter the plain results over the network's
-  slices(false, sl);
+  // 4. network on every other column
+  e = predict(s, q, p, d, pc, rank, st);
+  if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: prediction", e);
+  // 5. PLUDE, a feature that the plain kernel also updates
+  sl.n = 0;
+  add_slices(19);
   hipLaunchKernelGGL(surr::copy_columns, dim3(gx, sl.n), dim3(256), 0, st, sl, s->list, nsel, nproma, NP_C, 0);
   e = hipGetLastError();
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: scatter", e);
