@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "fp64_math.h"
 
 namespace cloudsc_gpu {
 
@@ -28,6 +29,26 @@ __device__ __forceinline__ float m_log(float x) { return logf(x); }
 __device__ __forceinline__ double m_exp(double x) { return exp(x); }
 __device__ __forceinline__ double m_pow(double x, double y) { return pow(x, y); }
 __device__ __forceinline__ double m_log(double x) { return log(x); }
+// The CLOUDSC sweep's exponentials and powers: FP32 as above, FP64 by the table functions, which suit a kernel that runs
+// one or two waves to a SIMD (the point kernels, with 3 and more waves, are 2 to 4 % slower with them).
+// s_pow(s_base(x), y) = x^y, and s_base_pow(b, y) is the base x^y: in FP64 the logarithm, two thirds of a power, is taken
+// once for several powers of a base, and a power that only serves as a base not at all; FP32's is two instructions,
+// which the compiler shares by itself.
+struct Base32 {
+  float x;
+};
+__device__ __forceinline__ float s_exp(float x) { return m_exp(x); }
+__device__ __forceinline__ Base32 s_base(float x) { return Base32{x}; }
+__device__ __forceinline__ float s_pow(Base32 b, float y) { return m_pow(b.x, y); }
+__device__ __forceinline__ Base32 s_base_pow(Base32 b, float y) { return Base32{m_pow(b.x, y)}; }
+__device__ __forceinline__ float s_pow15(float x) { return m_pow(x, 1.5f); }
+__device__ __forceinline__ double s_exp(double x) { return fp64::exp(x); }
+__device__ __forceinline__ fp64::Log s_base(double x) { return fp64::log(x); }
+__device__ __forceinline__ double s_pow(const fp64::Log& b, double y) { return fp64::pow(b, y); }
+__device__ __forceinline__ fp64::Log s_base_pow(const fp64::Log& b, double y) { return fp64::log_of_pow(b, y); }
+__device__ __forceinline__ double s_pow15(double x) { return x * sqrt(x); }
+template <typename R>
+__device__ __forceinline__ R s_pow(R x, R y) { return s_pow(s_base(x), y); }
 #ifdef CLOUDSC_FAST_DIV
 // FP32 division as reciprocal (v_rcp_f32, 1 ulp) times numerator instead of the ~10-instruction
 // IEEE sequence.  Measured against the FP64 oracle on 8192 L137 columns, the FP32 kernel's
@@ -64,18 +85,19 @@ template <typename T>
 struct Sat {
   T alfa, el, ei;  // FOEALFA, EXP(R3LES*(T-RTT)/(T-R4LES)), EXP(R3IES*(T-RTT)/(T-R4IES))
 };
-template <typename T, typename KCT>
+template <typename T, typename KCT, bool SWEEP = false>
 __device__ __forceinline__ Sat<T> saturation(const KCT& c, T t) {
   Sat<T> s;
   T x = (m_max(c.rtice, m_min(c.rtwat, t)) - c.rtice) * c.rtwat_rtice_r;
   s.alfa = m_min(T(1), x * x);
-  s.el = m_exp(m_div(c.r3les * (t - c.rtt), t - c.r4les));
-  s.ei = m_exp(m_div(c.r3ies * (t - c.rtt), t - c.r4ies));
+  const T xl = m_div(c.r3les * (t - c.rtt), t - c.r4les), xi = m_div(c.r3ies * (t - c.rtt), t - c.r4ies);
+  s.el = SWEEP ? s_exp(xl) : m_exp(xl);
+  s.ei = SWEEP ? s_exp(xi) : m_exp(xi);
   return s;
 }
 
 // CLOUD_SUPERSATCHECK for one point, KFTLIQICE = 1 (cloud_supersatcheck.F90:111-226).
-template <typename T, typename KCT>
+template <typename T, typename KCT, bool SWEEP = false>
 __device__ __forceinline__ void supersatcheck(const KCT& c, T pt, T pq, T pa, T pp, T& t_adj, T& q_adj,
                                               T& a_adj, T& l_adj, T& i_adj) {
   const T zepsec = T(1.e-14);
@@ -83,7 +105,7 @@ __device__ __forceinline__ void supersatcheck(const KCT& c, T pt, T pq, T pa, T 
   T zt = m_max(pt, T(160));
   T za = m_max(m_min(pa, T(1)), T(0));
   const T zp_r = m_div(T(1), pp);
-  const Sat<T> s = saturation<T, KCT>(c, zt);
+  const Sat<T> s = saturation<T, KCT, SWEEP>(c, zt);
   const T foeeliq = c.r2es * s.el;
   const T zfoeeliq = m_min(foeeliq * zp_r, T(0.5));
   // FOEEW: water above RTT, ice below (FOEDELTA = MAX(0,SIGN(1,T-RTT)))

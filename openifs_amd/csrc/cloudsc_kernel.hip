@@ -108,7 +108,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
   const R zadvw = (ktype == 1 && c.rmfadvw > R(0)) ? R(1) - c.rmfadvw : R(1);                  // :696-703
   const R zadvwd = (ktype == 1 && c.rmfadvw > R(0)) ? R(1) - c.rmfadvw * c.rmfadvwdd : R(1);
   const R zconst = plsm > R(0.5) ? c.rcl_kk_cloud_num_land : c.rcl_kk_cloud_num_sea;          // :2063-2069
-  const R zconst_pow = m_pow(zconst, c.rcl_kkbaun);
+  const R zconst_pow = s_pow(zconst, c.rcl_kkbaun);
   const int ncldtop0 = c.ncldtop - 1;  // 0-based first level of the cloud scheme
 
   // Level-carried state (:1205-1211 and :1011)
@@ -140,9 +140,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
   // (FP32 138 -> 140, mixed 167 -> 166).  With the bases read where they are used (above), same box: mixed 655,360 x
   // L137 4.17 -> 3.84 ms, FP32 327,680 x L137 2.24 -> 2.02 ms, FP64 65,536 x L137 2.29 -> 1.99 ms, FP32 40,007 x L91 in
   // blocks of 100 563 -> 466 us, fused FP32 262,144 x L137 2.85 -> 2.45 ms.
-  // Earlier (before the truncation) the peak grows: mixed 3.84 -> 4.50 ms.  In FP64, whose state fills the registers,
-  // they are loaded after the supersaturation check instead (65,536 x L137: 1.99 ms, before the check 2.06 ms).
-  constexpr bool AHEAD = sizeof(R) == 4;
+  // Earlier (before the truncation) the peak grows: mixed 3.84 -> 4.50 ms.
   struct Level {
     R paph1, pap, t, q, a, ct, cq, ca, vfl, vfi, lude1, lude2, ql, qi, qr, qs, cl, ci, cr, cs;
     R mfu_n, mfd_n, lu_n, lude, snde1, snde2;
@@ -243,7 +241,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
     R ql = ql0, qi = qi0, qr = qr0, qs = qs0;
 
     // saturation values (:1087-1115)
-    const Sat<R> sat = saturation<R, KC>(c, ztp1);
+    const Sat<R> sat = saturation<R, KC, true>(c, ztp1);
     const R foeeliq = c.r2es * sat.el, foeeice = c.r2es * sat.ei;
     const R zfoeewm = m_min(m_div(c.r2es * (sat.alfa * sat.el + (R(1) - sat.alfa) * sat.ei), pap), R(0.5));
     const R zqsmix = m_div(zfoeewm, R(1) - c.retv * zfoeewm);
@@ -459,10 +457,11 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
       }
 
       // 4.1 sedimentation (:1783-1877)
-      const R zfallcorr = m_pow(m_div(c.rdensref, zrho), R(0.4));
+      const auto fallcorr_base = s_base(m_div(c.rdensref, zrho));
+      const R zfallcorr = s_pow(fallcorr_base, R(0.4));
       const R ztemp_r = R(0.5) * (qr + qxnm1_r);
-      const R zrlambda = m_pow(m_div(zrho * ztemp_r, c.rcl_lam1r), c.rcl_lam2r);
-      const R vfall_r = c.rxfallspeedrain * zfallcorr * c.rcl_const7r * m_pow(zrlambda, c.rcl_dr);
+      const auto zrlambda = s_base_pow(s_base(m_div(zrho * ztemp_r, c.rcl_lam1r)), c.rcl_lam2r);
+      const R vfall_r = c.rxfallspeedrain * zfallcorr * c.rcl_const7r * s_pow(zrlambda, c.rcl_dr);
       const R vfall_i = c.rvice, vfall_s = c.rvsnow;
       if (above_top) {
         fsrc_i = pf_i * zdtgdp;
@@ -510,10 +509,11 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
             c_acc = e.acc * ptsphy * c.rcl_kkaac;
           }
         }
-        zrainaut = c_aut * m_pow(zliqcld, c.rcl_kkbauq - R(1)) * zconst_pow;
+        const auto liq_base = s_base(zliqcld);
+        zrainaut = c_aut * s_pow(liq_base, c.rcl_kkbauq - R(1)) * zconst_pow;
         qbrl = qbrl + zrainaut;
         if (zraincld > zepsec)
-          zrainacc = c_acc * m_pow(zliqcld, c.rcl_kkbac - R(1)) * m_pow(zraincld, c.rcl_kkbac);
+          zrainacc = c_acc * s_pow(liq_base, c.rcl_kkbac - R(1)) * s_pow(zraincld, c.rcl_kkbac);
         qbrl = qbrl + zrainacc;
       }
 
@@ -532,16 +532,16 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
         const R zqe = m_max(R(0), m_min(qv, zqsliq));
         if (zcovpclr > zepsec && zraincldm1 > zepsec && zqe < zzrh * zqsliq) {
           const R zpreclr = zraincldm1;
-          const R zfallcorr2 = m_pow(m_div(c.rdensref, zrho), R(0.4f));
+          const R zfallcorr2 = s_pow(fallcorr_base, R(0.4f));
           const R zesatliq = c.rv_rd * foeeliq;
-          const R zlambda = m_pow(m_div(c.rcl_lam1r, zrho * zpreclr), c.rcl_lam2r);
+          const auto zlambda = s_base_pow(s_base(m_div(c.rcl_lam1r, zrho * zpreclr)), c.rcl_lam2r);
           const R t = ztp1;
           const R zevap_denom = c.rcl_cdenom1 * zesatliq - c.rcl_cdenom2 * t * zesatliq + c.rcl_cdenom3 * (t * t * t) * pap;
-          const R zcorr2 = m_div(m_pow(m_div(t, R(273.)), R(1.5)) * R(393.), t + R(120.));
+          const R zcorr2 = m_div(s_pow15(m_div(t, R(273.))) * R(393.), t + R(120.));
           const R zsubsat = m_max(zzrh * zqsliq - zqe, R(0));
           const R zbeta = m_div(R(0.15), zqsliq) * (t * t) * zesatliq * c.rcl_const1r * m_div(zcorr2, zevap_denom) *
-                          (m_div(R(0.78), m_pow(zlambda, c.rcl_const4r)) +
-                           m_div(c.rcl_const2r * m_sqrt(zrho * zfallcorr2), m_sqrt(zcorr2) * m_pow(zlambda, c.rcl_const3r)));
+                          (m_div(R(0.78), s_pow(zlambda, c.rcl_const4r)) +
+                           m_div(c.rcl_const2r * m_sqrt(zrho * zfallcorr2), m_sqrt(zcorr2) * s_pow(zlambda, c.rcl_const3r)));
           const R zdenom = R(1) + zbeta * ptsphy * zcorqsliq;
           const R zdpevap = m_div(zcovpclr * zbeta * ptsphy * zsubsat, zdenom);
           const RD zevap = m_min(RD(zdpevap), qxfg_r);
@@ -561,13 +561,13 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
         }
         if (ztp1 < c.rtt - R(5.) && qxfg_l > rlmin) {
           const R zsupersatice = m_div(zqsliq - zqsice, zqsice);
-          const R zicenuclei = R(1000.0) * m_exp(R(12.96) * zsupersatice - R(0.639));
+          const R zicenuclei = R(1000.0) * s_exp(R(12.96) * zsupersatice - R(0.639));
           const R t = ztp1;
           const R zadd = m_div(c.rlstt * (m_div(c.rlstt, c.rv * t) - R(1)), R(2.4E-2) * t);
           const R zbdd = m_div(c.rv * t * pap, R(2.21) * zvpice);
-          const R zcvds = m_div(R(7.8) * m_pow(m_div(zicenuclei, zrho), R(0.666)) * zsupersatice, R(8.87) * (zadd + zbdd));
+          const R zcvds = m_div(R(7.8) * s_pow(m_div(zicenuclei, zrho), R(0.666)) * zsupersatice, R(8.87) * (zadd + zbdd));
           const R zice0 = m_max(zicecld, m_div(zicenuclei * c.riceinit, zrho));
-          const R zinew = m_pow(R(0.666) * zcvds * ptsphy + m_pow(zice0, R(0.666)), R(1.5));
+          const R zinew = s_pow15(R(0.666) * zcvds * ptsphy + s_pow(zice0, R(0.666)));
           RD zdepos = m_max(c.rcl_overlapliqice * za * (zinew - zice0), R(0));
           zdepos = m_min(zdepos, qxfg_l);
           const R zinfactor = m_min(m_div(zicenuclei, R(15000.)), R(1));
@@ -587,11 +587,11 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
           const R t = ztp1;
           const R zaplusb = c.rcl_apb1 * zvpice - c.rcl_apb2 * zvpice * t + pap * c.rcl_apb3 * (t * t * t);
           const R zcorrfac = m_sqrt(m_div(R(1), zrho));
-          const R zcorrfac2 = m_pow(m_div(t, R(273.0)), R(1.5)) * m_div(R(393.0), t + R(120.0));
-          const R zpr02 = zrho * zsnowcld * c.rcl_const1s;
+          const R zcorrfac2 = s_pow15(m_div(t, R(273.0))) * m_div(R(393.0), t + R(120.0));
+          const auto zpr02 = s_base(zrho * zsnowcld * c.rcl_const1s);
           const R zterm1 = m_div(zsupersatice * (t * t) * zvpice * zcorrfac2 * c.rcl_const2s, zrho * zaplusb);
-          const R zterm2 = R(0.65) * c.rcl_const6s * m_pow(zpr02, c.rcl_const4s) +
-                           m_div(c.rcl_const3s * m_sqrt(zcorrfac) * m_sqrt(zrho) * m_pow(zpr02, c.rcl_const5s), m_sqrt(zcorrfac2));
+          const R zterm2 = R(0.65) * c.rcl_const6s * s_pow(zpr02, c.rcl_const4s) +
+                           m_div(c.rcl_const3s * m_sqrt(zcorrfac) * m_sqrt(zrho) * s_pow(zpr02, c.rcl_const5s), m_sqrt(zcorrfac2));
           R zpsdep = m_max(zcovptot * zterm1 * zterm2 * ptsphy, R(0));
           zpsdep = m_div(m_min(zpsdep, qv - zqsmix), zcorqsmix);
           vs = vs - zpsdep;
@@ -605,10 +605,10 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
 
       // 4.8 ice -> snow autoconversion (:2769-2800)
       if (ztp1 <= c.rtt && zicecld > zepsec) {
-        const R zzco = ptsphy * c.rsnowlin1 * m_exp(c.rsnowlin2 * (ztp1 - c.rtt));
+        const R zzco = ptsphy * c.rsnowlin1 * s_exp(c.rsnowlin2 * (ztp1 - c.rtt));
         const R r = m_div(zicecld, c.rlcritsnow);
         const R ztemp = R(-1.) * (r * r);
-        zsnowaut = (ztemp < R(50.0)) ? zzco * (R(1) - m_exp(ztemp)) : zzco;
+        zsnowaut = (ztemp < R(50.0)) ? zzco * (R(1) - s_exp(ztemp)) : zzco;
         qbsi = qbsi + zsnowaut;
       }
 
@@ -649,9 +649,9 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
         if (ztp1 < c.rtt) {
           R zfrzmax;
           if (llrainliq) {
-            const R zlambda = m_pow(m_div(c.rcl_lam1r, zrho * qr), c.rcl_lam2r);
+            const auto zlambda = s_base_pow(s_base(m_div(c.rcl_lam1r, zrho * qr)), c.rcl_lam2r);
             const R ztemp = m_min(c.rcl_fzrab * (ztp1 - c.rtt), R(50.));
-            const R zfrz = ptsphy * m_div(c.rcl_const5r, zrho) * (m_exp(ztemp) - R(1.)) * m_pow(zlambda, c.rcl_const6r);
+            const R zfrz = ptsphy * m_div(c.rcl_const5r, zrho) * (s_exp(ztemp) - R(1.)) * s_pow(zlambda, c.rcl_const6r);
             zfrzmax = m_max(zfrz, R(0));
           } else {
             const R zcons1 = m_abs(m_div(ptsphy * (R(1) + R(0.5) * (c.rtt - ztp1)), c.rtaumel));
@@ -678,9 +678,9 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
       // 4.9 riming of snow (:2975-3017)
       if (ztp1 <= c.rtt && zliqcld > zepsec) {
         if (zsnowcld > zepsec && zcovptot > R(0.01)) {
-          const R zfallcorr3 = m_pow(m_div(c.rdensref, zrho), R(0.4f));
+          const R zfallcorr3 = s_pow(fallcorr_base, R(0.4f));
           zsnowrime = c.rcl_effrime * zcovptot * ptsphy * c.rcl_const7s * zfallcorr3 *
-                        m_pow(zrho * zsnowcld * c.rcl_const1s, c.rcl_const8s);
+                        s_pow(zrho * zsnowcld * c.rcl_const1s, c.rcl_const8s);
           zsnowrime = m_min(zsnowrime, R(1));
           qbsl = qbsl + zsnowrime;
         }
@@ -688,11 +688,12 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
 
       // PSD slopes, PSACR and PIACR (:3029-3198)
       if (ztp1 <= c.rtt && prainfrac < zepsec && zraincld > zepsec) {
-        const R zlamr = m_pow(m_div(c.rcl_lam1r, zrho * zraincld), c.rcl_lam2r);
-        const R zn0r = c.rcl_x1r * m_pow(zlamr, c.rcl_x2r);
+        const auto lamr_base = s_base(m_div(c.rcl_lam1r, zrho * zraincld));
+        const R zlamr = s_pow(lamr_base, c.rcl_lam2r);
+        const R zn0r = c.rcl_x1r * s_pow(s_base_pow(lamr_base, c.rcl_lam2r), c.rcl_x2r);
         const R lr3 = zlamr * zlamr * zlamr;
         if (zsnowcld > zepsec) {
-          const R zlams = m_pow(m_div(c.rcl_lam1s, zrho * zsnowcld), c.rcl_lam2s);
+          const R zlams = s_pow(m_div(c.rcl_lam1s, zrho * zsnowcld), c.rcl_lam2s);
           const R zfalldiff = m_max(m_abs(vfall_r - vfall_s), (vfall_r + vfall_s) / R(8.));
           const R zfac = m_div(c.rpi * c.rpi * c.rdenswat * R(1.0) * zrho * zn0r * c.rcl_x1s, zlams * lr3);
           const R zrat = m_div(zlamr, zlams);
@@ -701,7 +702,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
           bud.set(PSACR, zpsacr);
         }
         if (zicecld > zepsec) {
-          const R zlami = m_pow(m_div(c.rcl_lam1s, zrho * zicecld), c.rcl_lam2s);
+          const R zlami = s_pow(m_div(c.rcl_lam1s, zrho * zicecld), c.rcl_lam2s);
           const R zfalldiff = m_max(m_abs(vfall_r - vfall_i), (vfall_r + vfall_i) / R(8.));
           const R zfac = m_div(c.rpi * c.rpi * c.rdenswat * R(0.1) * zrho * zn0r * c.rcl_x1s, zlami * lr3);
           const R zrat = m_div(zlamr, zlami);
@@ -722,7 +723,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
           const R den = m_max(m_abs(dd), c.zepsilon);
           const R zpreclr = R(m_div(qxfg_s * RD(zcovpclr), RD(dd < R(0) ? -den : den)));
           const R zbeta1 = m_div(m_div(m_sqrt(m_div(pap, paph_surf)), c.rvrfactor) * zpreclr, m_max(zcovpclr, zepsec));
-          const R zbeta = c.rg * c.rpecons * m_pow(zbeta1, R(0.5777));
+          const R zbeta = c.rg * c.rpecons * s_pow(zbeta1, R(0.5777));
           const R zdenom = R(1) + zbeta * ptsphy * zcorqsice;
           const R zdpr = m_div(zcovpclr * zbeta * (zqsice - zqe), zdenom) * zdp * c.zrg_r;
           const R zdpevap = zdpr * zdtgdp;
@@ -821,7 +822,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
         ta = zda * zqtmst;
       }
 
-      if (AHEAD && has_next) nxt = load(k + 1);
+      if (has_next) nxt = load(k + 1);
       // 6.4 CLOUD_SUPERSATCHECK on the updated state (:3765-3777), in R
       {
         const R zq_upd = pq + ptsphy * (tq + tcml_q);
@@ -829,7 +830,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
         const R za_upd = pa + ptsphy * (ta + tcml_a);
         const R pp = ssc_off ? LD(fresh()->p.pap, i2 + (uint32_t)ssc_off * E, jo) : pap;
         R t_adj, q_adj, a_adj, l_adj, i_adj;
-        supersatcheck<R, KC>(c, zt_upd, zq_upd, za_upd, pp, t_adj, q_adj, a_adj, l_adj, i_adj);
+        supersatcheck<R, KC, true>(c, zt_upd, zq_upd, za_upd, pp, t_adj, q_adj, a_adj, l_adj, i_adj);
         tq = tq + R(q_adj) * zqtmst;
         tt = tt + R(t_adj) * zqtmst;
         ta = ta + R(a_adj) * zqtmst;
@@ -886,7 +887,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
       }
     }
 
-    if (has_next && !(AHEAD && (int)k >= ncldtop0)) nxt = load(k + 1);
+    if (has_next && (int)k < ncldtop0) nxt = load(k + 1);
 
     // store tendencies of this level (levels above NCLDTOP keep the tidy-up terms only)
     CArgs* const g = fresh();
