@@ -31,3 +31,28 @@ def test_fp64_on_grids_of_any_size(ngptot, nproma, params91):
         g, r = columns(out[n], nproma), columns(ref[n], nproma)
         np.testing.assert_array_equal(np.isnan(g), np.isnan(r), err_msg=n)
         assert relrms(g, r) <= 1e-12, n
+
+
+@pytest.mark.parametrize("nproma,default", [(64, True), (100, True), (64, False), (100, False)])
+@pytest.mark.parametrize("fused", [False, True])
+def test_fp64_at_two_waves_per_simd_equals_one(nproma, default, fused, params91):
+    """Launches of more waves than the chip has SIMDs use another instantiation; the columns are the same bit for bit."""
+    import copy
+
+    from openifs_amd import satadj as A
+
+    params = copy.copy(params91)
+    if not default:
+        params.rcldiff = params.rcldiff * 1.5
+
+    make = A.FusedFields if fused else C.BlockedFields
+    big, small = (make(n, nproma, 91, "dp", "cuda", fill=0.0) for n in (66000, 40 * nproma))
+    (A.synth_device if fused else C.synth_device)(big, params, 5)
+    for n in big.t:
+        small[n].copy_(big[n][:40])
+    call = A.satadj_cloudsc_blocked if fused else C.cloudsc_blocked
+    call(big, params, 900.0)
+    call(small, params, 900.0)
+    torch.cuda.synchronize()
+    for n in OUT:
+        assert torch.equal(big[n][:40], small[n]), n
