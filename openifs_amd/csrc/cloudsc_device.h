@@ -96,8 +96,10 @@ __device__ __forceinline__ Sat<T> saturation(const KCT& c, T t) {
   return s;
 }
 
-// CLOUD_SUPERSATCHECK for one point, KFTLIQICE = 1 (cloud_supersatcheck.F90:111-226).
-template <typename T, typename KCT, bool SWEEP = false>
+// CLOUD_SUPERSATCHECK for one point, KFTLIQICE = 1 (cloud_supersatcheck.F90:111-226).  SHARE (FP64 inside an FP32
+// point, whose result is rounded to FP32): the quotients by the two temperature differences and by the two saturation
+// denominators from one division each.
+template <typename T, typename KCT, bool SWEEP = false, bool SHARE = false>
 __device__ __forceinline__ void supersatcheck(const KCT& c, T pt, T pq, T pa, T pp, T& t_adj, T& q_adj,
                                               T& a_adj, T& l_adj, T& i_adj) {
   const T zepsec = T(1.e-14);
@@ -105,19 +107,39 @@ __device__ __forceinline__ void supersatcheck(const KCT& c, T pt, T pq, T pa, T 
   T zt = m_max(pt, T(160));
   T za = m_max(m_min(pa, T(1)), T(0));
   const T zp_r = m_div(T(1), pp);
-  const Sat<T> s = saturation<T, KCT, SWEEP>(c, zt);
+  const T dl = zt - c.r4les, di = zt - c.r4ies;
+  Sat<T> s;
+  T fl, fi;  // 1 / dl^2, 1 / di^2
+  if constexpr (SHARE) {
+    const T w = m_div(T(1), dl * di), rl = w * di, ri = w * dl;
+    const T x = (m_max(c.rtice, m_min(c.rtwat, zt)) - c.rtice) * c.rtwat_rtice_r;
+    s.alfa = m_min(T(1), x * x);
+    s.el = m_exp(c.r3les * (zt - c.rtt) * rl);
+    s.ei = m_exp(c.r3ies * (zt - c.rtt) * ri);
+    fl = rl * rl, fi = ri * ri;
+  } else {
+    s = saturation<T, KCT, SWEEP>(c, zt);
+    fl = m_div(T(1), dl * dl), fi = m_div(T(1), di * di);
+  }
   const T foeeliq = c.r2es * s.el;
   const T zfoeeliq = m_min(foeeliq * zp_r, T(0.5));
   // FOEEW: water above RTT, ice below (FOEDELTA = MAX(0,SIGN(1,T-RTT)))
   const T foeew = (zt - c.rtt >= T(0)) ? c.r2es * s.el : c.r2es * s.ei;
   const T zfoeeice = m_min(foeew * zp_r, T(0.5));
   const T zfokoop = m_min(zfoeeice * (c.rkoop1 - c.rkoop2 * zt), zfoeeliq);
-  T zqsliqk = m_div(zfokoop, T(1) - c.retv * zfokoop);
   const T zfoeemix = m_min(c.r2es * (s.alfa * s.el + (T(1) - s.alfa) * s.ei) * zp_r, T(0.5));
-  const T zcor = m_div(T(1), T(1) - c.retv * zfoeemix);
+  const T dk = T(1) - c.retv * zfokoop, dm = T(1) - c.retv * zfoeemix;
+  T zqsliqk, zcor;
+  if constexpr (SHARE) {
+    const T w = m_div(T(1), dk * dm);
+    zqsliqk = zfokoop * (w * dm);
+    zcor = w * dk;
+  } else {
+    zqsliqk = m_div(zfokoop, dk);
+    zcor = m_div(T(1), dm);
+  }
   const T zqsmix = zfoeemix * zcor;
-  const T dl = zt - c.r4les, di = zt - c.r4ies;
-  const T foedem = s.alfa * c.r5alvcp * m_div(T(1), dl * dl) + (T(1) - s.alfa) * c.r5alscp * m_div(T(1), di * di);
+  const T foedem = s.alfa * c.r5alvcp * fl + (T(1) - s.alfa) * c.r5alscp * fi;
   const T zcorqsmix = T(1) + zqsmix * zcor * foedem;
   zqsliqk = T(0.5) * (zqsliqk + zqsmix);
   T zqslim = za * zqsmix + (T(1) - za) * zqsliqk;

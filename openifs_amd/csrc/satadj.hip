@@ -42,13 +42,21 @@ template <typename R>
 struct Vec<R, 1> {
   typedef R type;
 };
+// Loads and stores of words that one point alone touches, with the non-temporal hint; half-level pressures, which two
+// points of a column read (and the surface's, which all do), stay plain.  FP32 160,000 x L91 in blocks of 64: 253 us all
+// plain, 232 all non-temporal, 220 like this; 655,360 x L137: 1.52, 1.44 and 1.38 ms; blocks of 75: 239, 233 and 219 us.
 template <int V, typename R>
 __device__ __forceinline__ typename Vec<R, V>::type LDV(const R* base, uint32_t u, uint32_t v) {
+  return __builtin_nontemporal_load(
+      reinterpret_cast<const typename Vec<R, V>::type*>(reinterpret_cast<const char*>(base) + (u + v)));
+}
+template <int V, typename R>
+__device__ __forceinline__ typename Vec<R, V>::type LDK(const R* base, uint32_t u, uint32_t v) {
   return *reinterpret_cast<const typename Vec<R, V>::type*>(reinterpret_cast<const char*>(base) + (u + v));
 }
 template <int V, typename R>
 __device__ __forceinline__ void STV(R* base, uint32_t u, uint32_t v, typename Vec<R, V>::type x) {
-  *reinterpret_cast<typename Vec<R, V>::type*>(reinterpret_cast<char*>(base) + (u + v)) = x;
+  __builtin_nontemporal_store(x, reinterpret_cast<typename Vec<R, V>::type*>(reinterpret_cast<char*>(base) + (u + v)));
 }
 template <int V, typename R>
 __device__ __forceinline__ R lane(const typename Vec<R, V>::type& x, int j) {
@@ -67,8 +75,8 @@ __device__ __forceinline__ void set_lane(typename Vec<R, V>::type& x, int j, R y
 
 // One lane handles V consecutive columns of one level (V = 2 when NPROMA is even and every array is aligned to
 // 2 words, else 1); lanes of a wave cover consecutive columns, so each load and store instruction moves one
-// contiguous row segment of 64 V words.  Measured at 655,360 columns x L137: V = 2 is 9 % faster than V = 1 in
-// FP32 (1.40 vs 1.53 ms) and 7 % in FP64; V = 4 is no faster than V = 1 (its 93 VGPRs halve the waves per SIMD).
+// contiguous row segment of 64 V words.  Measured at 655,360 columns x L137, plain loads: V = 2 is 9 % faster than V = 1
+// in FP32 (1.40 vs 1.53 ms) and 7 % in FP64; V = 4 is no faster than V = 1 (its 93 VGPRs halve the waves per SIMD).
 template <typename R, typename RD, typename KC, typename KCD, int V>
 __global__ __launch_bounds__(256) void satadj_kernel(const KC c, const KCD cd, const SatPtrs<R> p, const SatDims d) {
   typedef typename Vec<R, V>::type VT;
@@ -93,7 +101,7 @@ __global__ __launch_bounds__(256) void satadj_kernel(const KC c, const KCD cd, c
   } else {
     const VT pt = LDV<V>(p.pt, o2, 0u), pq = LDV<V>(p.pq, o2, 0u), pa = LDV<V>(p.pa, o2, 0u);
     const VT pl = LDV<V>(p.pl, oc, 0u), pi = LDV<V>(p.pi, oc, 0u), pap = LDV<V>(p.pap, o2, 0u);
-    const VT ph0 = LDV<V>(p.paph, oh, 0u), ph1 = LDV<V>(p.paph, oh, lstep), ps = LDV<V>(p.paph, os, 0u);
+    const VT ph0 = LDK<V>(p.paph, oh, 0u), ph1 = LDK<V>(p.paph, oh, lstep), ps = LDK<V>(p.paph, os, 0u);
     const VT tct = LDV<V>(p.tcml_t, o2, 0u), tcq = LDV<V>(p.tcml_q, o2, 0u), tca = LDV<V>(p.tcml_a, o2, 0u);
     const VT tcl = LDV<V>(p.tcml_l, oc, 0u), tci = LDV<V>(p.tcml_i, oc, 0u);
     const VT hrsw = LDV<V>(p.phrsw, o2, 0u), hrlw = LDV<V>(p.phrlw, o2, 0u);
