@@ -24,6 +24,9 @@ using cloudsc_gpu::m_sqrt;
 
 using cloudsc_gpu::LD;
 using cloudsc_gpu::ST;
+using cloudsc_gpu::LDN;
+using cloudsc_gpu::STN;
+using cloudsc_gpu::xcd_group;
 
 // Constants of one launch in the storage precision (cloudsc2.F90:243-253 and the TCST/TTHF/TECLDP/TEPHLI values).
 template <typename R>
@@ -110,6 +113,9 @@ __device__ __forceinline__ void adjust(const C2Const<R>& c, R psp, R& pt, R& pq)
 }
 
 // Work-group size: 64, 128 and 256 run within 1 % of each other at 655,360 x L137 in FP32.
+// The column kernels move 27 (CLOUDST) to 35 words per point at the rate of a copy.  Non-temporal words in aligned blocks
+// and contiguous columns per XCD: CLOUD_S_LAYER on CLOUDST, FP32 327,680 x L137 1,081 -> 1,057 us (4.8 TB/s), 100,000 x
+// L91 in blocks of 64 263 -> 245 us, 40,000 x L91 in blocks of 100 247 -> 240 us.
 constexpr int CLOUDSC2_BLOCK = 128;
 
 // SATUR with KFLAG = 2 (satur.F90:110-141): the saturation specific humidity of the mixed phase at (t, p), in the
@@ -137,7 +143,7 @@ __device__ __forceinline__ R satur(const C2Const<R>& c, R t, R paprsf) {
 template <typename R, bool UNI, bool LAYER>
 __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<R> c, const C2Ptrs<R> p,
                                                                   const C2Dims d) {
-  const uint32_t g = blockIdx.x * CLOUDSC2_BLOCK + threadIdx.x;
+  const uint32_t g = xcd_group(blockIdx.x, gridDim.x) * CLOUDSC2_BLOCK + threadIdx.x;
   const uint32_t nproma = (uint32_t)d.nproma;
   const int klev = d.klev;
   if (g >= (uint32_t)d.ngpblks * nproma) return;
@@ -153,16 +159,16 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
   auto ath = [&](int k) { return bh + (uint32_t)k * lstep; };
   if constexpr (LAYER) {  // TENDENCY_LOC%CLD(:,:,NCLDQR/NCLDQS) = 0 on every column of the block (:164-165)
     for (int k = 0; k < klev; ++k) {
-      if (p.ptenr) ST(p.ptenr, at2(k), jo, R(0));
-      if (p.ptens) ST(p.ptens, at2(k), jo, R(0));
+      if (p.ptenr) STN<UNI>(p.ptenr, at2(k), jo, R(0));
+      if (p.ptens) STN<UNI>(p.ptens, at2(k), jo, R(0));
     }
   }
   const int kfdia = std::min(d.kfdia, d.ngptot - (int)(b * nproma));
   if ((int)jl < d.kidia - 1 || (int)jl >= kfdia) return;
   const R ptsphy = c.ptsphy;
   if constexpr (LAYER) {  // (:168-169)
-    if (p.pprectype) ST(p.pprectype, b * lstep, jo, R(0));
-    if (p.pfzra) ST(p.pfzra, b * lstep, jo, R(0));
+    if (p.pprectype) STN<UNI>(p.pprectype, b * lstep, jo, R(0));
+    if (p.pfzra) STN<UNI>(p.pfzra, b * lstep, jo, R(0));
   }
   const R zeps1 = R(1.e-12), zeps2 = R(1.e-10), zqmax = R(0.5);
 
@@ -178,19 +184,19 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
   }
   // outputs the level loop does not reach (:297-320): PCLC, PCOVPTOT zero, PFPLSL/PFPLSN zero at the top
   for (int k = 0; k < d.ktdia - 1; ++k) {
-    if (!LAYER || p.pclc) ST(p.pclc, at2(k), jo, R(0));
-    ST(p.pcovptot, at2(k), jo, R(0));
+    if (!LAYER || p.pclc) STN<UNI>(p.pclc, at2(k), jo, R(0));
+    STN<UNI>(p.pcovptot, at2(k), jo, R(0));
     if constexpr (LAYER) {  // (PCLC - PA)/TSPHY with PCLC = 0 above KTDIA (:155-158)
-      if (p.ptena) ST(p.ptena, at2(k), jo, c.zqtmst * (R(0) - LD(p.pa, at2(k), jo)));
+      if (p.ptena) STN<UNI>(p.ptena, at2(k), jo, c.zqtmst * (R(0) - LD(p.pa, at2(k), jo)));
     }
   }
-  ST(p.pfplsl, ath(0), jo, R(0));
-  ST(p.pfplsn, ath(0), jo, R(0));
-  ST(p.pfhpsl, ath(0), jo, -R(0) * c.rlvtt);  // (:694-699), as -PFPLSL*RLVTT
-  ST(p.pfhpsn, ath(0), jo, -R(0) * c.rlstt);
+  STN<UNI>(p.pfplsl, ath(0), jo, R(0));
+  STN<UNI>(p.pfplsn, ath(0), jo, R(0));
+  STN<UNI>(p.pfhpsl, ath(0), jo, -R(0) * c.rlvtt);  // (:694-699), as -PFPLSL*RLVTT
+  STN<UNI>(p.pfhpsn, ath(0), jo, -R(0) * c.rlstt);
   for (int k = 1; k < d.ktdia; ++k) {  // half levels the loop leaves as they are
-    ST(p.pfhpsl, ath(k), jo, -LD(p.pfplsl, ath(k), jo) * c.rlvtt);
-    ST(p.pfhpsn, ath(k), jo, -LD(p.pfplsn, ath(k), jo) * c.rlstt);
+    STN<UNI>(p.pfhpsl, ath(k), jo, -LD(p.pfplsl, ath(k), jo) * c.rlvtt);
+    STN<UNI>(p.pfhpsn, ath(k), jo, -LD(p.pfplsn, ath(k), jo) * c.rlstt);
   }
   const R paph_surf = LD(p.paphp1, ath(klev), jo);
 
@@ -202,14 +208,14 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
   auto load = [&](int k) {
     const uint32_t j = at2(k);
     Level v;
-    v.tm1 = LD(p.ptm1, j, jo); v.gtent = LD(p.pgtent, j, jo); v.qm1 = LD(p.pqm1, j, jo);
-    v.gtenq = LD(p.pgtenq, j, jo); v.l = LD(p.pl, j, jo); v.gtenl = LD(p.pgtenl, j, jo); v.i = LD(p.pi, j, jo);
-    v.gteni = LD(p.pgteni, j, jo); v.paph1 = LD(p.paphp1, ath(k + 1), jo);
-    v.qs = LAYER ? R(0) : LD(p.pqs, j, jo);
-    v.a = (LAYER && p.ptena) ? LD(p.pa, j, jo) : R(0);
-    v.app1 = LD(p.papp1, j, jo); v.lude = LD(p.plude, j, jo);
-    v.lu_next = k < klev - 1 ? LD(p.plu, j + lstep, jo) : R(0);
-    v.mfu = LD(p.pmfu, j, jo); v.mfd = LD(p.pmfd, j, jo);
+    v.tm1 = LDN<UNI>(p.ptm1, j, jo); v.gtent = LDN<UNI>(p.pgtent, j, jo); v.qm1 = LDN<UNI>(p.pqm1, j, jo);
+    v.gtenq = LDN<UNI>(p.pgtenq, j, jo); v.l = LDN<UNI>(p.pl, j, jo); v.gtenl = LDN<UNI>(p.pgtenl, j, jo); v.i = LDN<UNI>(p.pi, j, jo);
+    v.gteni = LDN<UNI>(p.pgteni, j, jo); v.paph1 = LDN<UNI>(p.paphp1, ath(k + 1), jo);
+    v.qs = LAYER ? R(0) : LDN<UNI>(p.pqs, j, jo);
+    v.a = (LAYER && p.ptena) ? LDN<UNI>(p.pa, j, jo) : R(0);
+    v.app1 = LDN<UNI>(p.papp1, j, jo); v.lude = LDN<UNI>(p.plude, j, jo);
+    v.lu_next = k < klev - 1 ? LDN<UNI>(p.plu, j + lstep, jo) : R(0);
+    v.mfu = LDN<UNI>(p.pmfu, j, jo); v.mfd = LDN<UNI>(p.pmfd, j, jo);
     return v;
   };
 
@@ -234,7 +240,7 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
     // CLOUD_S_LAYER's SATUR at the first-guess temperature (cloud_s_layer.F90:112-118), else the PQS input
     const R pqs = LAYER ? satur(c, ztp1, papp1) : cur.qs;
     if constexpr (LAYER) {
-      if (p.pqsat) ST(p.pqsat, i2, jo, pqs);
+      if (p.pqsat) STN<UNI>(p.pqsat, i2, jo, pqs);
     }
 
     // 3.1 (:352-416)
@@ -414,20 +420,20 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
     zsfln = zsfln + (R(1.0) - zfwatr) * zdr2;
     zrfreeze = zrfreeze + zrfreeze2;
 
-    ST(p.ptenq, i2, jo, -(zcondl + zcondi) + (plude + zevapr + zevaps) * zgdp);
-    ST(p.ptent, i2, jo, tendency_t(zcondl, zcondi, zrfreeze));
-    ST(p.ptenl, i2, jo, (zqlwc - zl) * c.zqtmst);
-    ST(p.pteni, i2, jo, (zqiwc - zi) * c.zqtmst);
-    if (!LAYER || p.pclc) ST(p.pclc, i2, jo, pclc);
+    STN<UNI>(p.ptenq, i2, jo, -(zcondl + zcondi) + (plude + zevapr + zevaps) * zgdp);
+    STN<UNI>(p.ptent, i2, jo, tendency_t(zcondl, zcondi, zrfreeze));
+    STN<UNI>(p.ptenl, i2, jo, (zqlwc - zl) * c.zqtmst);
+    STN<UNI>(p.pteni, i2, jo, (zqiwc - zi) * c.zqtmst);
+    if (!LAYER || p.pclc) STN<UNI>(p.pclc, i2, jo, pclc);
     if constexpr (LAYER) {  // (:155-158)
-      if (p.ptena) ST(p.ptena, i2, jo, c.zqtmst * (pclc - cur.a));
+      if (p.ptena) STN<UNI>(p.ptena, i2, jo, c.zqtmst * (pclc - cur.a));
     }
-    ST(p.pcovptot, i2, jo, pcovptot);
+    STN<UNI>(p.pcovptot, i2, jo, pcovptot);
     const uint32_t ih = ath(k + 1);
-    ST(p.pfplsl, ih, jo, zrfln);
-    ST(p.pfplsn, ih, jo, zsfln);
-    ST(p.pfhpsl, ih, jo, -zrfln * c.rlvtt);
-    ST(p.pfhpsn, ih, jo, -zsfln * c.rlstt);
+    STN<UNI>(p.pfplsl, ih, jo, zrfln);
+    STN<UNI>(p.pfplsn, ih, jo, zsfln);
+    STN<UNI>(p.pfhpsl, ih, jo, -zrfln * c.rlvtt);
+    STN<UNI>(p.pfhpsn, ih, jo, -zsfln * c.rlstt);
     zrfl = zrfln;
     zsfl = zsfln;
     paph0 = paph1;
@@ -442,7 +448,7 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
 template <typename R, bool UNI, bool LAYER>
 __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R> c, const C2Ptrs<R> p,
                                                                  const C2Dims d) {
-  const uint32_t g = blockIdx.x * CLOUDSC2_BLOCK + threadIdx.x;
+  const uint32_t g = xcd_group(blockIdx.x, gridDim.x) * CLOUDSC2_BLOCK + threadIdx.x;
   const uint32_t nproma = (uint32_t)d.nproma;
   const int klev = d.klev;
   if (g >= (uint32_t)d.ngpblks * nproma) return;
@@ -458,8 +464,8 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
   auto ath = [&](int k) { return bh + (uint32_t)k * lstep; };
   if constexpr (LAYER) {  // (:164-165), every column of the block
     for (int k = 0; k < klev; ++k) {
-      if (p.ptenr) ST(p.ptenr, at2(k), jo, R(0));
-      if (p.ptens) ST(p.ptens, at2(k), jo, R(0));
+      if (p.ptenr) STN<UNI>(p.ptenr, at2(k), jo, R(0));
+      if (p.ptens) STN<UNI>(p.ptens, at2(k), jo, R(0));
     }
   }
   const int kfdia = std::min(d.kfdia, d.ngptot - (int)(b * nproma));
@@ -469,8 +475,8 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
   const R zcons3 = R(2.5E6) / R(1005.);  // (:215)
   const R zpecons = R(1.E-5);           // (:217)
   if constexpr (LAYER) {
-    if (p.pprectype) ST(p.pprectype, b * lstep, jo, R(0));
-    if (p.pfzra) ST(p.pfzra, b * lstep, jo, R(0));
+    if (p.pprectype) STN<UNI>(p.pprectype, b * lstep, jo, R(0));
+    if (p.pfzra) STN<UNI>(p.pfzra, b * lstep, jo, R(0));
   }
   // eta of the tropopause (:234-247)
   R ztrpaus = R(0.1);
@@ -487,27 +493,27 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
   auto wrap_state = [&](int k, R clc, R lwp, R iwp, R a, R l, R i) {
     if constexpr (LAYER) {
       const uint32_t j = at2(k);
-      if (p.ptena) ST(p.ptena, j, jo, c.zqtmst * (clc - a));
-      ST(p.ptenl, j, jo, c.zqtmst * (lwp - l));
-      ST(p.pteni, j, jo, c.zqtmst * (iwp - i));
+      if (p.ptena) STN<UNI>(p.ptena, j, jo, c.zqtmst * (clc - a));
+      STN<UNI>(p.ptenl, j, jo, c.zqtmst * (lwp - l));
+      STN<UNI>(p.pteni, j, jo, c.zqtmst * (iwp - i));
     }
   };
   for (int k = 0; k < d.ktdia - 1; ++k) {
-    if (!LAYER || p.pclc) ST(p.pclc, at2(k), jo, R(0));
-    if (!LAYER || p.pqiwp) ST(p.pqiwp, at2(k), jo, R(0));
-    if (!LAYER || p.pqlwp) ST(p.pqlwp, at2(k), jo, R(0));
-    ST(p.pcovptot, at2(k), jo, R(0));
+    if (!LAYER || p.pclc) STN<UNI>(p.pclc, at2(k), jo, R(0));
+    if (!LAYER || p.pqiwp) STN<UNI>(p.pqiwp, at2(k), jo, R(0));
+    if (!LAYER || p.pqlwp) STN<UNI>(p.pqlwp, at2(k), jo, R(0));
+    STN<UNI>(p.pcovptot, at2(k), jo, R(0));
     if constexpr (LAYER)
       wrap_state(k, R(0), R(0), R(0), p.ptena ? LD(p.pa, at2(k), jo) : R(0), LD(p.pl, at2(k), jo),
                  LD(p.pi, at2(k), jo));
   }
-  ST(p.pfplsl, ath(0), jo, R(0));
-  ST(p.pfplsn, ath(0), jo, R(0));
-  ST(p.pfhpsl, ath(0), jo, -R(0) * c.rlvtt);  // (:629-634)
-  ST(p.pfhpsn, ath(0), jo, -R(0) * c.rlstt);
+  STN<UNI>(p.pfplsl, ath(0), jo, R(0));
+  STN<UNI>(p.pfplsn, ath(0), jo, R(0));
+  STN<UNI>(p.pfhpsl, ath(0), jo, -R(0) * c.rlvtt);  // (:629-634)
+  STN<UNI>(p.pfhpsn, ath(0), jo, -R(0) * c.rlstt);
   for (int k = 1; k < d.ktdia; ++k) {
-    ST(p.pfhpsl, ath(k), jo, -LD(p.pfplsl, ath(k), jo) * c.rlvtt);
-    ST(p.pfhpsn, ath(k), jo, -LD(p.pfplsn, ath(k), jo) * c.rlstt);
+    STN<UNI>(p.pfhpsl, ath(k), jo, -LD(p.pfplsl, ath(k), jo) * c.rlvtt);
+    STN<UNI>(p.pfhpsn, ath(k), jo, -LD(p.pfplsn, ath(k), jo) * c.rlstt);
   }
   const R paph_surf = LD(p.paphp1, ath(klev), jo);
 
@@ -518,14 +524,14 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
   auto load = [&](int k) {
     const uint32_t j = at2(k);
     Level v;
-    v.tm1 = LD(p.ptm1, j, jo); v.gtent = LD(p.pgtent, j, jo); v.qm1 = LD(p.pqm1, j, jo);
-    v.gtenq = LD(p.pgtenq, j, jo); v.paph1 = LD(p.paphp1, ath(k + 1), jo); v.app1 = LD(p.papp1, j, jo);
-    v.lude = LD(p.plude, j, jo);
-    v.qs = LAYER ? R(0) : LD(p.pqs, j, jo);
-    v.lu_next = k < klev - 1 ? LD(p.plu, j + lstep, jo) : R(0);
-    v.a = (LAYER && p.ptena) ? LD(p.pa, j, jo) : R(0);
-    v.l = LAYER ? LD(p.pl, j, jo) : R(0);
-    v.i = LAYER ? LD(p.pi, j, jo) : R(0);
+    v.tm1 = LDN<UNI>(p.ptm1, j, jo); v.gtent = LDN<UNI>(p.pgtent, j, jo); v.qm1 = LDN<UNI>(p.pqm1, j, jo);
+    v.gtenq = LDN<UNI>(p.pgtenq, j, jo); v.paph1 = LDN<UNI>(p.paphp1, ath(k + 1), jo); v.app1 = LDN<UNI>(p.papp1, j, jo);
+    v.lude = LDN<UNI>(p.plude, j, jo);
+    v.qs = LAYER ? R(0) : LDN<UNI>(p.pqs, j, jo);
+    v.lu_next = k < klev - 1 ? LDN<UNI>(p.plu, j + lstep, jo) : R(0);
+    v.a = (LAYER && p.ptena) ? LDN<UNI>(p.pa, j, jo) : R(0);
+    v.l = LAYER ? LDN<UNI>(p.pl, j, jo) : R(0);
+    v.i = LAYER ? LDN<UNI>(p.pi, j, jo) : R(0);
     return v;
   };
   R zrfl = R(0), zsfl = R(0), zcovptot = R(0);
@@ -543,7 +549,7 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
     const R papp1 = cur.app1, plude = cur.lude;
     const R pqs = LAYER ? satur(c, ztp1, papp1) : cur.qs;
     if constexpr (LAYER) {
-      if (p.pqsat) ST(p.pqsat, i2, jo, pqs);
+      if (p.pqsat) STN<UNI>(p.pqsat, i2, jo, pqs);
     }
     // critical relative humidity (:263-290)
     R zcrh = R(0);
@@ -690,18 +696,18 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
     zrfln = zrfln + zfwatr * zdr;
     zsfln = zsfln + (R(1.0) - zfwatr) * zdr;
 
-    ST(p.ptenq, i2, jo, tendency_q(zrfln, zsfln));
-    ST(p.ptent, i2, jo, tendency_t(zrfln, zsfln, zrfreeze));
-    if (!LAYER || p.pclc) ST(p.pclc, i2, jo, pclc);
-    if (!LAYER || p.pqlwp) ST(p.pqlwp, i2, jo, pqlwp);
-    if (!LAYER || p.pqiwp) ST(p.pqiwp, i2, jo, pqiwp);
-    ST(p.pcovptot, i2, jo, pcovptot);
+    STN<UNI>(p.ptenq, i2, jo, tendency_q(zrfln, zsfln));
+    STN<UNI>(p.ptent, i2, jo, tendency_t(zrfln, zsfln, zrfreeze));
+    if (!LAYER || p.pclc) STN<UNI>(p.pclc, i2, jo, pclc);
+    if (!LAYER || p.pqlwp) STN<UNI>(p.pqlwp, i2, jo, pqlwp);
+    if (!LAYER || p.pqiwp) STN<UNI>(p.pqiwp, i2, jo, pqiwp);
+    STN<UNI>(p.pcovptot, i2, jo, pcovptot);
     wrap_state(k, pclc, pqlwp, pqiwp, cur.a, cur.l, cur.i);
     const uint32_t ih = ath(k + 1);
-    ST(p.pfplsl, ih, jo, zrfln);
-    ST(p.pfplsn, ih, jo, zsfln);
-    ST(p.pfhpsl, ih, jo, -zrfln * c.rlvtt);
-    ST(p.pfhpsn, ih, jo, -zsfln * c.rlstt);
+    STN<UNI>(p.pfplsl, ih, jo, zrfln);
+    STN<UNI>(p.pfplsn, ih, jo, zsfln);
+    STN<UNI>(p.pfhpsl, ih, jo, -zrfln * c.rlvtt);
+    STN<UNI>(p.pfhpsn, ih, jo, -zsfln * c.rlstt);
     zrfl = zrfln;
     zsfl = zsfln;
     paph0 = paph1;
