@@ -56,3 +56,40 @@ def test_fp64_at_two_waves_per_simd_equals_one(nproma, default, fused, params91)
     torch.cuda.synchronize()
     for n in OUT:
         assert torch.equal(big[n][:40], small[n]), n
+
+
+def _block_call(params, inp, prec, n, klev, kidia, kfdia):
+    """Columns 0 .. n-1 of a one-block field set through the per-block entry, outputs prefilled with NaN."""
+    arrs = {}
+    for name, _, role in C.BLOCKED_ARRAYS:
+        if name in inp:
+            x = inp[name][0][..., :n]
+            arrs[name] = np.asfortranarray(x.T if x.ndim < 3 else x.transpose(2, 1, 0))
+    full = C.allocate_block(n, klev, prec, fill=np.nan)
+    for name, x in arrs.items():
+        full[name][...] = x
+    C.CLOUDSC(params, kidia, kfdia, n, klev, 900.0, full, precision=prec)
+    return full
+
+
+def test_per_block_entry_at_all_image_sizes(params137):
+    """Blocks that grow and shrink the page-locked image, that exceed its limit (1,000 FP64 columns: array by array) and
+    that cover a window, from one thread and from several at once, against the blocked launch."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    n = 1000
+    inp, out = run(params137, "dp", n, n, 137, 71)
+
+    def check(m, kidia, kfdia):
+        got = _block_call(params137, inp, "dp", m, 137, kidia, kfdia)
+        for name in OUT:
+            ref = out[name][0][..., :m]
+            ref = (ref.T if ref.ndim < 3 else ref.transpose(2, 1, 0)).copy()
+            rows = slice(kidia - 1, kfdia)
+            np.testing.assert_array_equal(got[name][rows], ref[rows], err_msg=f"{name} {m} {kidia}:{kfdia}")
+        assert np.isnan(got["ptendency_loc_t"][kfdia:]).all() and np.isnan(got["pfplsl"][: kidia - 1]).all()
+
+    for m, kidia, kfdia in [(8, 1, 8), (300, 1, 300), (33, 1, 20), (n, 1, n), (64, 1, 64)]:
+        check(m, kidia, kfdia)
+    with ThreadPoolExecutor(4) as ex:
+        list(ex.map(lambda m: check(m, 1, m), [40, 100, 8, 64, 200, 16, 128, 32]))
