@@ -638,7 +638,8 @@ struct cloudsc_surrogate {
   int* count = nullptr;
   int list_cap = 0;
   int* count_host = nullptr;  // pinned
-  hipEvent_t counted = nullptr;
+  hipEvent_t counted = nullptr, joined = nullptr;
+  hipStream_t side = nullptr;  // the rerun columns, beside the network's first batch
   void* comp = nullptr;
   size_t comp_bytes = 0;
   std::vector<void*> allocs;
@@ -685,9 +686,9 @@ void launch_features(cloudsc_surrogate* s, const KPtrs<float>& p, const surr::Di
 }
 
 // Network prediction for all columns, in batches of max_batch, the first of whose features are already there; with rank,
-// columns of rank >= 0 are taken from the compact field set pc instead.
+// columns of rank >= 0 are taken from the compact field set pc instead, which is complete at the event `ready`.
 hipError_t predict(cloudsc_surrogate* s, const cloudsc_params_t* q, const KPtrs<float>& p, const surr::Dims& d,
-                   const KPtrs<float>& pc, const int* rank, hipStream_t st) {
+                   const KPtrs<float>& pc, const int* rank, hipEvent_t ready, hipStream_t st) {
   hipError_t e = hipSuccess;
   const int ntotal = d.ngpblks * d.nproma;
   if (ntotal > d.ngptot)
@@ -700,19 +701,21 @@ hipError_t predict(cloudsc_surrogate* s, const cloudsc_params_t* q, const KPtrs<
   const bool vec = bits % 16 == 0;
   auto* diag = rank ? (vec ? surr::diagnostics<true, 4> : surr::diagnostics<true, 1>)
                     : (vec ? surr::diagnostics<false, 4> : surr::diagnostics<false, 1>);
-  hipLaunchKernelGGL(diag, dim3(nblk(d.ngptot, vec ? 1024 : 256), 12, nblk(d.klev + 1, surr::LEV)), dim3(256), 0, st, p,
-                     pc, rank, d, q->ncldtop);
   for (int c0 = 0; c0 < d.ngptot && e == hipSuccess; c0 += s->max_batch) {
     const int n = std::min(s->max_batch, d.ngptot - c0);
     if (c0 > 0) launch_features(s, p, d, c0, st);
     e = mlp::forward(s->net, s->X, surr::pad128(n), s->Y, nullptr, nullptr, st);
+    if (e == hipSuccess && c0 == 0 && ready) e = hipStreamWaitEvent(st, ready, 0);
     if (e != hipSuccess) break;
     hipLaunchKernelGGL(rank ? surr::outputs<true> : surr::outputs<false>,
                        dim3(nblk(n, surr::TILE), nblk(surr::NT * d.klev, surr::TILE)), dim3(256), 0, st, p, pc, rank, d,
                        c0, n, s->nout, s->mu_y, s->sd_y, s->Y, (float)q->rtt, (float)q->rlvtt, (float)q->rlstt);
     e = hipGetLastError();
   }
-  return e;
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(diag, dim3(nblk(d.ngptot, vec ? 1024 : 256), 12, nblk(d.klev + 1, surr::LEV)), dim3(256), 0, st, p,
+                     pc, rank, d, q->ncldtop);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -754,8 +757,10 @@ int cloudsc_surrogate_create(cloudsc_surrogate_t** out, int klev, int n_hidden, 
          F((size_t)max_batch * s->nout, &s->T) || F((size_t)max_batch * s->nout, &s->Y) || F(1, &s->loss_acc) ||
          salloc(s, sizeof(int), (void**)&s->count);
   if (!rc && (hipHostMalloc((void**)&s->count_host, sizeof(int), hipHostMallocDefault) != hipSuccess ||
-              hipEventCreateWithFlags(&s->counted, hipEventDisableTiming) != hipSuccess))
-    rc = fail(CLOUDSC_ENOMEM, "cloudsc_surrogate_create: pinned count or event");
+              hipEventCreateWithFlags(&s->counted, hipEventDisableTiming) != hipSuccess ||
+              hipEventCreateWithFlags(&s->joined, hipEventDisableTiming) != hipSuccess ||
+              hipStreamCreateWithFlags(&s->side, hipStreamNonBlocking) != hipSuccess))
+    rc = fail(CLOUDSC_ENOMEM, "cloudsc_surrogate_create: pinned count, events or stream");
   if (rc) {
     cloudsc_surrogate_destroy(s);
     return rc < 0 ? rc : CLOUDSC_ENOMEM;
@@ -786,6 +791,8 @@ int cloudsc_surrogate_destroy(cloudsc_surrogate_t* s) {
   if (s->comp) (void)hipFree(s->comp);
   if (s->count_host) (void)hipHostFree(s->count_host);
   if (s->counted) (void)hipEventDestroy(s->counted);
+  if (s->joined) (void)hipEventDestroy(s->joined);
+  if (s->side) (void)hipStreamDestroy(s->side);
   delete s;
   return CLOUDSC_OK;
 }
@@ -915,7 +922,7 @@ int cloudsc_surrogate_predict_sp(cloudsc_surrogate_t* s, CLOUDSC_BLOCKED_ARGS(fl
   int rc = check_fields(s, ydparams, ngptot, nproma, klev, ngpblks, p);
   if (rc) return rc;
   launch_features(s, p, d, 0, st);
-  hipError_t e = predict(s, ydparams, p, d, p, nullptr, st);
+  hipError_t e = predict(s, ydparams, p, d, p, nullptr, nullptr, st);
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_surrogate_predict_sp", e);
   return CLOUDSC_OK;
 }
@@ -972,7 +979,7 @@ int cloudsc_hybrid_sp_c(cloudsc_surrogate_t* s, float rerun_fraction, uint64_t r
   const int nsel = *s->count_host;
   if (n_plain) *n_plain = nsel;
   if (nsel == 0) {
-    e = predict(s, q, p, d, p, nullptr, st);
+    e = predict(s, q, p, d, p, nullptr, nullptr, st);
     if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: prediction", e);
     return CLOUDSC_OK;
   }
@@ -1039,7 +1046,14 @@ int cloudsc_hybrid_sp_c(cloudsc_surrogate_t* s, float rerun_fraction, uint64_t r
   for (int i = 0; i < narr; ++i)
     if (arrs[i].in) add_slices(i);
   const unsigned gx = std::min<unsigned>(nblk((long)nsel * (L + 1), 256), 4096u);
-  hipLaunchKernelGGL(surr::copy_columns, dim3(gx, sl.n), dim3(256), 0, st, sl, s->list, nsel, nproma, NP_C, 1);
+  // Steps 2 and 3 run beside the network's first batch: the gather is bound by memory where the products are by the matrix
+  // cores, and the plain kernel has too few columns to occupy the chip.  The side stream starts where the count is known
+  // (behind all earlier work of st) and st waits for it before the first outputs.  262,144 columns, 3 % rerun: 5.90 -> 5.26
+  // ms.
+  hipStream_t side = s->side;
+  e = hipStreamWaitEvent(side, s->counted, 0);
+  if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: side stream", e);
+  hipLaunchKernelGGL(surr::copy_columns, dim3(gx, sl.n), dim3(256), 0, side, sl, s->list, nsel, nproma, NP_C, 1);
   e = hipGetLastError();
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: gather", e);
   // 3. plain kernel on the compact set
@@ -1054,10 +1068,11 @@ int cloudsc_hybrid_sp_c(cloudsc_surrogate_t* s, float rerun_fraction, uint64_t r
   pc.pfsqrf = C(32); pc.pfsqsf = C(33); pc.pfcqrng = C(34); pc.pfcqsng = C(35); pc.pfsqltur = C(36);
   pc.pfsqitur = C(37); pc.pfplsl = C(38); pc.pfplsn = C(39); pc.pfhpsl = C(40); pc.pfhpsn = C(41);
   const KDims kd{nsel, NP_C, klev, ncb, 1, NP_C};
-  e = cloudsc_gpu::launch_cloudsc<float, float>(*q, (double)ptsphy, pc, kd, 0, st);
+  e = cloudsc_gpu::launch_cloudsc<float, float>(*q, (double)ptsphy, pc, kd, 0, side);
+  if (e == hipSuccess) e = hipEventRecord(s->joined, side);
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: plain kernel", e);
   // 4. network on every other column
-  e = predict(s, q, p, d, pc, rank, st);
+  e = predict(s, q, p, d, pc, rank, s->joined, st);
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: prediction", e);
   // 5. PLUDE, a feature that the plain kernel also updates
   sl.n = 0;
