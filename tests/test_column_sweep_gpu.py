@@ -93,3 +93,36 @@ def test_per_block_entry_at_all_image_sizes(params137):
         check(m, kidia, kfdia)
     with ThreadPoolExecutor(4) as ex:
         list(ex.map(lambda m: check(m, 1, m), [40, 100, 8, 64, 200, 16, 128, 32]))
+
+
+@pytest.mark.parametrize("prec", ["sp", "mixed"])
+@pytest.mark.parametrize("nproma,ncldtop,default", [(64, None, True), (100, None, True), (32, 2, True), (75, 91, True),
+                                                    (128, 2, False), (33, None, False)])
+def test_three_wave_kernel_equals_one_wave_kernel(prec, nproma, ncldtop, default, params91):
+    """Small launches take the kernel of three waves to 64 columns, large ones that of one: bit for bit the same, for a
+    first cloud level at the top, at the bottom and between, and blocks that leave parts of waves empty."""
+    import copy
+
+    params = copy.copy(params91)
+    if ncldtop:
+        params.ncldtop = ncldtop
+    if not default:
+        params.rcldiff = params.rcldiff * 1.5
+    big = C.BlockedFields(49300, nproma, 91, prec, "cuda", fill=0.0)
+    C.synth_device(big, params, 9)
+    starts = {1: 0, 40 * nproma: 0, 41 * nproma - 7: 3}
+    small = {}
+    for n, b0 in starts.items():
+        f = C.BlockedFields(n, nproma, 91, prec, "cuda", fill=0.0)
+        for name in f.t:
+            f[name].copy_(big[name][b0:b0 + f.ngpblks])
+        small[n] = f
+    C.cloudsc_blocked(big, params, 900.0)
+    for n, b0 in starts.items():
+        f = small[n]
+        C.cloudsc_blocked(f, params, 900.0)
+        torch.cuda.synchronize()
+        for name in OUT:
+            got = columns(f[name].cpu().numpy(), nproma)[:n]
+            want = columns(big[name][b0:b0 + f.ngpblks].cpu().numpy(), nproma)[:n]
+            np.testing.assert_array_equal(got, want, err_msg=f"{name} {n}")
