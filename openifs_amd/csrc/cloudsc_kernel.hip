@@ -158,43 +158,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
     const R pcl_l = in.ql, pcl_i = in.qi;
     R tcml_t = in.ct, tcml_q = in.cq, tcml_a = in.ca, tcml_l = in.cl, tcml_i = in.ci;
 
-    if constexpr (SAT) {
-      if ((int)k >= ncldtop0) {  // CLOUD_SATADJ for this point, then TENDENCY_CML += its tendencies
-        SatIn<R> x;
-        x.pt = pt, x.pq = pq, x.pa = pa, x.pl = pcl_l, x.pi = pcl_i, x.pap = pap;
-        x.paph0 = paph_k, x.paph1 = paph_k1, x.psurf = paph_surf;
-        x.tct = tcml_t, x.tcq = tcml_q, x.tca = tcml_a, x.tcl = tcml_l, x.tci = tcml_i;
-        x.hrsw = in.hrsw, x.hrlw = in.hrlw, x.vdft = in.vdft, x.vdfq = in.vdfq;
-        x.lude3 = in.lude3, x.lude4 = in.lude4, x.vervel = in.vervel;
-        const SatOut<R> y = satadj_point<R, RD, KC, KCD>(c, cd, x);
-        tcml_t = tcml_t + y.t;
-        tcml_q = tcml_q + y.q;
-        tcml_a = tcml_a + y.a;
-        tcml_l = tcml_l + y.l;
-        tcml_i = tcml_i + y.i;
-        CArgs* const g = fresh();
-        STN<UNI>(g->s.tcml_t, i2, jo, tcml_t);
-        STN<UNI>(g->s.tcml_q, i2, jo, tcml_q);
-        STN<UNI>(g->s.tcml_a, i2, jo, tcml_a);
-        STN<UNI>(g->s.tcml_cld, i5, jo, tcml_l);
-        STN<UNI>(g->s.tcml_cld, i5 + sstep, jo, tcml_i);
-        if (tsat) {
-          STN<UNI>(g->s.tsat_t, i2, jo, y.t);
-          STN<UNI>(g->s.tsat_q, i2, jo, y.q);
-          STN<UNI>(g->s.tsat_a, i2, jo, y.a);
-          STN<UNI>(g->s.tsat_cld, i5, jo, y.l);
-          STN<UNI>(g->s.tsat_cld, i5 + sstep, jo, y.i);
-        }
-      } else if (tsat) {  // zero above NCLDTOP (cloud_satadj.F90:338-348); TENDENCY_CML unchanged
-        CArgs* const g = fresh();
-        STN<UNI>(g->s.tsat_t, i2, jo, R(0));
-        STN<UNI>(g->s.tsat_q, i2, jo, R(0));
-        STN<UNI>(g->s.tsat_a, i2, jo, R(0));
-        STN<UNI>(g->s.tsat_cld, i5, jo, R(0));
-        STN<UNI>(g->s.tsat_cld, i5 + sstep, jo, R(0));
-      }
-    }
-
+#include "sweep_satadj.inc"
 #include "sweep_state.inc"
     // Outputs of this level; defaults are those of levels above NCLDTOP.
     R qxn_l = R(0), qxn_i = R(0), qxn_r = R(0), qxn_s = R(0);
@@ -280,7 +244,7 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
 
 // ---------------------------------------------------------------------------
 // The same sweep by three waves to 64 columns, a level apart: the first loads level t and computes what depends on it
-// alone, the second runs the processes and the implicit solve of level t - 1, the third the tendencies, the
+// alone (and adjusts it, SAT), the second runs the processes and the implicit solve of level t - 1, the third the tendencies, the
 // supersaturation check and the stores of level t - 2.  They pass what the next one needs through LDS, a barrier per
 // level.  The parts are the ones of the kernel above, so the results are the same bit for bit.  A wave alone issues a
 // vector instruction in about half of its cycles and waits in a quarter (1,190 instructions a level, 3.6 us); here the
@@ -308,9 +272,9 @@ cloudsc_column_kernel(const KArgs<R, KC, KCD> args) {
 #define SWEEP_GET(n) R n = from[i++ * 64];
 #define SWEEP_SET(n) n = from[i++ * 64];
 
-template <typename R, typename RD, typename KC, typename KCD, bool UNI>
+template <typename R, typename RD, typename KC, typename KCD, bool UNI, bool SAT>
 __global__ __launch_bounds__(192) void cloudsc_pipeline_kernel(const KArgs<R, KC, KCD> args) {
-  constexpr bool SAT = false, BUD = false;
+  constexpr bool BUD = false;
   constexpr int NHEAD = 0 SWEEP_HEAD(SWEEP_COUNT), NKEEP = 0 SWEEP_KEEP(SWEEP_COUNT), NSOLVE = 0 SWEEP_SOLVE(SWEEP_COUNT);
   __shared__ R s_head[2][NHEAD][64], s_keep[3][NKEEP][64], s_solve[2][NSOLVE][64];
   const KC& c = args.c;
@@ -358,14 +322,18 @@ __global__ __launch_bounds__(192) void cloudsc_pipeline_kernel(const KArgs<R, KC
     const R zconst = LD(p.plsm, u1, jo) > R(0.5) ? c.rcl_kk_cloud_num_land : c.rcl_kk_cloud_num_sea;
     const R zconst_pow = s_pow(zconst, c.rcl_kkbaun);
 #include "sweep_load.inc"
+    const KCD& cd = args.cd;
+    const bool tsat = SAT && args.s.tsat_t;
     Level nxt = load(0);
     for (uint32_t k = 0; k < klev; ++k) {
+      const uint32_t i2 = b2 + k * lstep, i5 = b5 + k * lstep;
       const Level in = nxt;
       if (k + 1 < klev) nxt = load(k + 1);
       const R pmfu_n = in.mfu_n, pmfd_n = in.mfd_n, plu_n = in.lu_n, paph_k1 = in.paph1, pap = in.pap;
       const R pt = in.t, pq = in.q, pa = in.a, pvfl = in.vfl, pvfi = in.vfi, pludeli1 = in.lude1, pludeli2 = in.lude2;
       const R pcl_l = in.ql, pcl_i = in.qi, plude_in = in.lude, snde1 = in.snde1, snde2 = in.snde2;
-      const R tcml_t = in.ct, tcml_q = in.cq, tcml_a = in.ca, tcml_l = in.cl, tcml_i = in.ci;
+      R tcml_t = in.ct, tcml_q = in.cq, tcml_a = in.ca, tcml_l = in.cl, tcml_i = in.ci;
+#include "sweep_satadj.inc"
 #include "sweep_state.inc"
 #include "sweep_derived.inc"
 #include "sweep_early.inc"
@@ -763,7 +731,9 @@ hipError_t launch_variant(const LaunchCfg& l, bool uni, unsigned ncols, const KC
 // 64 columns then cut it.  The line lies where the work-groups no longer all run at once: LDS holds 3 of them on a CU in
 // FP32, 1 in FP64.  FP32 x L137 in blocks of 128: 16,384 columns 515 -> 321 us, 32,768 532 -> 366, 49,152 547 -> 410, but
 // 50,000 559 -> 713; in blocks of 100 x L91, whose rows share lines, 40,007 428 -> 353 us and 49,152 440 -> 458, so the
-// line is lower there.  Mixed 2,048 in blocks of 32 491 -> 328 us.  FP64 16,384 x L137 1.45 -> 0.84 ms.
+// line is lower there.  Mixed 2,048 in blocks of 32 491 -> 328 us.  FP64 16,384 x L137 1.45 -> 0.84 ms.  Fused with the
+// saturation adjustment: FP32 2,048 652 -> 393 us, 49,152 761 -> 657; mixed 10,000 780 -> 474 us; FP64 16,000 1.88 ->
+// 1.17 ms.
 // Launch settings (cloudsc_tune_set_launch) are those of the one-wave kernel and do not move the line.
 template <typename R>
 bool pipelined(unsigned ncols, bool uni) {
@@ -779,9 +749,12 @@ hipError_t launch_either(bool sat, const LaunchCfg& l, bool uni, unsigned ncols,
                        dim3(64), 0, stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, *bud});
     return hipGetLastError();
   }
-  if (!sat && pipelined<R>(ncols, uni)) {
+  if (pipelined<R>(ncols, uni)) {
     const KBudPtrs<R> nb{};
-    auto* kernel = uni ? cloudsc_pipeline_kernel<R, RD, KC, KCD, true> : cloudsc_pipeline_kernel<R, RD, KC, KCD, false>;
+    auto* kernel = sat ? (uni ? cloudsc_pipeline_kernel<R, RD, KC, KCD, true, true>
+                              : cloudsc_pipeline_kernel<R, RD, KC, KCD, false, true>)
+                       : (uni ? cloudsc_pipeline_kernel<R, RD, KC, KCD, true, false>
+                              : cloudsc_pipeline_kernel<R, RD, KC, KCD, false, false>);
     hipLaunchKernelGGL(kernel, dim3((ncols + 63) / 64), dim3(192), 0, stream,
                        KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
     return hipGetLastError();
