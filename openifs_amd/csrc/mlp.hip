@@ -54,9 +54,26 @@ struct EpiArgs {
   float batch;       // EPI_LOSS: rows of the batch
 };
 
-__device__ __forceinline__ float sigmoid(float z) { return 1.0f / (1.0f + __expf(-z)); }
-
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// 1 / (1 + exp(-z)).  For every float x from 1 to 2^126 one Newton step on v_rcp_f32 gives the correctly rounded 1 / x
+// (all 1.06e9 checked against the division), in 3 instructions for the division's 10, which were two thirds of the hidden
+// layers' epilogues (65,536 x 1,024 x 1,920 258 -> 247 us); beyond (z < -87), where 1 / x is denormal, the division.
+__device__ __forceinline__ f32x4 sigmoid(f32x4 z) {
+  f32x4 x, r;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    x[t] = 1.0f + __expf(-z[t]);
+    const float r0 = __builtin_amdgcn_rcpf(x[t]);
+    r[t] = __builtin_fmaf(__builtin_fmaf(-x[t], r0, 1.0f), r0, r0);
+  }
+  const float most = __builtin_fmaxf(__builtin_fmaxf(x[0], x[1]), __builtin_fmaxf(x[2], x[3]));
+  if (__builtin_expect(most > 0x1p126f, 0)) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) r[t] = 1.0f / x[t];
+  }
+  return r;
+}
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
 // Epilogue of a wave's FM x FN fragments of C^T = B A^T: register r of lane l holds C[m][n] with m = lane & 31 of the
@@ -105,12 +122,15 @@ __device__ __forceinline__ void epilogue(const EpiArgs& e, const f32x16 (&acc)[F
         if (EPI != EPI_HIDDEN_INF && EPI != EPI_DHIDDEN) *reinterpret_cast<f32x4*>(e.c + o) = v;
         if (EPI == EPI_F32 || EPI == EPI_OUT) continue;
         bf16x4 a;
+        f32x4 sg;
+        if (EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_INF) sg = sigmoid(v);
+        if (EPI == EPI_DHIDDEN) sg = sigmoid(z[i][j][q]);
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           if (EPI == EPI_HIDDEN || EPI == EPI_HIDDEN_INF) {
-            a[t] = (bf16)(v[t] * sigmoid(v[t]));
+            a[t] = (bf16)(v[t] * sg[t]);
           } else if (EPI == EPI_DHIDDEN) {
-            const float zt = z[i][j][q][t], s = sigmoid(zt);
+            const float zt = z[i][j][q][t], s = sg[t];
             a[t] = (bf16)(v[t] * (s * (1.0f + zt * (1.0f - s))));
           } else {
             const float d = v[t] - z[i][j][q][t];
@@ -302,11 +322,11 @@ __global__ __launch_bounds__(64 * NW) void gemm_ring(const bf16* __restrict__ A,
 // The large-product kernel: 256 x 256 block tile, 8 waves as 2 x 4, each computing 128 rows x 64 columns in 32x32
 // fragments; contraction steps of 64, so that a load takes every row's full 128-byte line (half lines take as many L2
 // requests), in an LDS ring of 3 stages for A, which comes from HBM, and 2 for B, which stays in L2 (160 KB in all).
-// The fragments of a quarter step are read while the quarter before multiplies.  65,536 x 1,024 x 1,920 takes 258 us
-// (1,000 TF/s; with the loads left out 218 us: the matrix cores' clock falls under this load), x 1,024 160 us, of which
-// 46 us are the epilogues (stores and the sigmoids' divisions), during which a CU's matrix cores idle; with two full
-// LDS buffers of 64, waited for at each step, it was 278 and 166 us.  Two groups of 128 x 256 on a CU, so that one's
-// epilogue would overlap the other's products, ask for 1.5 times the bytes: 361 and 174 us.
+// The fragments of a quarter step are read while the quarter before multiplies.  65,536 x 1,024 x 1,920 takes 247 us
+// (1,040 TF/s; with the loads left out 218 us: the matrix cores' clock falls under this load), x 1,024 151 us, of which
+// some 40 us are the epilogues, during which a CU's matrix cores idle; with two full LDS buffers of 64, waited for at
+// each step, the sigmoid's division and stores of 8 bytes a row it was 278 and 166 us.  Two groups of 128 x 256 on a CU,
+// so that one's epilogue would overlap the other's products, ask for 1.5 times the bytes: 361 and 174 us.
 template <int EPI>
 __global__ __launch_bounds__(512) void gemm_wide(const bf16* __restrict__ A, int lda, const bf16* __restrict__ B,
                                                  int ldb, int K, EpiArgs e) {

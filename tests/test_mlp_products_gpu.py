@@ -112,3 +112,22 @@ def test_statistics_match_numpy(ngptot, nproma, params91):
     np.testing.assert_allclose(nrm["mu_y"], y.mean(axis=0), rtol=1e-5, atol=1e-5 * np.abs(y).max())
     live = nrm["wgt_y"] > 0
     np.testing.assert_allclose(nrm["sd_y"][live], y.std(axis=0)[live], rtol=1e-3)
+
+
+def test_activation_over_its_whole_range():
+    """silu of biases from -92 to 92, each through one weight: bf16 resolution of the value, also beyond -87, where
+    1 / (1 + exp(-z)) is denormal."""
+    torch = pytest.importorskip("torch")
+    from openifs_amd import surrogate as S
+
+    m = S.MLP(128, 128, 1, 128, 128, seed=3)
+    z = np.concatenate([np.linspace(-92, -86, 64), np.linspace(-86, 92, 64)]).astype(np.float32)
+    scale = np.where(z < -40, 2.0 ** 100, 1.0).astype(np.float32)
+    m.weight(0, np.zeros((128, 128), np.float32))
+    m.bias(0, z)
+    m.weight(1, np.diag(scale))
+    m.bias(1, np.zeros(128, np.float32))
+    y = m.forward(torch.zeros(128, 128, dtype=torch.bfloat16, device=DEV)).cpu().numpy().astype(np.float64)
+    with np.errstate(over="ignore"):  # FP32 throughout: exp(-z) overflows below -88.7 and the activation is 0
+        want = (z * (np.float32(1) / (np.float32(1) + np.exp(-z)))).astype(np.float64) * scale
+    assert np.all(np.abs(y - want) <= 2.0 ** -8 * np.abs(want) + 1e-30)
