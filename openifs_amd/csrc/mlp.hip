@@ -213,9 +213,9 @@ __device__ __forceinline__ void landed() {
   asm volatile("" ::: "memory");
 }
 
-// The kernel of the training products: a TBM x TBN tile per 256 lanes (2 x 2 waves), contraction steps of 64 in a ring
-// of 4 LDS stages filled 3 steps ahead.  These products have about one tile per CU, so one wave per SIMD has to cover
-// the load latency by itself: a step of 128 x 128 multiplies for ~0.2 us at the matrix cores' rate and its loads take
+// The kernel of the training products: a TBM x TBN tile by NW waves (2 x NW/2), contraction steps of 64 in a ring of 4
+// LDS stages filled 3 steps ahead.  These products have about one tile per CU, so the loads ahead have to cover the
+// latency: a step of 128 x 128 multiplies for ~0.2 us at the matrix cores' rate and its loads take
 // several times that; it measures 0.5 us, which is the rate the tiles come from L2 (16 TB/s over the chip).  The stages
 // are separate LDS objects and the step loop is unrolled over them, so that the compiler can tell a read of one stage
 // from the loads in flight into the others.  4,096 x 1,024 x 1,024 with the hidden layer's epilogue (25 MB stored):

@@ -4,8 +4,8 @@
 // the BF16 MLP of mlp.hip.  Feature and target matrices are built directly from the IFS blocked fields
 // (NPROMA, KLEV[,n], NGPBLKS) through LDS-tiled transposes, so that both the blocked reads and the row-major
 // matrix writes are coalesced.  The hybrid entry reruns a seeded random subset of columns, and every column its
-// gate flags, through the plain kernel: the flagged columns are gathered into a compact blocked field set,
-// run by cloudsc_blocked_sp_c's kernel and scattered back.
+// gate flags, through the plain kernel: those columns are gathered into a compact blocked field set and run by
+// cloudsc_blocked_sp_c's kernel, and the output kernels take them from there.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -139,10 +139,13 @@ __device__ __forceinline__ float target(const KPtrs<float>& p, const Dims& d, in
 // 16 entries are in flight together, which needs the array of an entry chosen as a scalar address ahead of one load
 // (a load in each branch of the choice waits for its data where the branches meet), and from entry to entry only the
 // offset moves on (a division and a 64-bit product per entry cost more than the loads).  Features of 65,536 columns x
-// L137 (830 MB): 366 -> 224 us; targets of 4,096 columns 21 -> 12 us.
+// L137 (720 MB): 366 -> 224 us; with 16-byte stores of the matrix, in another run, 234 -> 217, and with non-temporal
+// loads 200 (3.6 TB/s); of 4,096 columns 21.7 -> 20.5 us.  Targets of 4,096 columns 21 -> 12 us.
 constexpr int ENT = 16;
 
-// Feature matrix X [M x nin] (bf16, standardised) for columns col0 .. col0+M-1.
+// Feature matrix X [M x nin] (bf16, standardised) for columns col0 .. col0+M-1.  NT: the loads carry the non-temporal hint
+// (the rule stands at launch_features_rows).
+template <bool NT>
 __global__ __launch_bounds__(256) void features(KPtrs<float> p, Dims d, int col0, int M, int nin,
                                                 const float* __restrict__ mu, const float* __restrict__ rsd,
                                                 bf16* __restrict__ X) {
@@ -160,7 +163,7 @@ __global__ __launch_bounds__(256) void features(KPtrs<float> p, Dims d, int col0
     size_t o = fidx(c, k, s.s, s.n, L, np);
 #pragma unroll
     for (int i = 0; i < ENT; ++i) {
-      a[i] = s.p[o];
+      a[i] = NT ? __builtin_nontemporal_load(s.p + o) : s.p[o];
       t[i] = pap[i] = 0.0f;
       if (k + 1 < L) {
         ++k;
@@ -193,10 +196,14 @@ __global__ __launch_bounds__(256) void features(KPtrs<float> p, Dims d, int col0
     }
   }
   __syncthreads();
-#pragma unroll 4
-  for (int i = ty; i < TILE; i += 4) {  // write X rows: lanes over entries
-    const int c = c0 + i, e = e0 + tx;
-    if (c < M && e < nin) X[(size_t)c * nin + e] = (bf16)tile[tx][i];
+  typedef bf16 __attribute__((ext_vector_type(8))) bf16x8;
+  const int q = 8 * (tx & 7), e = e0 + q;  // write X rows: 8 lanes x 8 entries to each (nin is a multiple of 128)
+#pragma unroll
+  for (int i = 8 * ty + (tx >> 3); i < TILE; i += 32) {
+    bf16x8 v;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = (bf16)tile[q + j][i];
+    if (c0 + i < M && e < nin) *reinterpret_cast<bf16x8*>(X + (size_t)(c0 + i) * nin + e) = v;
   }
 }
 
@@ -679,10 +686,21 @@ surr::Sat sat_consts(const cloudsc_params_t* q) {
                    (float)q->rtt,  (float)q->rtice, (float)q->rtwat_rtice_r, (float)q->retv};
 }
 
-void launch_features(cloudsc_surrogate* s, const KPtrs<float>& p, const surr::Dims& d, int c0, hipStream_t st) {
-  const int M = surr::pad128(std::min(s->max_batch, d.ngptot - c0));
-  hipLaunchKernelGGL(surr::features, dim3(nblk(M, surr::TILE), nblk(s->nin, surr::TILE)), dim3(256), 0, st, p, d, c0, M,
+// The loads of the features carry the non-temporal hint for the batches of 8,192 columns or more whose rows are whole
+// lines (NPROMA a multiple of 64): prediction for 16,384 columns 159 -> 149 us, for 50,000 607 -> 579, for 131,072
+// 2,074 -> 2,055.  Smaller batches can leave the state in the caches for the next call (4,096 columns 55 -> 56 us,
+// training in batches of 1,024 slower by 1.5 %); a line of a ragged row is read by two waves (no gain with NPROMA 75 and
+// 100); and the first batch of a hybrid call is gathered from right after (60,000 columns 980 -> 993 us): `reread`.
+void launch_features_rows(cloudsc_surrogate* s, const KPtrs<float>& p, const surr::Dims& d, int c0, int M,
+                          bool reread, hipStream_t st) {
+  auto* kernel = !reread && d.nproma % 64 == 0 && M >= 8192 ? surr::features<true> : surr::features<false>;
+  hipLaunchKernelGGL(kernel, dim3(nblk(M, surr::TILE), nblk(s->nin, surr::TILE)), dim3(256), 0, st, p, d, c0, M,
                      s->nin, s->mu_x, s->rsd_x, s->X);
+}
+
+void launch_features(cloudsc_surrogate* s, const KPtrs<float>& p, const surr::Dims& d, int c0, bool reread,
+                     hipStream_t st) {
+  launch_features_rows(s, p, d, c0, surr::pad128(std::min(s->max_batch, d.ngptot - c0)), reread, st);
 }
 
 // Network prediction for all columns, in batches of max_batch, the first of whose features are already there; with rank,
@@ -703,7 +721,7 @@ hipError_t predict(cloudsc_surrogate* s, const cloudsc_params_t* q, const KPtrs<
                     : (vec ? surr::diagnostics<false, 4> : surr::diagnostics<false, 1>);
   for (int c0 = 0; c0 < d.ngptot && e == hipSuccess; c0 += s->max_batch) {
     const int n = std::min(s->max_batch, d.ngptot - c0);
-    if (c0 > 0) launch_features(s, p, d, c0, st);
+    if (c0 > 0) launch_features(s, p, d, c0, false, st);
     e = mlp::forward(s->net, s->X, surr::pad128(n), s->Y, nullptr, nullptr, st);
     if (e == hipSuccess && c0 == 0 && ready) e = hipStreamWaitEvent(st, ready, 0);
     if (e != hipSuccess) break;
@@ -898,8 +916,7 @@ int cloudsc_surrogate_train(cloudsc_surrogate_t* s, float lr, int batch, float* 
   const int M = batch;
   hipError_t e = hipGetLastError();
   for (int c0 = 0; c0 + M <= ngptot && e == hipSuccess; c0 += M, ++nb) {
-    hipLaunchKernelGGL(surr::features, dim3(nblk(M, surr::TILE), nblk(s->nin, surr::TILE)), dim3(256), 0, st, p, d,
-                       c0, M, s->nin, s->mu_x, s->rsd_x, s->X);
+    launch_features_rows(s, p, d, c0, M, false, st);
     hipLaunchKernelGGL(surr::targets, dim3(nblk(M, surr::TILE), nblk(s->nout, surr::TILE)), dim3(256), 0, st, p, d,
                        c0, M, s->nout, s->mu_y, s->rsd_y, s->T);
     e = hipGetLastError();
@@ -921,7 +938,7 @@ int cloudsc_surrogate_predict_sp(cloudsc_surrogate_t* s, CLOUDSC_BLOCKED_ARGS(fl
   SURR_PTRS;
   int rc = check_fields(s, ydparams, ngptot, nproma, klev, ngpblks, p);
   if (rc) return rc;
-  launch_features(s, p, d, 0, st);
+  launch_features(s, p, d, 0, false, st);
   hipError_t e = predict(s, ydparams, p, d, p, nullptr, nullptr, st);
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_surrogate_predict_sp", e);
   return CLOUDSC_OK;
@@ -971,7 +988,7 @@ int cloudsc_hybrid_sp_c(cloudsc_surrogate_t* s, float rerun_fraction, uint64_t r
   if (e == hipSuccess) e = hipMemcpyAsync(s->count_host, s->count, sizeof(int), hipMemcpyDeviceToHost, st);
   if (e == hipSuccess) e = hipEventRecord(s->counted, st);
   if (e == hipSuccess) {
-    launch_features(s, p, d, 0, st);  // runs while the host learns the count
+    launch_features(s, p, d, 0, true, st);  // runs while the host learns the count
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipEventSynchronize(s->counted);

@@ -99,3 +99,33 @@ def test_hybrid_merges_plain_columns(ngptot, nproma, params91):
         if k == "ptendency_loc_cld":  # the fifth species is no output
             got[k], want = got[k][:, :4], want[:, :4]
         np.testing.assert_array_equal(got[k], want, err_msg=k)
+
+
+# padded batches on both sides of 8,192 columns, of blocks of whole 64-column tiles (non-temporal loads from 8,192 on)
+# and of ragged blocks (never): the same columns through the same network, so the same bits
+@pytest.mark.parametrize("ngptot", [8064, 8065, 8192, 8321])
+@pytest.mark.parametrize("nproma", [64, 128])
+def test_features_do_not_depend_on_the_blocking(ngptot, nproma, params91):
+    torch = pytest.importorskip("torch")
+    from openifs_amd import cloudsc as C
+    from openifs_amd import surrogate as S
+    from tests.helpers import columns
+
+    def fields(np_):
+        f = C.BlockedFields(ngptot, np_, 91, "sp", DEV, fill=SENTINEL)  # a slot that the prediction leaves alone
+        C.synth_device(f, params91, 11)
+        return f
+
+    f, g, stats = fields(nproma), fields(75), fields(75)
+    for n in C.INPUT_NAMES:
+        a, b = columns(f[n].cpu().numpy(), nproma)[:ngptot], columns(g[n].cpu().numpy(), 75)[:ngptot]
+        np.testing.assert_array_equal(a, b, err_msg=n)
+    sur = S.Surrogate(91, hidden=128, hidden_layers=1, max_batch=16384, seed=3)
+    C.cloudsc_blocked(stats, params91, 3600.0)  # in-out fields change: a set of its own
+    sur.fit_norm(stats, params91)
+    for x in (f, g):
+        sur.predict(x, params91)
+    for n in ("ptendency_loc_t", "ptendency_loc_q", "ptendency_loc_a", "ptendency_loc_cld", "pfplsl", "pfplsn"):
+        a, b = columns(f[n].cpu().numpy(), nproma)[:ngptot], columns(g[n].cpu().numpy(), 75)[:ngptot]
+        np.testing.assert_array_equal(a, b, err_msg=n)
+        assert n.startswith("pf") or n == "ptendency_loc_cld" or np.abs(a).max() > 0, n
