@@ -71,6 +71,16 @@ def build_oracle():
     return os.path.join(ROOT, "oracle", "liboracle_cloudsc.so")
 
 
+FP64_CHECK_SRC = os.path.join(ROOT, "tests", "hip", "fp64_check.hip")
+FP64_CHECK = os.path.join(ROOT, "tests", "hip", "libfp64_check.so")
+
+
+def build_fp64_check():
+    """The FP64 functions of the column kernels as a library of their own, for the tests."""
+    _run([HIPCC, *HIP_FLAGS, "-shared", "-o", FP64_CHECK, FP64_CHECK_SRC])
+    return FP64_CHECK
+
+
 FLANG = os.environ.get("FLANG", "/opt/rocm/lib/llvm/bin/flang")
 FORTRAN_MOD = os.path.join(HERE, "fortran", "cloudsc_hip_mod.F90")
 FORTRAN_DRIVER_SRC = os.path.join(ROOT, "tests", "fortran", "cloudsc_fortran_driver.F90")
@@ -95,6 +105,7 @@ def build_fortran():
 def build_all(verbose=False):
     lib = build_hip(verbose)
     orc = build_oracle()
+    build_fp64_check()
     build_fortran()
     return lib, orc
 

@@ -106,8 +106,10 @@ __device__ __forceinline__ Log log(double x) {
   return Log{hi, (b - (hi - kb)) + fma_(s * u, q, fma_(k, c->ln2_42_lo, sl + sl)), x};
 }
 
-// x^y where x is 0, infinite, negative or NaN; v = |x|^y for a finite negative x.
+// x^y where x is 0, infinite, negative or NaN; v = |x|^y for a finite negative x.  x^0 is 1 for each of them: exponents
+// are parameters of the scheme, and the sweep takes powers of 0 wherever there is no rain.
 __device__ __forceinline__ double pow_special(double x, double y, double v) {
+  if (y == 0.0) return 1.0;
   const double ax = __builtin_fabs(x), inf = __builtin_inf();
   const bool whole = __builtin_rint(y) == y;
   const bool odd = whole && __builtin_rint(0.5 * y) != 0.5 * y;
@@ -119,7 +121,7 @@ __device__ __forceinline__ double pow_special(double x, double y, double v) {
 }
 __device__ __forceinline__ bool ordinary(double x) { return x > 0.0 && x < __builtin_inf(); }
 
-// x^y from log(x), for a finite y that is not 0.  Largest error 0.69 ulp (the library's pow 1.33), exp 0.69 (0.87).
+// x^y from log(x), for a finite y.  Largest error 0.69 ulp (the library's pow 1.33), exp 0.69 (0.87).
 __device__ __forceinline__ double pow(const Log& b, double y) {
   const TablePtr c = constants();
   const double p = y * b.hi, pl = fma_(y, b.lo, fma_(y, b.hi, -p));
@@ -134,7 +136,10 @@ __device__ __forceinline__ double pow(const Log& b, double y) {
 __device__ __forceinline__ Log log_of_pow(const Log& b, double y) {
   const double p = y * b.hi;
   Log r{p, fma_(y, b.lo, fma_(y, b.hi, -p)), b.x};
-  if (!ordinary(b.x)) r.x = pow_special(b.x, y, 1.0);
+  if (!ordinary(b.x)) {
+    r.x = pow_special(b.x, y, 1.0);
+    if (y == 0.0) r.hi = r.lo = 0.0;  // log of infinity or NaN is no number
+  }
   return r;
 }
 
