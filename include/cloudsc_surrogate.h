@@ -33,7 +33,8 @@ int cloudsc_mlp_create(cloudsc_mlp_t **out, int n_in, int n_hidden, int n_hidden
 int cloudsc_mlp_destroy(cloudsc_mlp_t *m);
 /* n_layers = n_hidden_layers + 1; din/dout (may be NULL) receive each linear layer's widths. */
 int cloudsc_mlp_dims(const cloudsc_mlp_t *m, int *n_layers, int *din, int *dout);
-/* y[M x n_out] (fp32) = network(x[M x n_in] bf16). */
+/* y[M x n_out] (fp32) = network(x[M x n_in] bf16).  Here and below a pointer needs its element's alignment only; x at a
+ * multiple of 16 bytes takes the faster kernels. */
 int cloudsc_mlp_forward(cloudsc_mlp_t *m, const uint16_t *x, int M, float *y, void *stream);
 /* Forward + backward for L = sum_{m,n} wgt[n] (y[m,n] - t[m,n])^2 / M; x and its transpose xT[n_in x M] (must not be
  * NULL; not read: the weight-gradient products transpose x themselves). */

@@ -55,6 +55,9 @@ struct EpiArgs {
 };
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// At pointers and leading dimensions of a caller, who need only align them to the element: the same instructions.
+typedef f32x4 __attribute__((aligned(4))) f32x4_any;
+typedef bf16x8 __attribute__((aligned(2))) bf16x8_any;
 
 // 1 / (1 + exp(-z)).  For every float x from 1 to 2^126 one Newton step on v_rcp_f32 gives the correctly rounded 1 / x
 // (all 1.06e9 checked against the division), in 3 instructions for the division's 10, which were two thirds of the hidden
@@ -97,13 +100,13 @@ __device__ __forceinline__ void epilogue(const EpiArgs& e, const f32x16 (&acc)[F
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
     if (BIAS) bias[j] = *reinterpret_cast<const f32x4*>(e.bias + col + j * 32);
-    if (EPI == EPI_LOSS) wgt[j] = *reinterpret_cast<const f32x4*>(e.wgt + col + j * 32);
+    if (EPI == EPI_LOSS) wgt[j] = *reinterpret_cast<const f32x4_any*>(e.wgt + col + j * 32);
     if (READZ)
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          z[i][j][q] = *reinterpret_cast<const f32x4*>(e.z + (size_t)(row + i * 32 + 8 * q) * e.ldc + col + j * 32);
+          z[i][j][q] = *reinterpret_cast<const f32x4_any*>(e.z + (size_t)(row + i * 32 + 8 * q) * e.ldc + col + j * 32);
   }
   float l = 0.0f;
 #pragma unroll
@@ -119,7 +122,7 @@ __device__ __forceinline__ void epilogue(const EpiArgs& e, const f32x16 (&acc)[F
         const size_t o = (size_t)(row + i * 32 + 8 * q) * e.ldc + col + j * 32;
         f32x4 v = *reinterpret_cast<const tile4*>(rd + 256 * q + 4 * ((lane & 7) ^ ((4 * q + (lane >> 4)) & 7)));
         if (BIAS) v = v + bias[j];
-        if (EPI != EPI_HIDDEN_INF && EPI != EPI_DHIDDEN) *reinterpret_cast<f32x4*>(e.c + o) = v;
+        if (EPI != EPI_HIDDEN_INF && EPI != EPI_DHIDDEN) *reinterpret_cast<f32x4_any*>(e.c + o) = v;
         if (EPI == EPI_F32 || EPI == EPI_OUT) continue;
         bf16x4 a;
         f32x4 sg;
@@ -155,12 +158,13 @@ __device__ __forceinline__ void epilogue(const EpiArgs& e, const f32x16 (&acc)[F
 }
 
 // One operand tile of TB rows x 64 contraction entries in LDS, filled by global_load_lds_dwordx4 (lane l of a load
-// writes 16 bytes at 16 l).  Each lane fetches the global chunk that belongs in its LDS slot.
+// writes 16 bytes at 16 l).  Each lane fetches the global chunk that belongs in its LDS slot.  DIRECT = false: the same
+// through registers, for matrices that start at an address that is no multiple of 16, which loads into LDS do not take.
 //  T = false: the matrix is [rows][K].  LDS row r of 128 bytes, chunk c (16 B) in slot c ^ ((r >> 1) & 7): a fragment
 //    read (16 lanes = 16 consecutive rows, one chunk) finds its rows in distinct slots of the banks.
 //  T = true: the matrix is [K][rows].  LDS row k of TB entries, its 64-byte chunk c in slot c ^ f(k) such that the 4
 //    rows k..k+3 which one transposing read touches lie in distinct quarters of the banks.
-template <int TB, bool T, int NW>
+template <int TB, bool T, int NW, bool DIRECT = true>
 struct Tile {
   static constexpr int W = T ? TB * 2 : 128;        // bytes per LDS row
   static constexpr int NLD = TB * 128 / 1024 / NW;  // loads per wave
@@ -181,7 +185,10 @@ struct Tile {
         const int r = 8 * g + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
         src = p + (size_t)r * ld + (CLAMP ? min(k0 + 8 * c, K - 8) : k0 + 8 * c);
       }
-      __builtin_amdgcn_global_load_lds((const void*)src, (lbf16*)(lds + g * 512), 16, 0, 0);
+      if constexpr (DIRECT)
+        __builtin_amdgcn_global_load_lds((const void*)src, (lbf16*)(lds + g * 512), 16, 0, 0);
+      else
+        *reinterpret_cast<bf16x8*>(lds + g * 512 + 8 * lane) = *reinterpret_cast<const bf16x8_any*>(src);
     }
   }
   // MFMA 32x32x16 operand: lane l supplies row (l & 31) of the 32-row block rb and k = ks + 8 (l >> 5) .. +7.  A
@@ -222,12 +229,12 @@ __device__ __forceinline__ void landed() {
 // 18 us, x 1,920: 26 us; the register-staged kernel with transposed copies of every activation and gradient that this
 // one replaces took 39 us on average over the three, the weight gradient 25 -> 16 us and the input gradient 35 -> 20 us
 // (1,024 x 1,024).
-template <int EPI, int TBM, int TBN, int NW, bool TA, bool TB>
+template <int EPI, int TBM, int TBN, int NW, bool TA, bool TB, bool DIRECT = true>
 __global__ __launch_bounds__(64 * NW) void gemm_ring(const bf16* __restrict__ A, int lda, const bf16* __restrict__ B,
                                                  int ldb, int K, EpiArgs e) {
   constexpr int WN = NW / 2, WCOL = TBN / WN, FM = TBM / 64, FN = WCOL / 32;  // 2 x WN waves of FM x FN fragments
-  typedef Tile<TBM, TA, NW> OpA;
-  typedef Tile<TBN, TB, NW> OpB;
+  typedef Tile<TBM, TA, NW, DIRECT> OpA;
+  typedef Tile<TBN, TB, NW, DIRECT> OpB;
   constexpr int ELEMS = (TBM + TBN) * 64, NLD = OpA::NLD + OpB::NLD;
   __shared__ __attribute__((aligned(1024))) bf16 s0[ELEMS], s1[ELEMS], s2[ELEMS], s3[ELEMS];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -566,10 +573,18 @@ int dev_alloc(cloudsc_mlp* m, size_t bytes, void** p) {
 }
 
 // Tile choice: 256 x 256 where that gives a tile for every CU (256), else 128 x 128 where that gives one for every
-// other CU, else 64 x 64.
+// other CU, else 64 x 64.  Operands of a caller (the input x, cloudsc_mlp_gemm_tn) that do not start at a multiple of 16
+// bytes: 64 x 64 through registers, the same bits.
 template <int EPI, bool TA = false, bool TB = false>
 hipError_t gemm(const bf16* A, int lda, const bf16* B, int ldb, int M, int N, int K, const mlp::EpiArgs& e,
                 hipStream_t s, int splits = 1) {
+  if constexpr (EPI == mlp::EPI_F32 || EPI == mlp::EPI_HIDDEN || EPI == mlp::EPI_HIDDEN_INF) {
+    if (((uintptr_t)A | (uintptr_t)B) % 16 != 0) {
+      hipLaunchKernelGGL((mlp::gemm_ring<EPI, 64, 64, 4, TA, TB, false>), dim3(N / 64, M / 64, splits), dim3(256), 0, s,
+                         A, lda, B, ldb, K, e);
+      return hipGetLastError();
+    }
+  }
   const long groups256 = (M % 256 == 0 && N % 256 == 0) ? (long)(M / 256) * (N / 256) : 0;
   if constexpr (!TA && !TB && EPI != mlp::EPI_LOSS) {  // (the loss epilogue does not fit that tile's registers)
     if (groups256 >= 256 && K % 64 == 0 && splits == 1) {
