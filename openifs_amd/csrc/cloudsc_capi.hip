@@ -390,6 +390,11 @@ int per_block(const cloudsc_params_t* q, int kidia, int kfdia, int klon, int kle
     stream = w->stream;
   }
   uint32_t* d_warn = (uint32_t*)(base + warn_off);
+  // An error return waits for what is queued: the thread's next call repacks the image, and the caller may free the arrays.
+  auto fail_idle = [&](const char* what, hipError_t err) {
+    (void)hipStreamSynchronize(stream);
+    return fail(CLOUDSC_EHIP, what, err);
+  };
   (void)hipGetLastError();  // a stale error of an earlier call is not this launch's
   hipError_t e = hipSuccess;
   char* image = nullptr;  // the thread's, where the block fits it
@@ -417,7 +422,7 @@ int per_block(const cloudsc_params_t* q, int kidia, int kfdia, int klon, int kle
       if (arrs[i].n)
         e = hipMemcpyAsync(base + off[i], arrs[i].host, arrs[i].n * arrs[i].esz, hipMemcpyHostToDevice, stream);
   }
-  if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc: copy to device", e);
+  if (e != hipSuccess) return fail_idle("cloudsc: copy to device", e);
   auto D = [&](int i) { return (R*)((image && arrs[i].host_out ? image : base) + off[i]); };
   KPtrs<R> p;
   p.pt = D(0); p.pq = D(1); p.tcml_t = D(2); p.tcml_q = D(3); p.tcml_a = D(4); p.tcml_cld = D(5);
@@ -447,7 +452,7 @@ int per_block(const cloudsc_params_t* q, int kidia, int kfdia, int klon, int kle
   bp.ra = R(q->ra); bp.rpi = R(q->rpi); bp.rcloud_frac_std = R(q->rcloud_frac_std);
   e = cloudsc_gpu::launch_cloudsc<R, RD>(*q, (double)ptsphy, p, d, kidia - 1, stream, nullptr,
                                          (budgets || fsd || inh) ? &bp : nullptr);
-  if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc: kernel launch", e);
+  if (e != hipSuccess) return fail_idle("cloudsc: kernel launch", e);
   uint32_t warn[2] = {0, 0};
   if (image) {
     copy_counters<<<1, 64, 0, stream>>>(d_warn, (uint32_t*)(image + warn_off));
@@ -459,7 +464,7 @@ int per_block(const cloudsc_params_t* q, int kidia, int kfdia, int klon, int kle
     if (e == hipSuccess) e = hipMemcpyAsync(warn, d_warn, sizeof(warn), hipMemcpyDeviceToHost, stream);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(stream);
-  if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc: copy to host", e);
+  if (e != hipSuccess) return fail_idle("cloudsc: copy to host", e);
   if (image) {
     for (int i = 0; i < narr; ++i)
       if (arrs[i].host_out && arrs[i].n) std::memcpy(arrs[i].host_out, image + off[i], arrs[i].n * arrs[i].esz);
