@@ -1068,6 +1068,13 @@ int cloudsc_hybrid_sp_c(cloudsc_surrogate_t* s, float rerun_fraction, uint64_t r
   // (behind all earlier work of st) and st waits for it before the first outputs.  262,144 columns, 3 % rerun: 5.90 -> 5.26
   // ms.
   hipStream_t side = s->side;
+  // An error return leaves nothing on the side stream that still reads the caller's fields.
+  struct Idle {
+    hipStream_t s;
+    ~Idle() {
+      if (s) (void)hipStreamSynchronize(s);
+    }
+  } unjoined{side};
   e = hipStreamWaitEvent(side, s->counted, 0);
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: side stream", e);
   hipLaunchKernelGGL(surr::copy_columns, dim3(gx, sl.n), dim3(256), 0, side, sl, s->list, nsel, nproma, NP_C, 1);
@@ -1097,6 +1104,7 @@ int cloudsc_hybrid_sp_c(cloudsc_surrogate_t* s, float rerun_fraction, uint64_t r
   hipLaunchKernelGGL(surr::copy_columns, dim3(gx, sl.n), dim3(256), 0, st, sl, s->list, nsel, nproma, NP_C, 0);
   e = hipGetLastError();
   if (e != hipSuccess) return fail(CLOUDSC_EHIP, "cloudsc_hybrid_sp_c: scatter", e);
+  unjoined.s = nullptr;
   return CLOUDSC_OK;
 }
 

@@ -41,6 +41,43 @@ for name in ("hipLaunchKernel", "hipMemcpyAsync", "hipHostMalloc", "hipMalloc", 
 print(json.dumps(res))
 """
 
+HYBRID = """
+klev, ngptot, nproma, batch = 3, 300, 64, 128
+p = C.default_params(900.0, 91)
+p.ncldtop = 2
+from openifs_amd import surrogate as S
+
+L = S._lib()
+arm()
+h = ctypes.c_void_p()
+rc = L.cloudsc_surrogate_create(ctypes.byref(h), klev, 128, 1, batch, ctypes.c_uint64(1))
+assert rc == 0, L.cloudsc_last_error()
+ngpblks = (ngptot + nproma - 1) // nproma
+arr = {n: np.ones(C.blocked_shape(kind, nproma, klev, ngpblks), np.int32 if kind == "1di" else np.float32)
+       for n, kind, _ in C.BLOCKED_ARRAYS}
+n = ctypes.c_int()
+
+def call():
+    return L.cloudsc_hybrid_sp_c(h, ctypes.c_float(0.5), ctypes.c_uint64(1), ctypes.c_float(1e30), ctypes.byref(n),
+                                 ctypes.byref(p), ngptot, nproma, klev, ngpblks, ctypes.c_float(900.0),
+                                 *C.blocked_args(arr, lambda x: x.ctypes.data), ctypes.c_void_p(0))
+
+res = []
+for sel in (0, 40):
+    fake.fake_select(sel)
+    arm()
+    assert call() == 0 and n.value == sel, L.cloudsc_last_error()
+    for name in ("hipLaunchKernel", "hipMemcpyAsync", "hipEventRecord", "hipStreamWaitEvent", "hipEventSynchronize"):
+        arm()
+        call()
+        for i in range(1, calls(name) + 1):
+            arm(name, i)
+            ok = call() == 0
+            res.append([name, i, ok, fake.fake_pending(None) if not ok else 0])
+print(json.dumps(res))
+"""
+
+
 @pytest.fixture(scope="module")
 def fake(tmp_path_factory):
     return fake_device.build(str(tmp_path_factory.mktemp("fake")))
@@ -54,3 +91,11 @@ def test_per_block_entry_waits_for_its_stream(fake, prec, klon, flags):
     for name, nth, ok, pending in res:
         assert pending == 0, f"call {nth} of {name} failed, {pending} operations left"
         assert ok or name != "hipHostMalloc"  # without page-locked memory: array by array
+
+
+def test_hybrid_waits_for_its_side_stream(fake):
+    """The caller's stream is the caller's to wait for; the object's own is not."""
+    res = fake_device.run(fake, HYBRID)
+    assert sum(not ok for _, _, ok, _ in res) > 10
+    for name, nth, ok, pending in res:
+        assert pending == 0, f"call {nth} of {name} failed, {pending} operations left on the side stream"
