@@ -71,14 +71,14 @@ def build_oracle():
     return os.path.join(ROOT, "oracle", "liboracle_cloudsc.so")
 
 
-FP64_CHECK_SRC = os.path.join(ROOT, "tests", "hip", "fp64_check.hip")
-FP64_CHECK = os.path.join(ROOT, "tests", "hip", "libfp64_check.so")
+DEVICE_CHECK_SRC = os.path.join(ROOT, "tests", "hip", "device_check.hip")
+DEVICE_CHECK = os.path.join(ROOT, "tests", "hip", "libdevice_check.so")
 
 
-def build_fp64_check():
-    """The FP64 functions of the column kernels as a library of their own, for the tests."""
-    _run([HIPCC, *HIP_FLAGS, "-shared", "-o", FP64_CHECK, FP64_CHECK_SRC])
-    return FP64_CHECK
+def build_device_check():
+    """Device functions of the column kernels as a library of their own, for the tests."""
+    _run([HIPCC, *HIP_FLAGS, "-shared", "-o", DEVICE_CHECK, DEVICE_CHECK_SRC])
+    return DEVICE_CHECK
 
 
 FLANG = os.environ.get("FLANG", "/opt/rocm/lib/llvm/bin/flang")
@@ -105,7 +105,7 @@ def build_fortran():
 def build_all(verbose=False):
     lib = build_hip(verbose)
     orc = build_oracle()
-    build_fp64_check()
+    build_device_check()
     build_fortran()
     return lib, orc
 

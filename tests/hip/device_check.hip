@@ -1,6 +1,7 @@
-// The FP64 functions of the column kernels on arrays, for tests/test_fp64_math_gpu.py.
+// Device functions of the column kernels, for tests/test_fp64_math_gpu.py and tests/test_group_order.py.
 #include <hip/hip_runtime.h>
 
+#include "../../openifs_amd/csrc/cloudsc_device.h"
 #include "../../openifs_amd/csrc/fp64_math.h"
 
 // which: 0 exp(x), 1 x^y, 2 (x^y)^z with x^y as a base only
@@ -21,3 +22,6 @@ extern "C" int fp64_check(int which, const double* x, const double* y, const dou
   hipLaunchKernelGGL(evaluate, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, which, x, y, z, out, n);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
+
+// The order of work-groups on the XCDs, on the host.
+extern "C" unsigned group_order(unsigned id, unsigned n) { return cloudsc_gpu::xcd_group(id, n); }

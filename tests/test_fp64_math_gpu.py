@@ -20,7 +20,7 @@ ULP = 0.75
 
 
 def evaluate(which, x, y=None, z=None):
-    lib = ctypes.CDLL(B.FP64_CHECK)
+    lib = ctypes.CDLL(B.DEVICE_CHECK)
     args = [torch.from_numpy(np.broadcast_to(np.asarray(0.0 if v is None else v, np.float64), np.shape(x)).copy()).cuda()
             for v in (x, y, z)]
     out = torch.empty_like(args[0])
