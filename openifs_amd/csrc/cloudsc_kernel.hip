@@ -674,12 +674,17 @@ hipError_t launch_kl(int kspec, unsigned ncols, const KC& c, const KCD& cd, cons
   return launch_one<BLOCK, WPE, 0, SAT, R, RD>(ncols, c, cd, p, d, ssc_off, s, stream);
 }
 
-// FP64 takes 277 registers, so one wave to a SIMD; bounded to 256, with 22 words spilled, two fit.  That pays as soon as
-// the launch has more waves than the chip has SIMDs (4 x 256): 98,304 columns x L137 3.04 -> 2.53 ms, 262,144 6.17 -> 5.18
-// ms, but 65,536 (a wave to each SIMD) 1.56 -> 1.84 ms.
+// FP64 takes more than 256 registers, so one wave to a SIMD; bounded to 256, with some 20 words spilled, two fit.  That
+// pays as soon as the launch has more waves than the chip has SIMDs (4 x 256): 66,000 columns x L137 2.96 -> 2.43 ms,
+// 131,072 3.00 -> 2.63, 200,000 5.84 -> 5.12, with run-time constants 3.04 -> 2.74, 3.12 -> 2.95 and 6.07 -> 5.71, but
+// 65,536 (a wave to each SIMD) 1.56 -> 1.84 ms.  Fused with the saturation adjustment it spills 100 and more and loses
+// everywhere: 66,000 columns 4.00 -> 4.13 ms, 131,072 4.10 -> 4.61, 200,000 7.92 -> 8.54, with run-time constants 3.99 ->
+// 4.66, 4.20 -> 5.31 and 8.08 -> 9.98.
 template <typename R, typename RD>
 constexpr bool is_fp64 = std::is_same<R, double>::value && std::is_same<RD, double>::value;
-inline bool two_waves(unsigned ncols) { return ncols > 64u * 4u * 256u; }
+inline bool two_waves(const KDims& d, unsigned ncols) {
+  return std::min(ncols, (unsigned)d.ngptot) > 64u * 4u * 256u;  // lanes of padding columns end at once
+}
 
 template <int BLOCK, bool SAT, typename R, typename RD, typename KC, typename KCD>
 hipError_t launch_wpe(const LaunchCfg& l, unsigned ncols, const KC& c, const KCD& cd, const KPtrs<R>& p,
@@ -687,9 +692,10 @@ hipError_t launch_wpe(const LaunchCfg& l, unsigned ncols, const KC& c, const KCD
   constexpr int v = variant_id<R, RD>();
   constexpr int w1 = v == 0 ? 2 : (v == 1 ? 4 : 3);
   constexpr int w2 = 4;  // mixed only
-  if (l.wpe == w1 || (is_fp64<R, RD> && l.wpe == 0 && two_waves(ncols)))
+  if (l.wpe == w1 || (is_fp64<R, RD> && l.wpe == 0 && two_waves(d, ncols)))
     return launch_kl<BLOCK, w1, SAT, R, RD>(l.kspec, ncols, c, cd, p, d, ssc_off, s, stream);
-  if (v == 2 && l.wpe == w2) return launch_kl<BLOCK, w2, SAT, R, RD>(l.kspec, ncols, c, cd, p, d, ssc_off, s, stream);
+  if constexpr (v == 2)
+    if (l.wpe == w2) return launch_kl<BLOCK, w2, SAT, R, RD>(l.kspec, ncols, c, cd, p, d, ssc_off, s, stream);
   return launch_kl<BLOCK, 0, SAT, R, RD>(l.kspec, ncols, c, cd, p, d, ssc_off, s, stream);
 }
 
@@ -698,8 +704,8 @@ hipError_t launch_variant(const LaunchCfg& l, bool uni, unsigned ncols, const KC
                           const KPtrs<R>& p, const KDims& d, int ssc_off, const KSatPtrs<R>& s, hipStream_t stream) {
   const KBudPtrs<R> nb{};
   if (!uni) {  // blocks not aligned to waves: per-lane block offsets, 256-lane groups
-    if constexpr (is_fp64<R, RD>) {
-      if (two_waves(ncols)) {
+    if constexpr (is_fp64<R, RD> && !SAT) {
+      if (two_waves(d, ncols)) {
         hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, 256, false, SAT, false, 2>), dim3((ncols + 255) / 256),
                            dim3(256), 0, stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
         return hipGetLastError();
@@ -721,8 +727,8 @@ hipError_t launch_variant(const LaunchCfg& l, bool uni, unsigned ncols, const KC
       return launch_one<512, 0, 0, SAT, R, RD>(ncols, c, cd, p, d, ssc_off, s, stream);
     default:
       if constexpr (tuned) return launch_wpe<256, SAT, R, RD>(l, ncols, c, cd, p, d, ssc_off, s, stream);
-      if constexpr (is_fp64<R, RD>)
-        if (two_waves(ncols)) return launch_one<256, 2, 0, SAT, R, RD>(ncols, c, cd, p, d, ssc_off, s, stream);
+      if constexpr (is_fp64<R, RD> && !SAT)
+        if (two_waves(d, ncols)) return launch_one<256, 2, 0, SAT, R, RD>(ncols, c, cd, p, d, ssc_off, s, stream);
       return launch_one<256, 0, 0, SAT, R, RD>(ncols, c, cd, p, d, ssc_off, s, stream);
   }
 }

@@ -1,0 +1,62 @@
+"""Which kernel a CLOUDSC launch takes, decided on the host by its size, blocks, arithmetic and constants.  No GPU needed."""
+import re
+
+import pytest
+
+from tests import fake_device
+
+SCRIPT = """
+from openifs_amd import autotune, satadj
+
+L = C.lib()
+some = np.ones(8, np.float64)  # nothing runs
+ptr = ctypes.c_void_p(some.ctypes.data)
+arm()
+res = []
+for step in {steps}:
+    if step[0] == "set":
+        autotune.set_launch(*step[1:])
+        continue
+    kind, prec, ncol, nproma, klev, default = step
+    p = C.default_params(900.0, klev)
+    if not default:
+        p.rcldiff *= 1.5
+    fn = ("cloudsc_blocked_" if kind == "plain" else "cloudsc_satadj_cloudsc_blocked_") + prec + "_c"
+    n = len(C.BLOCKED_ARRAYS) + (0 if kind == "plain" else {extra})
+    arm()
+    rc = getattr(L, fn)(ctypes.byref(p), ncol, nproma, klev, -(-ncol // nproma),
+                        (ctypes.c_double if prec == "dp" else ctypes.c_float)(900.0), *([ptr] * n), ctypes.c_void_p(0))
+    res.append([rc, log()])
+print(json.dumps(res))
+"""
+
+
+@pytest.fixture(scope="module")
+def routes(tmp_path_factory):
+    from openifs_amd import satadj as A
+
+    lib = fake_device.build(str(tmp_path_factory.mktemp("fake")))
+
+    def run(*steps):
+        out = []
+        for rc, log in fake_device.run(lib, SCRIPT.format(steps=list(steps), extra=len(A.SATADJ_EXTRA_INPUTS) + len(A.SATADJ_TENDENCY_OUT))):
+            assert rc == 0 and len(log) == 1, (rc, log)
+            if "pipeline" in log[0]:
+                out.append("three waves")
+            else:
+                block, wpe, kl = re.search(r"Li(\d+)ELb[01]ELb[01]ELb[01]ELi(\d+)ELi(\d+)E", log[0]).groups()
+                out.append((int(block), int(wpe), int(kl)))
+        return out
+
+    return run
+
+
+def test_fp64_at_two_waves_per_simd(routes):
+    """More waves than SIMDs (65,536 columns; padding counts for nothing), but never with the saturation adjustment."""
+    one, two = (256, 0, 0), (256, 2, 0)
+    assert routes(("plain", "dp", 65536, 64, 91, True), ("plain", "dp", 65537, 64, 91, True),
+                  ("plain", "dp", 65536, 100, 91, True), ("plain", "dp", 65537, 100, 91, True),
+                  ("plain", "dp", 65536, 100, 91, False), ("plain", "dp", 70000, 128, 91, False),
+                  ("plain", "dp", 20000, 100, 91, False)) == [one, two, one, two, one, two, one]
+    assert routes(*[("fused", "dp", 131072, n, 137, d) for n in (64, 100) for d in (True, False)]) == [one] * 4
+    assert routes(("plain", "mixed", 200000, 64, 91, False), ("plain", "sp", 200000, 100, 91, True)) == [one] * 2
