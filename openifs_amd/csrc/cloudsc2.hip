@@ -113,9 +113,7 @@ __device__ __forceinline__ void adjust(const C2Const<R>& c, R psp, R& pt, R& pq)
 }
 
 // Work-group size: 64, 128 and 256 run within 1 % of each other at 655,360 x L137 in FP32.
-// The column kernels move 27 (CLOUDST) to 35 words per point at the rate of a copy.  Non-temporal words in aligned blocks
-// and contiguous columns per XCD: CLOUD_S_LAYER on CLOUDST, FP32 327,680 x L137 1,081 -> 1,057 us (4.8 TB/s), 100,000 x
-// L91 in blocks of 64 263 -> 245 us, 40,000 x L91 in blocks of 100 247 -> 240 us.
+// LARGE: the form of a launch that fills the chip and the caches (the rule stands at large()).
 constexpr int CLOUDSC2_BLOCK = 128;
 
 // SATUR with KFLAG = 2 (satur.F90:110-141): the saturation specific humidity of the mixed phase at (t, p), in the
@@ -140,10 +138,11 @@ __device__ __forceinline__ R satur(const C2Const<R>& c, R t, R paprsf) {
 // LAYER: CLOUD_S_LAYER around CLOUDSC2 (cloud_s_layer.F90:112-176): PQS from SATUR at T + TSPHY*TENDENCY%T in the
 // sweep instead of an input, the cloud-fraction tendency (PCLC - PA)/TSPHY, zero rain and snow tendencies and
 // zero PPRECTYPE/PFZRA.
-template <typename R, bool UNI, bool LAYER>
+template <typename R, bool UNI, bool LARGE, bool LAYER>
 __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<R> c, const C2Ptrs<R> p,
                                                                   const C2Dims d) {
-  const uint32_t g = xcd_group(blockIdx.x, gridDim.x) * CLOUDSC2_BLOCK + threadIdx.x;
+  const uint32_t g = (LARGE && !UNI ? xcd_group(blockIdx.x, gridDim.x) : blockIdx.x) * CLOUDSC2_BLOCK + threadIdx.x;
+  constexpr bool NT = UNI && LARGE;
   const uint32_t nproma = (uint32_t)d.nproma;
   const int klev = d.klev;
   if (g >= (uint32_t)d.ngpblks * nproma) return;
@@ -159,16 +158,16 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
   auto ath = [&](int k) { return bh + (uint32_t)k * lstep; };
   if constexpr (LAYER) {  // TENDENCY_LOC%CLD(:,:,NCLDQR/NCLDQS) = 0 on every column of the block (:164-165)
     for (int k = 0; k < klev; ++k) {
-      if (p.ptenr) STN<UNI>(p.ptenr, at2(k), jo, R(0));
-      if (p.ptens) STN<UNI>(p.ptens, at2(k), jo, R(0));
+      if (p.ptenr) STN<NT>(p.ptenr, at2(k), jo, R(0));
+      if (p.ptens) STN<NT>(p.ptens, at2(k), jo, R(0));
     }
   }
   const int kfdia = std::min(d.kfdia, d.ngptot - (int)(b * nproma));
   if ((int)jl < d.kidia - 1 || (int)jl >= kfdia) return;
   const R ptsphy = c.ptsphy;
   if constexpr (LAYER) {  // (:168-169)
-    if (p.pprectype) STN<UNI>(p.pprectype, b * lstep, jo, R(0));
-    if (p.pfzra) STN<UNI>(p.pfzra, b * lstep, jo, R(0));
+    if (p.pprectype) STN<NT>(p.pprectype, b * lstep, jo, R(0));
+    if (p.pfzra) STN<NT>(p.pfzra, b * lstep, jo, R(0));
   }
   const R zeps1 = R(1.e-12), zeps2 = R(1.e-10), zqmax = R(0.5);
 
@@ -184,19 +183,19 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
   }
   // outputs the level loop does not reach (:297-320): PCLC, PCOVPTOT zero, PFPLSL/PFPLSN zero at the top
   for (int k = 0; k < d.ktdia - 1; ++k) {
-    if (!LAYER || p.pclc) STN<UNI>(p.pclc, at2(k), jo, R(0));
-    STN<UNI>(p.pcovptot, at2(k), jo, R(0));
+    if (!LAYER || p.pclc) STN<NT>(p.pclc, at2(k), jo, R(0));
+    STN<NT>(p.pcovptot, at2(k), jo, R(0));
     if constexpr (LAYER) {  // (PCLC - PA)/TSPHY with PCLC = 0 above KTDIA (:155-158)
-      if (p.ptena) STN<UNI>(p.ptena, at2(k), jo, c.zqtmst * (R(0) - LD(p.pa, at2(k), jo)));
+      if (p.ptena) STN<NT>(p.ptena, at2(k), jo, c.zqtmst * (R(0) - LD(p.pa, at2(k), jo)));
     }
   }
-  STN<UNI>(p.pfplsl, ath(0), jo, R(0));
-  STN<UNI>(p.pfplsn, ath(0), jo, R(0));
-  STN<UNI>(p.pfhpsl, ath(0), jo, -R(0) * c.rlvtt);  // (:694-699), as -PFPLSL*RLVTT
-  STN<UNI>(p.pfhpsn, ath(0), jo, -R(0) * c.rlstt);
+  STN<NT>(p.pfplsl, ath(0), jo, R(0));
+  STN<NT>(p.pfplsn, ath(0), jo, R(0));
+  STN<NT>(p.pfhpsl, ath(0), jo, -R(0) * c.rlvtt);  // (:694-699), as -PFPLSL*RLVTT
+  STN<NT>(p.pfhpsn, ath(0), jo, -R(0) * c.rlstt);
   for (int k = 1; k < d.ktdia; ++k) {  // half levels the loop leaves as they are
-    STN<UNI>(p.pfhpsl, ath(k), jo, -LD(p.pfplsl, ath(k), jo) * c.rlvtt);
-    STN<UNI>(p.pfhpsn, ath(k), jo, -LD(p.pfplsn, ath(k), jo) * c.rlstt);
+    STN<NT>(p.pfhpsl, ath(k), jo, -LD(p.pfplsl, ath(k), jo) * c.rlvtt);
+    STN<NT>(p.pfhpsn, ath(k), jo, -LD(p.pfplsn, ath(k), jo) * c.rlstt);
   }
   const R paph_surf = LD(p.paphp1, ath(klev), jo);
 
@@ -208,14 +207,14 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
   auto load = [&](int k) {
     const uint32_t j = at2(k);
     Level v;
-    v.tm1 = LDN<UNI>(p.ptm1, j, jo); v.gtent = LDN<UNI>(p.pgtent, j, jo); v.qm1 = LDN<UNI>(p.pqm1, j, jo);
-    v.gtenq = LDN<UNI>(p.pgtenq, j, jo); v.l = LDN<UNI>(p.pl, j, jo); v.gtenl = LDN<UNI>(p.pgtenl, j, jo); v.i = LDN<UNI>(p.pi, j, jo);
-    v.gteni = LDN<UNI>(p.pgteni, j, jo); v.paph1 = LDN<UNI>(p.paphp1, ath(k + 1), jo);
-    v.qs = LAYER ? R(0) : LDN<UNI>(p.pqs, j, jo);
-    v.a = (LAYER && p.ptena) ? LDN<UNI>(p.pa, j, jo) : R(0);
-    v.app1 = LDN<UNI>(p.papp1, j, jo); v.lude = LDN<UNI>(p.plude, j, jo);
-    v.lu_next = k < klev - 1 ? LDN<UNI>(p.plu, j + lstep, jo) : R(0);
-    v.mfu = LDN<UNI>(p.pmfu, j, jo); v.mfd = LDN<UNI>(p.pmfd, j, jo);
+    v.tm1 = LDN<NT>(p.ptm1, j, jo); v.gtent = LDN<NT>(p.pgtent, j, jo); v.qm1 = LDN<NT>(p.pqm1, j, jo);
+    v.gtenq = LDN<NT>(p.pgtenq, j, jo); v.l = LDN<NT>(p.pl, j, jo); v.gtenl = LDN<NT>(p.pgtenl, j, jo); v.i = LDN<NT>(p.pi, j, jo);
+    v.gteni = LDN<NT>(p.pgteni, j, jo); v.paph1 = LDN<NT>(p.paphp1, ath(k + 1), jo);
+    v.qs = LAYER ? R(0) : LDN<NT>(p.pqs, j, jo);
+    v.a = (LAYER && p.ptena) ? LDN<NT>(p.pa, j, jo) : R(0);
+    v.app1 = LDN<NT>(p.papp1, j, jo); v.lude = LDN<NT>(p.plude, j, jo);
+    v.lu_next = k < klev - 1 ? LDN<NT>(p.plu, j + lstep, jo) : R(0);
+    v.mfu = LDN<NT>(p.pmfu, j, jo); v.mfd = LDN<NT>(p.pmfd, j, jo);
     return v;
   };
 
@@ -240,7 +239,7 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
     // CLOUD_S_LAYER's SATUR at the first-guess temperature (cloud_s_layer.F90:112-118), else the PQS input
     const R pqs = LAYER ? satur(c, ztp1, papp1) : cur.qs;
     if constexpr (LAYER) {
-      if (p.pqsat) STN<UNI>(p.pqsat, i2, jo, pqs);
+      if (p.pqsat) STN<NT>(p.pqsat, i2, jo, pqs);
     }
 
     // 3.1 (:352-416)
@@ -420,20 +419,20 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
     zsfln = zsfln + (R(1.0) - zfwatr) * zdr2;
     zrfreeze = zrfreeze + zrfreeze2;
 
-    STN<UNI>(p.ptenq, i2, jo, -(zcondl + zcondi) + (plude + zevapr + zevaps) * zgdp);
-    STN<UNI>(p.ptent, i2, jo, tendency_t(zcondl, zcondi, zrfreeze));
-    STN<UNI>(p.ptenl, i2, jo, (zqlwc - zl) * c.zqtmst);
-    STN<UNI>(p.pteni, i2, jo, (zqiwc - zi) * c.zqtmst);
-    if (!LAYER || p.pclc) STN<UNI>(p.pclc, i2, jo, pclc);
+    STN<NT>(p.ptenq, i2, jo, -(zcondl + zcondi) + (plude + zevapr + zevaps) * zgdp);
+    STN<NT>(p.ptent, i2, jo, tendency_t(zcondl, zcondi, zrfreeze));
+    STN<NT>(p.ptenl, i2, jo, (zqlwc - zl) * c.zqtmst);
+    STN<NT>(p.pteni, i2, jo, (zqiwc - zi) * c.zqtmst);
+    if (!LAYER || p.pclc) STN<NT>(p.pclc, i2, jo, pclc);
     if constexpr (LAYER) {  // (:155-158)
-      if (p.ptena) STN<UNI>(p.ptena, i2, jo, c.zqtmst * (pclc - cur.a));
+      if (p.ptena) STN<NT>(p.ptena, i2, jo, c.zqtmst * (pclc - cur.a));
     }
-    STN<UNI>(p.pcovptot, i2, jo, pcovptot);
+    STN<NT>(p.pcovptot, i2, jo, pcovptot);
     const uint32_t ih = ath(k + 1);
-    STN<UNI>(p.pfplsl, ih, jo, zrfln);
-    STN<UNI>(p.pfplsn, ih, jo, zsfln);
-    STN<UNI>(p.pfhpsl, ih, jo, -zrfln * c.rlvtt);
-    STN<UNI>(p.pfhpsn, ih, jo, -zsfln * c.rlstt);
+    STN<NT>(p.pfplsl, ih, jo, zrfln);
+    STN<NT>(p.pfplsn, ih, jo, zsfln);
+    STN<NT>(p.pfhpsl, ih, jo, -zrfln * c.rlvtt);
+    STN<NT>(p.pfhpsn, ih, jo, -zsfln * c.rlstt);
     zrfl = zrfln;
     zsfl = zsfln;
     paph0 = paph1;
@@ -445,10 +444,11 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudsc2_kernel(const C2Const<
 // diagnostic water paths PQLWP/PQIWP.  One column per lane, as cloudsc2_kernel.  LAYER: CLOUD_S_LAYER with
 // LEPCLD2 false (cloud_s_layer.F90:112-176): PQS from SATUR, and the A/L/I tendencies (ZPATMP/ZPLTMP/ZPLSMP minus
 // the state)/TSPHY, zero rain and snow tendencies and zero PPRECTYPE/PFZRA.
-template <typename R, bool UNI, bool LAYER>
+template <typename R, bool UNI, bool LARGE, bool LAYER>
 __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R> c, const C2Ptrs<R> p,
                                                                  const C2Dims d) {
-  const uint32_t g = xcd_group(blockIdx.x, gridDim.x) * CLOUDSC2_BLOCK + threadIdx.x;
+  const uint32_t g = (LARGE && !UNI ? xcd_group(blockIdx.x, gridDim.x) : blockIdx.x) * CLOUDSC2_BLOCK + threadIdx.x;
+  constexpr bool NT = UNI && LARGE;
   const uint32_t nproma = (uint32_t)d.nproma;
   const int klev = d.klev;
   if (g >= (uint32_t)d.ngpblks * nproma) return;
@@ -464,8 +464,8 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
   auto ath = [&](int k) { return bh + (uint32_t)k * lstep; };
   if constexpr (LAYER) {  // (:164-165), every column of the block
     for (int k = 0; k < klev; ++k) {
-      if (p.ptenr) STN<UNI>(p.ptenr, at2(k), jo, R(0));
-      if (p.ptens) STN<UNI>(p.ptens, at2(k), jo, R(0));
+      if (p.ptenr) STN<NT>(p.ptenr, at2(k), jo, R(0));
+      if (p.ptens) STN<NT>(p.ptens, at2(k), jo, R(0));
     }
   }
   const int kfdia = std::min(d.kfdia, d.ngptot - (int)(b * nproma));
@@ -475,8 +475,8 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
   const R zcons3 = R(2.5E6) / R(1005.);  // (:215)
   const R zpecons = R(1.E-5);           // (:217)
   if constexpr (LAYER) {
-    if (p.pprectype) STN<UNI>(p.pprectype, b * lstep, jo, R(0));
-    if (p.pfzra) STN<UNI>(p.pfzra, b * lstep, jo, R(0));
+    if (p.pprectype) STN<NT>(p.pprectype, b * lstep, jo, R(0));
+    if (p.pfzra) STN<NT>(p.pfzra, b * lstep, jo, R(0));
   }
   // eta of the tropopause (:234-247)
   R ztrpaus = R(0.1);
@@ -493,27 +493,27 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
   auto wrap_state = [&](int k, R clc, R lwp, R iwp, R a, R l, R i) {
     if constexpr (LAYER) {
       const uint32_t j = at2(k);
-      if (p.ptena) STN<UNI>(p.ptena, j, jo, c.zqtmst * (clc - a));
-      STN<UNI>(p.ptenl, j, jo, c.zqtmst * (lwp - l));
-      STN<UNI>(p.pteni, j, jo, c.zqtmst * (iwp - i));
+      if (p.ptena) STN<NT>(p.ptena, j, jo, c.zqtmst * (clc - a));
+      STN<NT>(p.ptenl, j, jo, c.zqtmst * (lwp - l));
+      STN<NT>(p.pteni, j, jo, c.zqtmst * (iwp - i));
     }
   };
   for (int k = 0; k < d.ktdia - 1; ++k) {
-    if (!LAYER || p.pclc) STN<UNI>(p.pclc, at2(k), jo, R(0));
-    if (!LAYER || p.pqiwp) STN<UNI>(p.pqiwp, at2(k), jo, R(0));
-    if (!LAYER || p.pqlwp) STN<UNI>(p.pqlwp, at2(k), jo, R(0));
-    STN<UNI>(p.pcovptot, at2(k), jo, R(0));
+    if (!LAYER || p.pclc) STN<NT>(p.pclc, at2(k), jo, R(0));
+    if (!LAYER || p.pqiwp) STN<NT>(p.pqiwp, at2(k), jo, R(0));
+    if (!LAYER || p.pqlwp) STN<NT>(p.pqlwp, at2(k), jo, R(0));
+    STN<NT>(p.pcovptot, at2(k), jo, R(0));
     if constexpr (LAYER)
       wrap_state(k, R(0), R(0), R(0), p.ptena ? LD(p.pa, at2(k), jo) : R(0), LD(p.pl, at2(k), jo),
                  LD(p.pi, at2(k), jo));
   }
-  STN<UNI>(p.pfplsl, ath(0), jo, R(0));
-  STN<UNI>(p.pfplsn, ath(0), jo, R(0));
-  STN<UNI>(p.pfhpsl, ath(0), jo, -R(0) * c.rlvtt);  // (:629-634)
-  STN<UNI>(p.pfhpsn, ath(0), jo, -R(0) * c.rlstt);
+  STN<NT>(p.pfplsl, ath(0), jo, R(0));
+  STN<NT>(p.pfplsn, ath(0), jo, R(0));
+  STN<NT>(p.pfhpsl, ath(0), jo, -R(0) * c.rlvtt);  // (:629-634)
+  STN<NT>(p.pfhpsn, ath(0), jo, -R(0) * c.rlstt);
   for (int k = 1; k < d.ktdia; ++k) {
-    STN<UNI>(p.pfhpsl, ath(k), jo, -LD(p.pfplsl, ath(k), jo) * c.rlvtt);
-    STN<UNI>(p.pfhpsn, ath(k), jo, -LD(p.pfplsn, ath(k), jo) * c.rlstt);
+    STN<NT>(p.pfhpsl, ath(k), jo, -LD(p.pfplsl, ath(k), jo) * c.rlvtt);
+    STN<NT>(p.pfhpsn, ath(k), jo, -LD(p.pfplsn, ath(k), jo) * c.rlstt);
   }
   const R paph_surf = LD(p.paphp1, ath(klev), jo);
 
@@ -524,14 +524,14 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
   auto load = [&](int k) {
     const uint32_t j = at2(k);
     Level v;
-    v.tm1 = LDN<UNI>(p.ptm1, j, jo); v.gtent = LDN<UNI>(p.pgtent, j, jo); v.qm1 = LDN<UNI>(p.pqm1, j, jo);
-    v.gtenq = LDN<UNI>(p.pgtenq, j, jo); v.paph1 = LDN<UNI>(p.paphp1, ath(k + 1), jo); v.app1 = LDN<UNI>(p.papp1, j, jo);
-    v.lude = LDN<UNI>(p.plude, j, jo);
-    v.qs = LAYER ? R(0) : LDN<UNI>(p.pqs, j, jo);
-    v.lu_next = k < klev - 1 ? LDN<UNI>(p.plu, j + lstep, jo) : R(0);
-    v.a = (LAYER && p.ptena) ? LDN<UNI>(p.pa, j, jo) : R(0);
-    v.l = LAYER ? LDN<UNI>(p.pl, j, jo) : R(0);
-    v.i = LAYER ? LDN<UNI>(p.pi, j, jo) : R(0);
+    v.tm1 = LDN<NT>(p.ptm1, j, jo); v.gtent = LDN<NT>(p.pgtent, j, jo); v.qm1 = LDN<NT>(p.pqm1, j, jo);
+    v.gtenq = LDN<NT>(p.pgtenq, j, jo); v.paph1 = LDN<NT>(p.paphp1, ath(k + 1), jo); v.app1 = LDN<NT>(p.papp1, j, jo);
+    v.lude = LDN<NT>(p.plude, j, jo);
+    v.qs = LAYER ? R(0) : LDN<NT>(p.pqs, j, jo);
+    v.lu_next = k < klev - 1 ? LDN<NT>(p.plu, j + lstep, jo) : R(0);
+    v.a = (LAYER && p.ptena) ? LDN<NT>(p.pa, j, jo) : R(0);
+    v.l = LAYER ? LDN<NT>(p.pl, j, jo) : R(0);
+    v.i = LAYER ? LDN<NT>(p.pi, j, jo) : R(0);
     return v;
   };
   R zrfl = R(0), zsfl = R(0), zcovptot = R(0);
@@ -549,7 +549,7 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
     const R papp1 = cur.app1, plude = cur.lude;
     const R pqs = LAYER ? satur(c, ztp1, papp1) : cur.qs;
     if constexpr (LAYER) {
-      if (p.pqsat) STN<UNI>(p.pqsat, i2, jo, pqs);
+      if (p.pqsat) STN<NT>(p.pqsat, i2, jo, pqs);
     }
     // critical relative humidity (:263-290)
     R zcrh = R(0);
@@ -696,18 +696,18 @@ __global__ __launch_bounds__(CLOUDSC2_BLOCK) void cloudst_kernel(const C2Const<R
     zrfln = zrfln + zfwatr * zdr;
     zsfln = zsfln + (R(1.0) - zfwatr) * zdr;
 
-    STN<UNI>(p.ptenq, i2, jo, tendency_q(zrfln, zsfln));
-    STN<UNI>(p.ptent, i2, jo, tendency_t(zrfln, zsfln, zrfreeze));
-    if (!LAYER || p.pclc) STN<UNI>(p.pclc, i2, jo, pclc);
-    if (!LAYER || p.pqlwp) STN<UNI>(p.pqlwp, i2, jo, pqlwp);
-    if (!LAYER || p.pqiwp) STN<UNI>(p.pqiwp, i2, jo, pqiwp);
-    STN<UNI>(p.pcovptot, i2, jo, pcovptot);
+    STN<NT>(p.ptenq, i2, jo, tendency_q(zrfln, zsfln));
+    STN<NT>(p.ptent, i2, jo, tendency_t(zrfln, zsfln, zrfreeze));
+    if (!LAYER || p.pclc) STN<NT>(p.pclc, i2, jo, pclc);
+    if (!LAYER || p.pqlwp) STN<NT>(p.pqlwp, i2, jo, pqlwp);
+    if (!LAYER || p.pqiwp) STN<NT>(p.pqiwp, i2, jo, pqiwp);
+    STN<NT>(p.pcovptot, i2, jo, pcovptot);
     wrap_state(k, pclc, pqlwp, pqiwp, cur.a, cur.l, cur.i);
     const uint32_t ih = ath(k + 1);
-    STN<UNI>(p.pfplsl, ih, jo, zrfln);
-    STN<UNI>(p.pfplsn, ih, jo, zsfln);
-    STN<UNI>(p.pfhpsl, ih, jo, -zrfln * c.rlvtt);
-    STN<UNI>(p.pfhpsn, ih, jo, -zsfln * c.rlstt);
+    STN<NT>(p.pfplsl, ih, jo, zrfln);
+    STN<NT>(p.pfplsn, ih, jo, zsfln);
+    STN<NT>(p.pfhpsl, ih, jo, -zrfln * c.rlvtt);
+    STN<NT>(p.pfhpsn, ih, jo, -zsfln * c.rlstt);
     zrfl = zrfln;
     zsfl = zsfln;
     paph0 = paph1;
@@ -764,6 +764,36 @@ C2Ptrs<R> offset_ptrs(const C2Ptrs<R>& p, int64_t b0, int nproma, int klev) {
   return o;
 }
 
+// Large launches in aligned blocks move their words with the non-temporal hint: from 300 MB of fields on, of which the
+// 256 MB last-level cache keeps little for the next call.  FP32, CLOUDSC2, L137: 32,768 columns (450 MB) 254 -> 241 us,
+// 65,536 307 -> 290, but 16,384 (225 MB) 204 -> 231 and 2,048 178 -> 185; CLOUD_S_LAYER on CLOUDST, 65,536 334 -> 311,
+// 16,384 239 -> 257; FP64, 32,768 564 -> 541, 8,192 488 -> 506.
+// Large launches in other blocks whose rows are whole lines take contiguous columns on each XCD.  FP32 x L91 in blocks of
+// 32, CLOUDSC2: 65,536 columns 324 -> 290 us, 250,000 1,373 -> 1,010, but 32,768 171 -> 173; FP64 250,000 1,511 -> 1,386.
+// Rows that share lines keep the dispatcher's order: a level of all columns just fits the L2s or just does not, and the
+// order decides by chance (CLOUD_S_LAYER on CLOUDST, FP32, 131,072 columns: x L91 in blocks of 75 812 -> 610 us, x L137 in
+// blocks of 100 780 -> 940).  Small launches are slower in either form; their kernels are those without it.
+template <typename R>
+bool large(int64_t ncols, const C2Dims& d, bool layer, bool st) {
+  if (d.nproma % 64 == 0) {
+    const int words = st ? (layer ? 27 : 19) : (layer ? 33 : 25);
+    return ncols * d.klev * words * (int64_t)sizeof(R) > 300000000;
+  }
+  return d.nproma * sizeof(R) % 128 == 0 && ncols >= 65536;
+}
+template <typename R, bool UNI, bool LARGE, bool ST, bool LAYER>
+constexpr auto instance() {
+  if constexpr (ST)
+    return cloudst_kernel<R, UNI, LARGE, LAYER>;
+  else
+    return cloudsc2_kernel<R, UNI, LARGE, LAYER>;
+}
+template <typename R, bool ST, bool LAYER>
+auto pick(bool uni, bool big) {
+  return uni ? (big ? instance<R, true, true, ST, LAYER>() : instance<R, true, false, ST, LAYER>())
+             : (big ? instance<R, false, true, ST, LAYER>() : instance<R, false, false, ST, LAYER>());
+}
+
 template <typename R>
 hipError_t launch(const cloudsc_params_t& q, const cloudsc2_params_t& q2, bool ldrain1d, double ptsphy,
                   const C2Ptrs<R>& p, const C2Dims& d, hipStream_t stream, bool layer = false, bool st = false) {
@@ -782,22 +812,10 @@ hipError_t launch(const cloudsc_params_t& q, const cloudsc2_params_t& q2, bool l
     dc.ngptot = (int)(d.ngptot - b0 * d.nproma);
     const C2Ptrs<R> pc = offset_ptrs(p, b0, d.nproma, d.klev);
     const dim3 grid((unsigned)((nb * d.nproma + CLOUDSC2_BLOCK - 1) / CLOUDSC2_BLOCK));
-    if (st && layer && uni)
-      hipLaunchKernelGGL((cloudst_kernel<R, true, true>), grid, dim3(CLOUDSC2_BLOCK), 0, stream, c, pc, dc);
-    else if (st && layer)
-      hipLaunchKernelGGL((cloudst_kernel<R, false, true>), grid, dim3(CLOUDSC2_BLOCK), 0, stream, c, pc, dc);
-    else if (st && uni)
-      hipLaunchKernelGGL((cloudst_kernel<R, true, false>), grid, dim3(CLOUDSC2_BLOCK), 0, stream, c, pc, dc);
-    else if (st)
-      hipLaunchKernelGGL((cloudst_kernel<R, false, false>), grid, dim3(CLOUDSC2_BLOCK), 0, stream, c, pc, dc);
-    else if (layer && uni)
-      hipLaunchKernelGGL((cloudsc2_kernel<R, true, true>), grid, dim3(CLOUDSC2_BLOCK), 0, stream, c, pc, dc);
-    else if (layer)
-      hipLaunchKernelGGL((cloudsc2_kernel<R, false, true>), grid, dim3(CLOUDSC2_BLOCK), 0, stream, c, pc, dc);
-    else if (uni)
-      hipLaunchKernelGGL((cloudsc2_kernel<R, true, false>), grid, dim3(CLOUDSC2_BLOCK), 0, stream, c, pc, dc);
-    else
-      hipLaunchKernelGGL((cloudsc2_kernel<R, false, false>), grid, dim3(CLOUDSC2_BLOCK), 0, stream, c, pc, dc);
+    const bool big = large<R>(nb * d.nproma, d, layer, st);
+    auto* kernel = st ? (layer ? pick<R, true, true>(uni, big) : pick<R, true, false>(uni, big))
+                      : (layer ? pick<R, false, true>(uni, big) : pick<R, false, false>(uni, big));
+    hipLaunchKernelGGL(kernel, grid, dim3(CLOUDSC2_BLOCK), 0, stream, c, pc, dc);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
