@@ -42,21 +42,32 @@ template <typename R>
 struct Vec<R, 1> {
   typedef R type;
 };
-// Loads and stores of words that one point alone touches, with the non-temporal hint; half-level pressures, which two
+// Loads and stores of words that one point alone touches, with the non-temporal hint (NT); half-level pressures, which two
 // points of a column read (and the surface's, which all do), stay plain.  FP32 160,000 x L91 in blocks of 64: 253 us all
 // plain, 232 all non-temporal, 220 like this; 655,360 x L137: 1.52, 1.44 and 1.38 ms; blocks of 75: 239, 233 and 219 us.
-template <int V, typename R>
-__device__ __forceinline__ typename Vec<R, V>::type LDV(const R* base, uint32_t u, uint32_t v) {
-  return __builtin_nontemporal_load(
-      reinterpret_cast<const typename Vec<R, V>::type*>(reinterpret_cast<const char*>(base) + (u + v)));
-}
+// Launches whose fields the 256 MB last-level cache keeps for the next call, but not beside much else, use plain words:
+// FP32 x L91 in blocks of 75, 24,576 columns (215 MB) 41.7 us non-temporal, 37.2 plain, 12,288 (107 MB) 21.8 and 21.3,
+// 50,000 (437 MB) 79.0 and 78.6; x L137 in blocks of 64, 16,384 (215 MB) 37.8 and 35.6, 4,096 (54 MB) 13.3 and 14.2, 32,768
+// (430 MB) 72.6 and 78.1; FP64 x L137, 8,192 (215 MB) 52.7 and 49.2, 4,096 29.6 and 30.5, 16,384 94.7 and 98.8.
+inline bool nontemporal(int64_t bytes) { return bytes < 120000000 || bytes > 350000000; }
 template <int V, typename R>
 __device__ __forceinline__ typename Vec<R, V>::type LDK(const R* base, uint32_t u, uint32_t v) {
   return *reinterpret_cast<const typename Vec<R, V>::type*>(reinterpret_cast<const char*>(base) + (u + v));
 }
-template <int V, typename R>
+template <int V, bool NT, typename R>
+__device__ __forceinline__ typename Vec<R, V>::type LDV(const R* base, uint32_t u, uint32_t v) {
+  if constexpr (NT)
+    return __builtin_nontemporal_load(
+        reinterpret_cast<const typename Vec<R, V>::type*>(reinterpret_cast<const char*>(base) + (u + v)));
+  return LDK<V>(base, u, v);
+}
+template <int V, bool NT, typename R>
 __device__ __forceinline__ void STV(R* base, uint32_t u, uint32_t v, typename Vec<R, V>::type x) {
-  __builtin_nontemporal_store(x, reinterpret_cast<typename Vec<R, V>::type*>(reinterpret_cast<char*>(base) + (u + v)));
+  auto* q = reinterpret_cast<typename Vec<R, V>::type*>(reinterpret_cast<char*>(base) + (u + v));
+  if constexpr (NT)
+    __builtin_nontemporal_store(x, q);
+  else
+    *q = x;
 }
 template <int V, typename R>
 __device__ __forceinline__ R lane(const typename Vec<R, V>::type& x, int j) {
@@ -77,7 +88,7 @@ __device__ __forceinline__ void set_lane(typename Vec<R, V>::type& x, int j, R y
 // 2 words, else 1); lanes of a wave cover consecutive columns, so each load and store instruction moves one
 // contiguous row segment of 64 V words.  Measured at 655,360 columns x L137, plain loads: V = 2 is 9 % faster than V = 1
 // in FP32 (1.40 vs 1.53 ms) and 7 % in FP64; V = 4 is no faster than V = 1 (its 93 VGPRs halve the waves per SIMD).
-template <typename R, typename RD, typename KC, typename KCD, int V>
+template <typename R, typename RD, typename KC, typename KCD, int V, bool NT>
 __global__ __launch_bounds__(256) void satadj_kernel(const KC c, const KCD cd, const SatPtrs<R> p, const SatDims d) {
   typedef typename Vec<R, V>::type VT;
   const uint32_t np = (uint32_t)d.nproma, klev = (uint32_t)d.klev, npv = np / V;
@@ -99,15 +110,15 @@ __global__ __launch_bounds__(256) void satadj_kernel(const KC c, const KCD cd, c
   if ((int)k < c.ncldtop - 1) {  // :338-348
     ot = oq = oa = ol = oi = VT(R(0));
   } else {
-    const VT pt = LDV<V>(p.pt, o2, 0u), pq = LDV<V>(p.pq, o2, 0u), pa = LDV<V>(p.pa, o2, 0u);
-    const VT pl = LDV<V>(p.pl, oc, 0u), pi = LDV<V>(p.pi, oc, 0u), pap = LDV<V>(p.pap, o2, 0u);
+    const VT pt = LDV<V, NT>(p.pt, o2, 0u), pq = LDV<V, NT>(p.pq, o2, 0u), pa = LDV<V, NT>(p.pa, o2, 0u);
+    const VT pl = LDV<V, NT>(p.pl, oc, 0u), pi = LDV<V, NT>(p.pi, oc, 0u), pap = LDV<V, NT>(p.pap, o2, 0u);
     const VT ph0 = LDK<V>(p.paph, oh, 0u), ph1 = LDK<V>(p.paph, oh, lstep), ps = LDK<V>(p.paph, os, 0u);
-    const VT tct = LDV<V>(p.tcml_t, o2, 0u), tcq = LDV<V>(p.tcml_q, o2, 0u), tca = LDV<V>(p.tcml_a, o2, 0u);
-    const VT tcl = LDV<V>(p.tcml_l, oc, 0u), tci = LDV<V>(p.tcml_i, oc, 0u);
-    const VT hrsw = LDV<V>(p.phrsw, o2, 0u), hrlw = LDV<V>(p.phrlw, o2, 0u);
-    const VT vdft = LDV<V>(p.tvdf_t, o2, 0u), vdfq = LDV<V>(p.tvdf_q, o2, 0u);
-    const VT l3 = LDV<V>(p.pludeli, o4, 2u * s4), l4 = LDV<V>(p.pludeli, o4, 3u * s4);
-    const VT vv = LDV<V>(p.pvervel, o2, 0u);
+    const VT tct = LDV<V, NT>(p.tcml_t, o2, 0u), tcq = LDV<V, NT>(p.tcml_q, o2, 0u), tca = LDV<V, NT>(p.tcml_a, o2, 0u);
+    const VT tcl = LDV<V, NT>(p.tcml_l, oc, 0u), tci = LDV<V, NT>(p.tcml_i, oc, 0u);
+    const VT hrsw = LDV<V, NT>(p.phrsw, o2, 0u), hrlw = LDV<V, NT>(p.phrlw, o2, 0u);
+    const VT vdft = LDV<V, NT>(p.tvdf_t, o2, 0u), vdfq = LDV<V, NT>(p.tvdf_q, o2, 0u);
+    const VT l3 = LDV<V, NT>(p.pludeli, o4, 2u * s4), l4 = LDV<V, NT>(p.pludeli, o4, 3u * s4);
+    const VT vv = LDV<V, NT>(p.pvervel, o2, 0u);
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       SatIn<R> x;
@@ -125,11 +136,11 @@ __global__ __launch_bounds__(256) void satadj_kernel(const KC c, const KCD cd, c
     }
   }
   if (lo <= 0 && hi >= V) {
-    STV<V>(p.tloc_t, o2, 0u, ot);
-    STV<V>(p.tloc_q, o2, 0u, oq);
-    STV<V>(p.tloc_a, o2, 0u, oa);
-    STV<V>(p.tloc_l, oc, 0u, ol);
-    STV<V>(p.tloc_i, oc, 0u, oi);
+    STV<V, NT>(p.tloc_t, o2, 0u, ot);
+    STV<V, NT>(p.tloc_q, o2, 0u, oq);
+    STV<V, NT>(p.tloc_a, o2, 0u, oa);
+    STV<V, NT>(p.tloc_l, oc, 0u, ol);
+    STV<V, NT>(p.tloc_i, oc, 0u, oi);
   } else {  // a vector that straddles KIDIA or KFDIA: element stores inside the window only
 #pragma unroll
     for (int j = 0; j < V; ++j)
@@ -179,10 +190,10 @@ hipError_t launch_satadj_c(const KC& c, const KCD& cd, const SatPtrs<R>& p, cons
     pc.tloc_t += b0 * s2; pc.tloc_q += b0 * s2; pc.tloc_a += b0 * s2; pc.tloc_l += b0 * sc; pc.tloc_i += b0 * sc;
     const int64_t lanes = nb * (int64_t)d.klev * (d.nproma / (vec ? VW : 1));
     const unsigned grid = (unsigned)((lanes + 255) / 256);
-    if (vec)
-      hipLaunchKernelGGL((satadj_kernel<R, RD, KC, KCD, VW>), dim3(grid), dim3(256), 0, stream, c, cd, pc, dc);
-    else
-      hipLaunchKernelGGL((satadj_kernel<R, RD, KC, KCD, 1>), dim3(grid), dim3(256), 0, stream, c, cd, pc, dc);
+    const bool nt = nontemporal(nb * d.nproma * d.klev * 24 * (int64_t)sizeof(R));  // 24 words a point
+    auto* kernel = vec ? (nt ? satadj_kernel<R, RD, KC, KCD, VW, true> : satadj_kernel<R, RD, KC, KCD, VW, false>)
+                       : (nt ? satadj_kernel<R, RD, KC, KCD, 1, true> : satadj_kernel<R, RD, KC, KCD, 1, false>);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, c, cd, pc, dc);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
