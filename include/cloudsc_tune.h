@@ -3,15 +3,18 @@
  * (openifs_amd/autotune.py).  No counterpart in the reference: the IFS chooses only NPROMA.
  *
  * variant: 0 = cloudsc_blocked_dp_c, 1 = cloudsc_blocked_sp_c, 2 = cloudsc_blocked_mixed_c.
- * A launch configuration applies to launches with the given KLEV and the default configuration constants:
+ * A launch configuration set by cloudsc_tune_set_launch or cloudsc_tune_set_block applies to every launch with the given
+ * KLEV and the default configuration constants, which then runs the kernel of one wave to 64 columns with:
  *   block          columns per work-group, 64, 128, 256 or 512 (256 where nothing is set);
  *   waves_per_simd minimum waves per SIMD the kernel's register allocation must allow: 0 = the compiler's
- *                  choice (dp 1, sp 3, mixed 2 waves), or 2 (dp), 4 (sp), 3 or 4 (mixed), fewer registers per lane
+ *                  choice (dp 1, sp 3, mixed 3 waves), or 2 (dp), 4 (sp), 3 or 4 (mixed), fewer registers per lane
  *                  and possibly spills;
  *   klev_compiled  1 = use the kernel with the level count compiled in (instantiated for KLEV 137 and 91;
  *                  other KLEV fall back to the run-time kernel).
- * waves_per_simd and klev_compiled are instantiated for blocks of 128 and 256.  Process-wide; safe to call from
- * any thread.
+ * waves_per_simd and klev_compiled are instantiated for blocks of 128 and 256; in field blocks that are no multiple of 64
+ * columns work-groups have 256 lanes and no bound.  Where nothing is set, or a recorded launch, the library chooses by
+ * size: small launches take a kernel of three waves to 64 columns, and dp launches of more than 65,536 columns the bound of
+ * 2 waves.  The results do not depend on any of this.  Process-wide; safe to call from any thread.
  */
 #ifndef CLOUDSC_TUNE_H
 #define CLOUDSC_TUNE_H
@@ -28,6 +31,11 @@ int cloudsc_tune_get_block(int variant, int klev);
  * instantiated (see above). */
 int cloudsc_tune_set_launch(int variant, int klev, int block, int waves_per_simd, int klev_compiled);
 int cloudsc_tune_get_launch(int variant, int klev, int* block, int* waves_per_simd, int* klev_compiled);
+/* As cloudsc_tune_set_launch, for a launch found best on a large number of columns: it applies where the library's choice
+ * by size is the one-wave kernel, and waves_per_simd = 0 leaves that choice as it is. */
+int cloudsc_tune_set_recorded(int variant, int klev, int block, int waves_per_simd, int klev_compiled);
+/* 0: nothing is set for (variant, klev), 1: a recorded launch, 2: a launch for every size. */
+int cloudsc_tune_get_scope(int variant, int klev);
 
 #ifdef __cplusplus
 }

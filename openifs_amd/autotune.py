@@ -10,7 +10,8 @@ For each (variant, KLEV) it times, on seeded synthetic atmospheres of the reques
     compiled in (KLEV 137 and 91).
 It picks the fastest launch, and records it in openifs_amd/tuning/cloudsc_tuned.json under the device's
 architecture name.  `apply()` (called by openifs_amd.cloudsc when the library is loaded) installs the recorded
-launches through cloudsc_tune_set_launch; the recorded NPROMA is advice for hosts that choose their block length
+launches through cloudsc_tune_set_recorded, for launches that the library does not give to its kernel for small
+ones; the recorded NPROMA is advice for hosts that choose their block length
 (the IFS sets NPROMA in its namelist).
 """
 import argparse
@@ -41,6 +42,12 @@ def set_launch(variant, klev, block, waves=0, kspec=0):
              C.lib().cloudsc_tune_set_launch(VARIANTS[variant], klev, block, waves, kspec))
 
 
+def set_recorded(variant, klev, block, waves=0, kspec=0):
+    """As set_launch, for the launches that the library's choice by size gives to the one-wave kernel."""
+    C._check("cloudsc_tune_set_recorded",
+             C.lib().cloudsc_tune_set_recorded(VARIANTS[variant], klev, block, waves, kspec))
+
+
 def get_launch(variant, klev):
     b, w, k = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     C._check("cloudsc_tune_get_launch", C.lib().cloudsc_tune_get_launch(VARIANTS[variant], klev, ctypes.byref(b),
@@ -67,7 +74,7 @@ def time_launches(variant, klev, ncols, nproma, launches, reps=5, seed=4242, par
     plude0 = f["plude"].clone()
     stream = torch.cuda.current_stream()
     out = {}
-    old = get_launch(variant, klev)
+    old, scope = get_launch(variant, klev), C.lib().cloudsc_tune_get_scope(VARIANTS[variant], klev)
     try:
         for launch in launches:
             set_launch(variant, klev, *launch)
@@ -83,7 +90,10 @@ def time_launches(variant, klev, ncols, nproma, launches, reps=5, seed=4242, par
                     ts.append(e0.elapsed_time(e1))
             out[tuple(launch)] = float(np.median(ts))
     finally:
-        set_launch(variant, klev, *old)
+        if scope == 1:
+            set_recorded(variant, klev, *old)
+        else:
+            set_launch(variant, klev, *(old if scope else (0,)))
     del f, plude0
     torch.cuda.empty_cache()
     return out
@@ -150,7 +160,7 @@ def apply(cache=None, arch=None):
     for variant, per_klev in cache.get(arch, {}).items():
         for klev, rec in per_klev.items():
             launch = (int(rec["block"]), int(rec.get("waves", 0)), int(rec.get("klev_compiled", 0)))
-            set_launch(variant, int(klev), *launch)
+            set_recorded(variant, int(klev), *launch)
             applied[(variant, int(klev))] = launch
     return applied
 

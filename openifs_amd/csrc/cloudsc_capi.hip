@@ -618,6 +618,7 @@ extern "C" int cloudsc_tune_set_block(int variant, int klev, int block) {
   } else {
     cloudsc_gpu::LaunchCfg l;
     l.block = block;
+    l.scope = 2;
     cloudsc_gpu::set_tuned_launch(variant, klev, &l);
   }
   return CLOUDSC_OK;
@@ -627,7 +628,8 @@ extern "C" int cloudsc_tune_get_block(int variant, int klev) {
   return cloudsc_gpu::tuned_launch(variant, klev).block;
 }
 
-extern "C" int cloudsc_tune_set_launch(int variant, int klev, int block, int waves_per_simd, int klev_compiled) {
+namespace {
+int set_launch(int variant, int klev, int block, int waves_per_simd, int klev_compiled, int scope) {
   if (variant < 0 || variant > 2 || klev < 2)
     return cloudsc_capi::fail(CLOUDSC_EDIMS, "cloudsc_tune_set_launch: variant 0..2, KLEV >= 2");
   if (block == 0) {
@@ -638,6 +640,7 @@ extern "C" int cloudsc_tune_set_launch(int variant, int klev, int block, int wav
   l.block = block;
   l.wpe = waves_per_simd;
   l.kspec = klev_compiled;
+  l.scope = scope;
   if (!cloudsc_gpu::valid_launch(variant, l))
     return cloudsc_capi::fail(CLOUDSC_EDIMS,
                               "cloudsc_tune_set_launch: block 64/128/256/512; waves per SIMD 0, or 2 (dp), 4 (sp), "
@@ -646,6 +649,17 @@ extern "C" int cloudsc_tune_set_launch(int variant, int klev, int block, int wav
   cloudsc_gpu::set_tuned_launch(variant, klev, &l);
   return CLOUDSC_OK;
 }
+}  // namespace
+
+extern "C" int cloudsc_tune_set_launch(int variant, int klev, int block, int waves_per_simd, int klev_compiled) {
+  return set_launch(variant, klev, block, waves_per_simd, klev_compiled, 2);
+}
+
+extern "C" int cloudsc_tune_set_recorded(int variant, int klev, int block, int waves_per_simd, int klev_compiled) {
+  return set_launch(variant, klev, block, waves_per_simd, klev_compiled, 1);
+}
+
+extern "C" int cloudsc_tune_get_scope(int variant, int klev) { return cloudsc_gpu::tuned_launch(variant, klev).scope; }
 
 extern "C" int cloudsc_tune_get_launch(int variant, int klev, int* block, int* waves_per_simd, int* klev_compiled) {
   if (variant < 0 || variant > 2 || !block || !waves_per_simd || !klev_compiled)

@@ -132,6 +132,7 @@ struct LaunchCfg {
   int block = 256;  // columns per work-group: 64, 128, 256 or 512
   int wpe = 0;      // minimum waves per SIMD of the register allocation (0: compiler's choice)
   int kspec = 0;    // 1: use the instantiation with KLEV compiled in (137 and 91)
+  int scope = 0;    // 0: nothing set; 1: recorded, for launches that take the one-wave kernel; 2: set, for every launch
 };
 bool valid_launch(int variant, const LaunchCfg& l);
 LaunchCfg tuned_launch(int variant, int klev);

@@ -610,9 +610,9 @@ KPtrs<R> offset_ptrs(const KPtrs<R>& p, int64_t b0, int64_t nproma, int64_t klev
   return q;
 }
 
-// Launch configuration per (arithmetic variant, KLEV), set by the autotuner (cloudsc_tune_set_launch): work-group
-// size, minimum waves per SIMD of the register allocation, and whether the level count is compiled in.  Default:
-// 256 columns per group, the compiler's register allocation, run-time KLEV.
+// Launch configuration per (arithmetic variant, KLEV), set by a caller or from the autotuner's records
+// (include/cloudsc_tune.h): work-group size, minimum waves per SIMD of the register allocation, and whether the level
+// count is compiled in.  Default: 256 columns per group, the compiler's register allocation, run-time KLEV.
 namespace {
 std::mutex g_tune_mutex;
 std::map<std::pair<int, int>, LaunchCfg> g_tuned;
@@ -623,8 +623,9 @@ constexpr int variant_id() {
   return sizeof(R) == 8 ? 0 : (sizeof(RD) == 8 ? 2 : 1);  // 0 dp, 1 sp, 2 mixed
 }
 
-// Waves-per-SIMD bounds instantiated for each variant besides 0: dp holds its state in 256 registers (1 wave),
-// sp in 137 (3 waves), mixed in 177 (2 waves); each gets the next occupancy steps its state fits with few spills.
+// Waves-per-SIMD bounds instantiated for each variant besides 0: dp holds its state in more than 256 registers (1 wave),
+// sp in 138 and mixed in 166 (3 waves each, so mixed's bound of 3 changes nothing); each gets the next occupancy steps
+// that its state fits.
 bool valid_wpe(int variant, int wpe) {
   if (wpe == 0) return true;
   switch (variant) {
@@ -682,8 +683,8 @@ hipError_t launch_kl(int kspec, unsigned ncols, const KC& c, const KCD& cd, cons
 // 4.66, 4.20 -> 5.31 and 8.08 -> 9.98.
 template <typename R, typename RD>
 constexpr bool is_fp64 = std::is_same<R, double>::value && std::is_same<RD, double>::value;
-inline bool two_waves(const KDims& d, unsigned ncols) {
-  return std::min(ncols, (unsigned)d.ngptot) > 64u * 4u * 256u;  // lanes of padding columns end at once
+inline bool two_waves(const LaunchCfg& l, const KDims& d, unsigned ncols) {
+  return l.scope < 2 && std::min(ncols, (unsigned)d.ngptot) > 64u * 4u * 256u;  // lanes of padding columns end at once
 }
 
 template <int BLOCK, bool SAT, typename R, typename RD, typename KC, typename KCD>
@@ -692,7 +693,7 @@ hipError_t launch_wpe(const LaunchCfg& l, unsigned ncols, const KC& c, const KCD
   constexpr int v = variant_id<R, RD>();
   constexpr int w1 = v == 0 ? 2 : (v == 1 ? 4 : 3);
   constexpr int w2 = 4;  // mixed only
-  if (l.wpe == w1 || (is_fp64<R, RD> && l.wpe == 0 && two_waves(d, ncols)))
+  if (l.wpe == w1 || (is_fp64<R, RD> && l.wpe == 0 && two_waves(l, d, ncols)))
     return launch_kl<BLOCK, w1, SAT, R, RD>(l.kspec, ncols, c, cd, p, d, ssc_off, s, stream);
   if constexpr (v == 2)
     if (l.wpe == w2) return launch_kl<BLOCK, w2, SAT, R, RD>(l.kspec, ncols, c, cd, p, d, ssc_off, s, stream);
@@ -705,7 +706,7 @@ hipError_t launch_variant(const LaunchCfg& l, bool uni, unsigned ncols, const KC
   const KBudPtrs<R> nb{};
   if (!uni) {  // blocks not aligned to waves: per-lane block offsets, 256-lane groups
     if constexpr (is_fp64<R, RD> && !SAT) {
-      if (two_waves(d, ncols)) {
+      if (two_waves(l, d, ncols)) {
         hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, 256, false, SAT, false, 2>), dim3((ncols + 255) / 256),
                            dim3(256), 0, stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
         return hipGetLastError();
@@ -728,7 +729,7 @@ hipError_t launch_variant(const LaunchCfg& l, bool uni, unsigned ncols, const KC
     default:
       if constexpr (tuned) return launch_wpe<256, SAT, R, RD>(l, ncols, c, cd, p, d, ssc_off, s, stream);
       if constexpr (is_fp64<R, RD> && !SAT)
-        if (two_waves(d, ncols)) return launch_one<256, 2, 0, SAT, R, RD>(ncols, c, cd, p, d, ssc_off, s, stream);
+        if (two_waves(l, d, ncols)) return launch_one<256, 2, 0, SAT, R, RD>(ncols, c, cd, p, d, ssc_off, s, stream);
       return launch_one<256, 0, 0, SAT, R, RD>(ncols, c, cd, p, d, ssc_off, s, stream);
   }
 }
@@ -740,10 +741,10 @@ hipError_t launch_variant(const LaunchCfg& l, bool uni, unsigned ncols, const KC
 // line is lower there.  Mixed 2,048 in blocks of 32 491 -> 328 us.  FP64 16,384 x L137 1.45 -> 0.84 ms.  Fused with the
 // saturation adjustment: FP32 2,048 652 -> 393 us, 49,152 761 -> 657; mixed 10,000 780 -> 474 us; FP64 16,000 1.88 ->
 // 1.17 ms.
-// Launch settings (cloudsc_tune_set_launch) are those of the one-wave kernel and do not move the line.
+// A launch that a caller has set (cloudsc_tune_set_launch) is one of the one-wave kernel at every size.
 template <typename R>
-bool pipelined(unsigned ncols, bool uni) {
-  return ncols <= 64u * 256u * (sizeof(R) == 8 ? 1u : 3u) && (uni || ncols <= 40960u);
+bool pipelined(const LaunchCfg& l, unsigned ncols, bool uni) {
+  return l.scope < 2 && ncols <= 64u * 256u * (sizeof(R) == 8 ? 1u : 3u) && (uni || ncols <= 40960u);
 }
 
 template <typename R, typename RD, typename KC, typename KCD>
@@ -755,7 +756,7 @@ hipError_t launch_either(bool sat, const LaunchCfg& l, bool uni, unsigned ncols,
                        dim3(64), 0, stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, *bud});
     return hipGetLastError();
   }
-  if (pipelined<R>(ncols, uni)) {
+  if (pipelined<R>(l, ncols, uni)) {
     const KBudPtrs<R> nb{};
     auto* kernel = sat ? (uni ? cloudsc_pipeline_kernel<R, RD, KC, KCD, true, true>
                               : cloudsc_pipeline_kernel<R, RD, KC, KCD, false, true>)

@@ -60,3 +60,34 @@ def test_fp64_at_two_waves_per_simd(routes):
                   ("plain", "dp", 20000, 100, 91, False)) == [one, two, one, two, one, two, one]
     assert routes(*[("fused", "dp", 131072, n, 137, d) for n in (64, 100) for d in (True, False)]) == [one] * 4
     assert routes(("plain", "mixed", 200000, 64, 91, False), ("plain", "sp", 200000, 100, 91, True)) == [one] * 2
+
+
+def test_a_launch_that_is_set_is_used_at_every_size(routes):
+    """cloudsc_tune_set_launch holds for small launches too, and waves 0 is the compiler's choice beyond 65,536 FP64
+    columns; a recorded launch (autotune.apply, at the library's loading) leaves both choices to the library."""
+    small, big = ("plain", "sp", 2000, 64, 91, True), ("plain", "sp", 100000, 64, 91, True)
+    dp = ("plain", "dp", 100000, 128, 137, True)
+    assert routes(small, big, dp, ("set", "sp", 91, 128, 0, 0), small, big, ("set", "sp", 91, 0), small, big,
+                  ("set", "dp", 137, 256, 0, 0), dp, ("plain", "dp", 100000, 100, 137, True), ("set", "dp", 137, 128, 2, 1),
+                  dp, ("plain", "dp", 500, 128, 137, True)) == [
+        "three waves", (256, 4, 91), (256, 2, 0), (128, 0, 0), (128, 0, 0), "three waves", (256, 0, 0), (256, 0, 0),
+        (256, 0, 0), (128, 2, 137), (128, 2, 137)]
+
+
+@pytest.mark.gpu
+def test_timing_launches_leaves_the_settings_as_they_were():
+    pytest.importorskip("torch")
+    from openifs_amd import autotune as A
+    from openifs_amd import cloudsc as C
+
+    scope = lambda: C.lib().cloudsc_tune_get_scope(A.VARIANTS["sp"], 91)  # noqa: E731
+    was = scope(), A.get_launch("sp", 91)
+    try:
+        for prepare, want in ((lambda: A.set_launch("sp", 91, 0), 0), (lambda: A.set_recorded("sp", 91, 128, 4, 1), 1),
+                              (lambda: A.set_launch("sp", 91, 64), 2)):
+            prepare()
+            before = A.get_launch("sp", 91)
+            A.time_launches("sp", 91, 2048, 64, [(256, 0, 0), (128, 4, 1)], reps=1)
+            assert scope() == want and A.get_launch("sp", 91) == before
+    finally:
+        (A.set_recorded if was[0] == 1 else A.set_launch)("sp", 91, *(was[1] if was[0] else (0,)))
