@@ -737,14 +737,16 @@ hipError_t launch_variant(const LaunchCfg& l, bool uni, unsigned ncols, const KC
 // Launches with fewer waves than the chip has SIMDs (1,024) take the time of one wave, whatever their size; three waves to
 // 64 columns then cut it.  The line lies where the work-groups no longer all run at once: LDS holds 3 of them on a CU in
 // FP32, 1 in FP64.  FP32 x L137 in blocks of 128: 16,384 columns 515 -> 321 us, 32,768 532 -> 366, 49,152 547 -> 410, but
-// 50,000 559 -> 713; in blocks of 100 x L91, whose rows share lines, 40,007 428 -> 353 us and 49,152 440 -> 458, so the
-// line is lower there.  Mixed 2,048 in blocks of 32 491 -> 328 us.  FP64 16,384 x L137 1.45 -> 0.84 ms.  Fused with the
-// saturation adjustment: FP32 2,048 652 -> 393 us, 49,152 761 -> 657; mixed 10,000 780 -> 474 us; FP64 16,000 1.88 ->
-// 1.17 ms.
+// 50,000 559 -> 713.  Blocks that are no multiple of 64 columns are slower there: of 42 kinds of launch (FP32, mixed, fused,
+// run-time constants; L91, L137; blocks of 32, 75, 100) all gain at 45,000 columns, from 0 to 2 % (FP32 x L137, blocks of
+// 32 and 75, 700 -> 677 us) to 30 % (FP32 x L91, blocks of 100 434 -> 334, blocks of 32 459 -> 364), but at 49,000 those x
+// L91 gain or lose 5 % (FP32, blocks of 100 440 -> 426, blocks of 75 469 -> 491), so the line is at 704 groups there.
+// Mixed 2,048 in blocks of 32 491 -> 328 us.  FP64 16,384 x L137 1.45 -> 0.84 ms.  Fused with the saturation adjustment:
+// FP32 2,048 652 -> 393 us, 49,152 761 -> 657; mixed 10,000 780 -> 474 us; FP64 16,000 1.88 -> 1.17 ms.
 // A launch that a caller has set (cloudsc_tune_set_launch) is one of the one-wave kernel at every size.
 template <typename R>
 bool pipelined(const LaunchCfg& l, unsigned ncols, bool uni) {
-  return l.scope < 2 && ncols <= 64u * 256u * (sizeof(R) == 8 ? 1u : 3u) && (uni || ncols <= 40960u);
+  return l.scope < 2 && ncols <= 64u * 256u * (sizeof(R) == 8 ? 1u : 3u) && (uni || ncols <= 45056u);
 }
 
 template <typename R, typename RD, typename KC, typename KCD>

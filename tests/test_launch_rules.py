@@ -91,3 +91,16 @@ def test_timing_launches_leaves_the_settings_as_they_were():
             assert scope() == want and A.get_launch("sp", 91) == before
     finally:
         (A.set_recorded if was[0] == 1 else A.set_launch)("sp", 91, *(was[1] if was[0] else (0,)))
+
+
+def test_three_wave_launches_by_size(routes):
+    """One round of work-groups: 49,152 columns in FP32, 16,384 in FP64; 45,056 in blocks that are no multiple of 64."""
+    steps = []
+    for prec in ("sp", "mixed"):
+        for nproma, line in ((64, 49152), (32, 45056)):
+            for default in (True, False):
+                for kind in ("plain", "fused"):
+                    steps += [(kind, prec, line, nproma, 91, default), (kind, prec, line + nproma, nproma, 91, default)]
+    for nproma in (64, 32):
+        steps += [("plain", "dp", 16384, nproma, 91, True), ("plain", "dp", 16384 + nproma, nproma, 91, True)]
+    assert [r == "three waves" for r in routes(*steps)] == [True, False] * (len(steps) // 2)
