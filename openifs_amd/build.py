@@ -30,7 +30,7 @@ HIP_FLAGS = [
     # thresholds FP32 results fall on in almost every column, while unfused arithmetic keeps
     # the FP32 kernel as close to FP64 as the FP32 CPU oracle is.
     "-ffp-contract=off",
-    # FP32 exp/pow on v_exp_f32/v_log_f32 (FP64 keeps the accurate library functions)
+    # FP32 exp/pow on v_exp_f32/v_log_f32 (FP64 keeps accurate functions: the library's, in the column sweep its own)
     "-DCLOUDSC_FAST_TRANSCENDENTALS",
     # packed FP32 (v_pk_*_f32) is disabled for all device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

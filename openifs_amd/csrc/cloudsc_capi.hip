@@ -234,9 +234,13 @@ __global__ void copy_counters(const uint32_t* n, uint32_t* out) {
 
 // The calling thread's page-locked image of a block, kept between calls up to kStageBytes and given back at its end.
 // A block is 42 arrays, and its 64 copies between pageable arrays and the device cost more than the kernel.  With the
-// image the inputs go in one copy, and the kernel stores the outputs, which it writes once each and spread over the whole
-// sweep, into the image directly.  FP32, L137, 32 columns: 1,240 -> 675 us (kernel 460); FP32, L91, 512 columns 1,550 ->
-// 805 us; FP64, L137, 512 columns 3,620 -> 3,180 us.  (Inputs read from the image too: 655, 825 and 3,250 us.)
+// image the inputs go in one copy, and the kernel stores the outputs, spread over the whole sweep, into the image directly.
+// FP32, L137, 32 columns: 1,355 -> 430 us; FP32, L91, 512 columns 1,585 -> 625 us; FP64, L137, 512 columns 4,270 -> 2,380
+// us, 1,000 columns (61 MB) 6,560 -> 4,430 us.  (Inputs read from the image too: no gain.)  PLUDE, which the kernel reads
+// once a level, and PEXTRA, of which the budgets read and write up to 52 words a level, lie there too: on the device, with a
+// copy of their own, PLUDE changes nothing (FP32 32 columns 431 -> 436 us), and PEXTRA gains for few columns and loses for
+// many (FP32, all budgets: 8 columns 1,195 -> 1,120 us, 128 1,700 -> 1,745, 512 3,360 -> 3,750; without an image 1,555,
+// 2,390 and 4,270).
 constexpr size_t kStageBytes = size_t(64) << 20;
 struct Stage {
   char* p = nullptr;

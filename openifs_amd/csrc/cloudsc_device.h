@@ -182,8 +182,9 @@ __device__ __forceinline__ void ST(T* base, uint32_t u, uint32_t v, T x) {
 
 // The same with the non-temporal hint where NT: fields that a sweep reads or writes once, in whole lines.  Rows that share
 // a line with the next wave's (NPROMA no multiple of 64) keep the plain form: there the hint drops lines that are
-// needed again (FP32 40,007 x L91 in blocks of 100: 375 us without, 398 us with it; mixed 655,360 x L137 in blocks of
-// 128: 3.82 ms without, 3.76 ms with it).
+// needed again (FP32 40,007 x L91 in blocks of 100: 375 us without, 398 us with it, 131,072 x L137 1.47 and 1.72 ms; mixed
+// 655,360 x L137 in blocks of 128: 3.82 ms without, 3.76 ms with it).  Blocks of 32 have whole lines in FP32, but gain
+// nothing from it (66,000 to 200,000 columns within 2.5 % either way).
 template <bool NT, typename T>
 __device__ __forceinline__ T LDN(const T* base, uint32_t u, uint32_t v) {
   typedef const __attribute__((address_space(1))) char gchar;

@@ -501,7 +501,7 @@ __global__ void add_scalar(float* __restrict__ acc, const float* __restrict__ x)
 }
 
 // PRAINFRAC_TOPRFZ is zeroed for all KLON columns of every block, the padding of the last block included
-// (cloudsc.F90:1010); the network path writes the active columns in `outputs`.
+// (cloudsc.F90:1010); the network path writes the active columns in `diagnostics`.
 __global__ void zero_padding_columns(float* __restrict__ prainfrac, int ngptot, int ntotal) {
   const int c = ngptot + blockIdx.x * blockDim.x + threadIdx.x;
   if (c < ntotal) prainfrac[c] = 0.0f;
