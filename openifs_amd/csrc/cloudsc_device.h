@@ -204,13 +204,11 @@ __device__ __forceinline__ void STN(T* base, uint32_t u, uint32_t v, T x) {
 
 // Work-group number -> position in the grid.  The dispatcher deals consecutive work-groups to the 8 XCDs in turn; here
 // each XCD takes one contiguous eighth of the columns, so the groups that run together on it share the pages (and, in
-// ragged blocks, the lines) of the ~50 field arrays.  Where the number is no multiple of 8 the first XCDs have a group
-// more, and the last group, which may be padding, has to be one of those: their eighths come last.  (131,072 columns in
-// blocks of 100 are 512 groups and an empty one.  With that on the last XCD the first one had a 65th full group and the
-// chip ran a round for it: FP32 L137 1,408 us, 1,245 without; mixed 1,440 and 1,104, fused mixed 2,194 and 1,728.)
+// ragged blocks, the lines) of the ~50 field arrays.  A bijection for every grid size; the first XCDs have a group more
+// where the number is no multiple of 8, so a grid had better hold no group without work (the sweep's launcher sees to it).
 __host__ __device__ __forceinline__ uint32_t xcd_group(uint32_t id, uint32_t n) {
-  const uint32_t r = n & 7u, e = (id - n) & 7u, fewer = 8u - r;  // e: number of the eighth; the first 8 - r have one less
-  return e * (n >> 3) + (e > fewer ? e - fewer : 0u) + (id >> 3);
+  const uint32_t x = id & 7u, r = n & 7u;
+  return x * (n >> 3) + (x < r ? x : r) + (id >> 3);
 }
 
 }  // namespace cloudsc_gpu

@@ -657,12 +657,37 @@ void set_tuned_launch(int variant, int klev, const LaunchCfg* l) {
     g_tuned[{variant, klev}] = *l;
 }
 
+// Work-groups of `block` columns.  Columns of the last block beyond NGPTOT only have their PRAINFRAC_TOPRFZ cleared (:1010);
+// where they would be whole groups of a launch that fills the chip (a group on each CU), that is done apart (zero_padding):
+// in the XCD order the empty groups push full ones to other XCDs.  131,072 columns in blocks of 100 are 512 groups of 256 and
+// an empty one; dealt as 513, one XCD had 65 full groups and the chip ran a round for it: FP32 L137 1,430 us, 1,165
+// without, mixed 1,360 and 1,155, fused mixed 2,280 and 1,695.
+unsigned groups(const KDims& d, unsigned ncols, unsigned block) {
+  const unsigned active = std::min(ncols, (unsigned)d.ngptot), n = (ncols + block - 1) / block;
+  return n > 256u ? std::max(256u, (active + block - 1) / block) : n;
+}
+
+template <typename R>
+__global__ void clear(R* x, unsigned n) {
+  const unsigned i = blockIdx.x * 256u + threadIdx.x;
+  if (i < n) x[i] = R(0);
+}
+template <typename R>
+void zero_padding(const KPtrs<R>& p, unsigned ncols, unsigned ngroups, unsigned block, hipStream_t stream) {
+  const unsigned done = ngroups * block;
+  if (done < ncols)
+    hipLaunchKernelGGL(clear<R>, dim3((ncols - done + 255) / 256), dim3(256), 0, stream, p.prainfrac_toprfz + done,
+                       ncols - done);
+}
+
 template <int BLOCK, int WPE, int KL, bool SAT, typename R, typename RD, typename KC, typename KCD>
 hipError_t launch_one(unsigned ncols, const KC& c, const KCD& cd, const KPtrs<R>& p, const KDims& d, int ssc_off,
                       const KSatPtrs<R>& s, hipStream_t stream) {
   const KBudPtrs<R> nb{};
-  hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, BLOCK, true, SAT, false, WPE, KL>),
-                     dim3((ncols + BLOCK - 1) / BLOCK), dim3(BLOCK), 0, stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
+  const unsigned n = groups(d, ncols, BLOCK);
+  zero_padding(p, ncols, n, BLOCK, stream);
+  hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, BLOCK, true, SAT, false, WPE, KL>), dim3(n), dim3(BLOCK), 0,
+                     stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
   return hipGetLastError();
 }
 
@@ -705,15 +730,17 @@ hipError_t launch_variant(const LaunchCfg& l, bool uni, unsigned ncols, const KC
                           const KPtrs<R>& p, const KDims& d, int ssc_off, const KSatPtrs<R>& s, hipStream_t stream) {
   const KBudPtrs<R> nb{};
   if (!uni) {  // blocks not aligned to waves: per-lane block offsets, 256-lane groups
+    const unsigned n = groups(d, ncols, 256);
+    zero_padding(p, ncols, n, 256, stream);
     if constexpr (is_fp64<R, RD> && !SAT) {
       if (two_waves(l, d, ncols)) {
-        hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, 256, false, SAT, false, 2>), dim3((ncols + 255) / 256),
-                           dim3(256), 0, stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
+        hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, 256, false, SAT, false, 2>), dim3(n), dim3(256), 0, stream,
+                           KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
         return hipGetLastError();
       }
     }
-    hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, 256, false, SAT, false>), dim3((ncols + 255) / 256),
-                       dim3(256), 0, stream, KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
+    hipLaunchKernelGGL((cloudsc_column_kernel<R, RD, KC, KCD, 256, false, SAT, false>), dim3(n), dim3(256), 0, stream,
+                       KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
     return hipGetLastError();
   }
   // the tuned instantiations (register bound, compiled-in KLEV) exist for the default configuration of CLOUDSC
@@ -764,7 +791,9 @@ hipError_t launch_either(bool sat, const LaunchCfg& l, bool uni, unsigned ncols,
                               : cloudsc_pipeline_kernel<R, RD, KC, KCD, false, true>)
                        : (uni ? cloudsc_pipeline_kernel<R, RD, KC, KCD, true, false>
                               : cloudsc_pipeline_kernel<R, RD, KC, KCD, false, false>);
-    hipLaunchKernelGGL(kernel, dim3((ncols + 63) / 64), dim3(192), 0, stream,
+    const unsigned n = groups(d, ncols, 64);
+    zero_padding(p, ncols, n, 64, stream);
+    hipLaunchKernelGGL(kernel, dim3(n), dim3(192), 0, stream,
                        KArgs<R, KC, KCD>{c, cd, p, d, ssc_off, s, nb});
     return hipGetLastError();
   }
