@@ -573,8 +573,10 @@ int dev_alloc(cloudsc_mlp* m, size_t bytes, void** p) {
 }
 
 // Tile choice: 256 x 256 where that gives a tile for every CU (256), else 128 x 128 where that gives one for every
-// other CU, else 64 x 64.  Operands of a caller (the input x, cloudsc_mlp_gemm_tn) that do not start at a multiple of 16
-// bytes: 64 x 64 through registers, the same bits.
+// other CU, else 64 x 64.  Training's other products take 128 x 128 at any batch, also where it would give 256 tiles of
+// 256 x 256 (steps of 16,384 rows, 1,920 -> 3 x 1,024 -> 1,024: 1,367 us with those, register-staged, 819 with these; of
+// 65,536 rows 5,154 and 3,278 us).  Operands of a caller (the input x, cloudsc_mlp_gemm_tn) that do not start at a
+// multiple of 16 bytes: 64 x 64 through registers, the same bits.
 template <int EPI, bool TA = false, bool TB = false>
 hipError_t gemm(const bf16* A, int lda, const bf16* B, int ldb, int M, int N, int K, const mlp::EpiArgs& e,
                 hipStream_t s, int splits = 1) {
